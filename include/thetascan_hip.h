@@ -83,7 +83,9 @@ typedef struct ts_strided {
 
 typedef struct ts_scan_desc {
   int32_t B, H, T;
-  int32_t dk, dv;       /* feature widths of q/k and v, without ext columns  */
+  int32_t dk, dv;       /* feature widths of q/k and v, without ext columns
+                           (up to 128; bf16 scans without kept, initial or
+                           final states up to 384 keys and 512 values)        */
   int32_t dtype;        /* ts_dtype of q, k, v (and out for TS_OUT_STORE)    */
   int32_t retention;    /* ts_retention                                      */
   int32_t reverse;      /* 1: anti-causal scan (time axis read backwards)    */

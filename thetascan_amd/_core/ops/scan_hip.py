@@ -82,7 +82,21 @@ def _ext_arg(ext):
     return _lib.EXT_ARRAY, ext.to(torch.float32)
 
 
-MAX_WIDTH = 128  # widest key / value width one kernel launch handles
+MAX_WIDTH = 128  # widest key / value block of a carried state, and of an fp32 scan's launch
+# widest keys and values one bf16 call handles (no kept, initial or final states above MAX_WIDTH)
+WIDE_KEYS, WIDE_VALUES = 384, 512
+
+
+def _one_call(dtype: torch.dtype, dk: int, dv: int, out: torch.Tensor | None = None) -> bool:
+    """Whether one ts_scan_fwd call takes these widths (and writes ``out``)."""
+    if dk <= MAX_WIDTH and dv <= MAX_WIDTH:
+        return True
+    if dtype != torch.bfloat16 or dk > WIDE_KEYS or dv > WIDE_VALUES:
+        return False
+    # an output buffer of the kernel's padded width in 16-byte rows; any other
+    # is filled by the block-wise path
+    return out is None or (out.shape[-1] == -(-dv // 8) * 8 and out.stride(-1) == 1 and out.data_ptr() % 16 == 0
+                           and all(s % 8 == 0 for s in out.stride()[:3]))
 
 
 def scan_launch(
@@ -110,7 +124,8 @@ def scan_launch(
     init_state: torch.Tensor | None = None,
     final_out: torch.Tensor | None = None,
 ):
-    """One scan (several kernel launches when a width exceeds ``MAX_WIDTH``).
+    """One scan (several calls when a width exceeds what one takes, see
+    :func:`_one_call`).
 
     Returns ``(out, ext_out, final_state)`` as :func:`_scan_once`.  The scan
     is linear in each operand, so wide values split into independent value
@@ -128,14 +143,16 @@ def scan_launch(
     if workspace is not None or states_in or init_state is not None or final_out is not None:
         if dk > MAX_WIDTH or dv > MAX_WIDTH:
             raise NotImplementedError("hip scan: kept segment states and initial states need widths up to 128")
-    if dk <= MAX_WIDTH and dv <= MAX_WIDTH:
+    if want_final and (dk > MAX_WIDTH or dv > MAX_WIDTH):
+        raise NotImplementedError(f"hip scan: final state of widths dk={dk} dv={dv} above {MAX_WIDTH}")
+    if _one_call(q.dtype, dk, dv, out):
+        if dk > MAX_WIDTH and value_split > 64:
+            value_split = 0  # keys wider than MAX_WIDTH run in 64-column slices at most
         return _scan_once(q, k, v, retention=retention, log_alpha=log_alpha, decay=decay, reverse=reverse,
                           q_ext=q_ext, k_ext=k_ext, v_ext=v_ext, out=out, out_mode=out_mode, out_scale=out_scale,
                           want_ext_out=want_ext_out, ext_out=ext_out, want_final=want_final,
                           seg_chunks=seg_chunks, value_split=value_split, workspace=workspace,
                           states_in=states_in, init_state=init_state, final_out=final_out)
-    if want_final:
-        raise NotImplementedError(f"hip scan: final state of widths dk={dk} dv={dv} above {MAX_WIDTH}")
     kw = dict(retention=retention, log_alpha=log_alpha, decay=decay, reverse=reverse, seg_chunks=seg_chunks,
               value_split=value_split)
     B, H, T = q.shape[:3]
