@@ -802,6 +802,51 @@ int ts_blend_parts(const ts_blend_desc* desc, int32_t* nparts);
 int ts_blend_bwd(const ts_blend_desc* desc, const ts_strided* in, const float* coef, ts_strided dy,
                  const ts_strided* din, float* dcoef_part, hipStream_t stream);
 
+/* ------------------------------------------------------------- bank read */
+
+#define TS_BANK_MAX 8
+
+/* Every view's normalized read, the bank's blend and the output gate in one
+ * pass (engine.py:440-442, 526-528; block.py:683-722; gates.py:34-40):
+ *   y = (sum_j coef[j*H + h] (resid_j + scale num_j / (mass_j + eps))) * silu(g + g_bias)
+ * (without `normalize` scale num_j; without `gate` no silu factor), in fp32
+ * up to the one rounding of y. */
+typedef struct ts_bank_read_desc {
+  int32_t B, H, T, d;
+  int32_t n_views;      /* 1 .. TS_BANK_MAX                                    */
+  int32_t n_resid;      /* 1: one residual for every view; else n_views       */
+  int32_t dtype;        /* of every [B,H,T,d] tensor (16-byte rows)           */
+  int32_t normalize, gate;
+  float scale, eps;
+} ts_bank_read_desc;
+
+typedef struct ts_bank_read_io {
+  ts_strided num[TS_BANK_MAX];
+  ts_strided mass[TS_BANK_MAX];   /* fp32 [B,H,T] (normalize)                 */
+  ts_strided resid[TS_BANK_MAX];
+  ts_strided g;                   /* gate pre-activation (gate)               */
+  const float* coef;              /* fp32 [n_views][H]                        */
+  const float* gbias;             /* fp32 [H*d] or NULL                       */
+} ts_bank_read_io;
+
+int ts_bank_read_fwd(const ts_bank_read_desc* desc, const ts_bank_read_io* io, ts_strided y, hipStream_t stream);
+
+/* Slots of the partial sums ts_bank_read_bwd writes. */
+int ts_bank_read_parts(const ts_bank_read_desc* desc, int32_t* parts);
+
+typedef struct ts_bank_read_grads {
+  ts_strided dy;
+  ts_strided dnum[TS_BANK_MAX];
+  ts_strided dmass[TS_BANK_MAX];  /* fp32 [B,H,T] (normalize)                 */
+  ts_strided dresid[TS_BANK_MAX]; /* n_resid of them; NULL: not wanted        */
+  ts_strided dg;                  /* (gate)                                   */
+  float* dcoef_part;              /* [parts][n_views][H] or NULL              */
+  float* dgb_part;                /* [parts][H*d] (gate) or NULL              */
+} ts_bank_read_grads;
+
+int ts_bank_read_bwd(const ts_bank_read_desc* desc, const ts_bank_read_io* io, const ts_bank_read_grads* grads,
+                     hipStream_t stream);
+
 /* --------------------------------------------------------------- prefixes */
 
 /* Decayed prefix sum along T of an fp32 [B,H,T,F] stream:

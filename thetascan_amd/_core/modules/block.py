@@ -552,25 +552,33 @@ class ThetaScan(nn.Module):
         weights = self._weights()
         sharp = self.kernel_sharpness()
         controls = self.kernel_controls()
-        gate = self._read_gate(x, views)
+        request = self._read_gate(x, views, etas)
         reads = composed.memory_forward(weights, cfg, k, v_w, q, tuple(views), hrot=hrot, gain=sharp,
-                                        controls=controls, out_gate=gate)
-        if gate is not None and gate.applied:
-            # the read epilogue applied the output gate and wrote its output
-            # token-major: the projection reads it as [B,T,H*d] in place
-            return linear(reads[0].transpose(1, 2).reshape(B, T, H * d), self.proj_out.weight)
+                                        controls=controls, out_gate=request)
+        if request is not None and request.applied:
+            return self._project_out(reads[0])
         return self._blend_and_project(x, reads, etas)
 
-    def _read_gate(self, x: torch.Tensor, views):
-        """The output gate (block.py:721-722) as a request that the HIP read
-        epilogue of a single view may apply (composed.GateRequest), or None
-        where the gate stays a product after the read (banks: after the
-        blend)."""
+    def _read_gate(self, x: torch.Tensor, views, etas):
+        """The blend of a fast bank (block.py:683-695) and the output gate
+        (block.py:721-722) as a request that the HIP read epilogue may apply
+        (composed.OutputRequest), or None where there is nothing to apply or
+        it stays with the caller (a stale bank's views differ in dtype)."""
         cfg = self.cfg
-        if self.ogate is None or cfg.read_fade or len(views) != 1 or not x.is_cuda:
+        if not x.is_cuda or len(views) != 1 + len(etas) or (cfg.read_fade and cfg.read_fade_mode != "fast"):
             return None
-        lin = self.ogate.g.lin
-        return composed.GateRequest(x, lin.weight, lin.bias, cfg.n_heads, cfg.head_dim)
+        coef = maps.fast_coefficients(etas) if cfg.read_fade else None
+        if coef is None and self.ogate is None:
+            return None
+        lin = None if self.ogate is None else self.ogate.g.lin
+        return composed.OutputRequest(x, None if lin is None else lin.weight, None if lin is None else lin.bias,
+                                      cfg.n_heads, cfg.head_dim, coef)
+
+    def _project_out(self, y: torch.Tensor) -> torch.Tensor:
+        """The output projection of a read written token-major: [B,H,T,d] read
+        as [B,T,H*d] in place."""
+        B, H, T, d = y.shape
+        return linear(y.transpose(1, 2).reshape(B, T, H * d), self.proj_out.weight)
 
     def _temporal_views(self, x: torch.Tensor, backend: str):
         """The memory's temporal views (interface.py:198-327): the accumulator
@@ -647,5 +655,9 @@ class ThetaScan(nn.Module):
             pairs = interface.scan_views_mass(tuple(views), phi_q, phi_k, v_w, "m")
         else:
             pairs = [(num, None) for num in interface.scan_views(tuple(views), phi_q, phi_k, v_w, "m")]
+        nums, masses = [p[0] for p in pairs], [p[1] for p in pairs]
+        request = self._read_gate(x, views, etas)
+        if request is not None and request.fits(nums, masses, [resid]):
+            return self._project_out(request.read(nums, masses, [resid], s, cfg.eps))
         reads = [gn.normalized_read(num, mass, resid, s=s, eps=cfg.eps) for num, mass in pairs]
         return self._blend_and_project(x, reads, etas)

@@ -26,7 +26,7 @@ depth-1 GN writes and reads of the HIP GN kernels (``gn.write``,
 ``gn.read_stage``), every other GN block's RMSNorm, nonlinearity and Jacobian
 scales (``gn.act_rows``: any depth, both Gauss-Newton steps, SwiGLU), the
 normalized read epilogue in ``gn.normalized_read`` (HIP; with one view it
-also applies the output gate, see ``GateRequest``) and the per-head GEMMs in
+also applies the output gate, see ``OutputRequest``) and the per-head GEMMs in
 ``linear.head_matmul``.  The remaining elementwise work (the
 products of the scales with the GEMM outputs, the Jacobi division) is torch
 on the GPU.
@@ -39,48 +39,65 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 
-from . import gn, interface, kernel_features, maps
+from . import bankread, gn, interface, kernel_features, maps
 from .linear import head_matmul
 from ..modules.norms import rmsnorm
 
 
 # ------------------------------------------------------------------ output gate
 
-class GateRequest:
-    """An output gate silu(x W_g^T + b) (block.py:721-722) that the read
-    epilogue of a single view may apply.  ``pre`` is the [B,H,T,d] view of
-    the pre-activation x W_g^T without the bias, formed on first use (so a
-    read that does not take the gate costs no GEMM).  A read that applies
-    silu(pre + bias) inside its HIP epilogue writes its output token-major
-    (``gn.normalized_read``) and sets ``applied``; otherwise the caller
-    applies the gate itself."""
+class OutputRequest:
+    """What follows the reads of the last level, for a read epilogue that can
+    apply it: the blend of a bank's views (``coef`` [n,H], block.py:683-717;
+    None for a single view) and the output gate silu(x W_g^T + b)
+    (block.py:721-722; ``weight`` None: no gate).  ``pre`` is the [B,H,T,d]
+    view of the gate's pre-activation x W_g^T without the bias, formed on
+    first use (so a read that does not take the gate costs no GEMM).  A read
+    that applies the request in its HIP epilogue returns the one blended,
+    gated output, written token-major (``gn.normalized_read``,
+    ``bankread.bank_read``), and sets ``applied``; otherwise the caller blends
+    and gates the views' reads itself."""
 
-    def __init__(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, heads: int, width: int):
+    def __init__(self, x: torch.Tensor, weight: torch.Tensor | None, bias: torch.Tensor | None, heads: int,
+                 width: int, coef: torch.Tensor | None = None):
         self.x, self.weight, self.bias = x, weight, bias
         self.heads, self.width = heads, width
+        self.coef = coef
         self.applied = False
         self._pre = None
 
     @property
-    def pre(self) -> torch.Tensor:
-        if self._pre is None:
+    def pre(self) -> torch.Tensor | None:
+        if self._pre is None and self.weight is not None:
             from .linear import linear
 
             B, T, _ = self.x.shape
             self._pre = linear(self.x, self.weight).view(B, T, self.heads, self.width).transpose(1, 2)
         return self._pre
 
-    def fits(self, num: torch.Tensor, resid: torch.Tensor) -> bool:
-        """Whether the HIP read epilogue can apply the gate to this read."""
+    def fits(self, nums, masses, resids) -> bool:
+        """Whether a HIP read epilogue can apply this request to these reads
+        (``resids``: one residual for every view, or one each)."""
+        num = nums[0]
         B, T, _ = self.x.shape
-        return (num.is_cuda and num.dtype in (torch.bfloat16, torch.float32) and resid.dtype == num.dtype
-                and self.x.dtype == num.dtype and self.weight.dtype == num.dtype
-                and tuple(num.shape) == (B, self.heads, T, self.width) and resid.shape == num.shape)
+        if len(nums) != (1 if self.coef is None else self.coef.shape[0]):
+            return False
+        if self.weight is not None and not (self.x.dtype == num.dtype and self.weight.dtype == num.dtype):
+            return False
+        if tuple(num.shape) != (B, self.heads, T, self.width):
+            return False
+        if self.coef is not None:
+            return bankread.eligible(nums, masses, resids, self.heads)
+        return (self.weight is not None and num.is_cuda and num.dtype in (torch.bfloat16, torch.float32)
+                and resids[0].dtype == num.dtype and resids[0].shape == num.shape)
 
-    def read(self, num, mass, resid, s: float, eps: float) -> torch.Tensor:
-        """The gated read epilogue (marks the gate applied)."""
+    def read(self, nums, masses, resids, s: float, eps: float) -> torch.Tensor:
+        """The blended, gated read (marks the request applied)."""
         self.applied = True
-        return gn.normalized_read(num, mass, resid, s=s, eps=eps, gate=self.pre, gate_bias=self.bias)
+        if self.coef is not None:
+            return bankread.bank_read(nums, masses, resids, self.coef, s=s, eps=eps, gate=self.pre,
+                                      gate_bias=self.bias if self.weight is not None else None)
+        return gn.normalized_read(nums[0], masses[0], resids[0], s=s, eps=eps, gate=self.pre, gate_bias=self.bias)
 
 
 # ------------------------------------------------------------------ per-head products
@@ -426,13 +443,13 @@ class FastNet:
     def recall(self, q, steps, views):
         """f_theta_t(q_t) for every temporal view (engine.py:345-544)."""
         outs = [q] * len(views)
-        gate = self.out_gate if len(views) == 1 else None
+        gate = self.out_gate
         for l in range(len(self.layers)):
             last = gate if l == len(self.layers) - 1 else None
             if all(x is outs[0] for x in outs):
                 outs = self._read_layer(list(views), l, outs[0], steps, last)
             else:
-                outs = [self._read_layer([view], l, x, steps, last)[0] for view, x in zip(views, outs)]
+                outs = [self._read_layer([view], l, x, steps)[0] for view, x in zip(views, outs)]
         return tuple(outs)
 
     def _features_at(self, l, main, gate):
@@ -489,7 +506,7 @@ class FastNet:
 
     def _read_layer(self, group, l, x, steps, out_gate=None):
         """One depth level for the views of ``group``, which share the input
-        ``x``; ``out_gate`` is a ``GateRequest`` the last level may apply."""
+        ``x``; ``out_gate`` is an ``OutputRequest`` the last level may apply."""
         cfg = self.cfg
         if gn.read_eligible(cfg, self.layers, x):
             return self._read_layer_gn(group, l, x, steps, out_gate)
@@ -549,8 +566,9 @@ class FastNet:
                      for view, (num, mass) in zip(group, interface.scan_views_mass(group, hq, dep.feat, dep.pay, "m"))]
         else:
             pairs = [(num, None) for num in interface.scan_views(group, hq, dep.feat, dep.pay, "m")]
-        if out_gate is not None and len(pairs) == 1 and out_gate.fits(pairs[0][0], resid):
-            return [out_gate.read(pairs[0][0], pairs[0][1], resid, self.s, cfg.eps)]
+        nums, masses = [p[0] for p in pairs], [p[1] for p in pairs]
+        if out_gate is not None and out_gate.fits(nums, masses, [resid]):
+            return [out_gate.read(nums, masses, [resid], self.s, cfg.eps)]
         return [gn.normalized_read(num, mass, resid, s=self.s, eps=cfg.eps) for num, mass in pairs]
 
     def _read_layer_gn(self, group, l, x, steps, out_gate=None):
@@ -575,7 +593,7 @@ class FastNet:
                      for corr in interface.scan_views(group, x, dep.inp, dep.jac, "d")]
         else:
             stage = [(None, None, gn.READ_NONE)] * len(group)
-        outs = []
+        nums, masses, resids = [], [], []
         for view, (num1, mass1, kind) in zip(group, stage):
             h, resid = gn.read_stage(x, W1, W2, tau, num1, mass1, corr=kind, want_resid=True, s=self.s, eps=cfg.eps,
                                      nonlin=cfg.nonlin)
@@ -585,11 +603,13 @@ class FastNet:
                 mass2 = key_mass(cfg, view, hq, dep.feat, mass2)
             else:
                 num2, mass2 = interface.scan_views((view,), hq, dep.feat, dep.pay, "m")[0], None
-            if out_gate is not None and len(group) == 1 and out_gate.fits(num2, resid):
-                outs.append(out_gate.read(num2, mass2, resid, self.s, cfg.eps))
-            else:
-                outs.append(gn.normalized_read(num2, mass2, resid, s=self.s, eps=cfg.eps))
-        return outs
+            nums.append(num2)
+            masses.append(mass2)
+            resids.append(resid)
+        if out_gate is not None and out_gate.fits(nums, masses, resids):
+            return [out_gate.read(nums, masses, resids, self.s, cfg.eps)]
+        return [gn.normalized_read(num, mass, resid, s=self.s, eps=cfg.eps)
+                for num, mass, resid in zip(nums, masses, resids)]
 
 
 @dataclass(frozen=True)
@@ -602,6 +622,7 @@ class _Written(Deposit):
 def memory_forward(layers, cfg, k, v, q, views, hrot=None, gain=None, controls=None, out_gate=None):
     """The memory read f_theta_t(q_t) of every temporal view after writing
     keys ``k`` and values ``v`` (engine.py:260-553).  ``out_gate`` is an
-    optional ``GateRequest`` (its ``applied`` tells whether the read took it)."""
+    optional ``OutputRequest`` (its ``applied`` tells whether the reads took it;
+    one blended, gated output is returned then)."""
     net = FastNet(layers, cfg, hrot=hrot, gain=gain, controls=controls, out_gate=out_gate)
     return net.recall(q, net.deposits(k, v), views)

@@ -408,6 +408,28 @@ class GnReadBwdIO(ctypes.Structure):
     ]
 
 
+BANK_MAX = 8  # views of one ts_bank_read call
+
+
+class BankReadDesc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("B", "H", "T", "d", "n_views", "n_resid", "dtype", "normalize", "gate")] + [
+        ("scale", ctypes.c_float), ("eps", ctypes.c_float)]
+
+
+class BankReadIO(ctypes.Structure):
+    _fields_ = [
+        ("num", Strided * BANK_MAX), ("mass", Strided * BANK_MAX), ("resid", Strided * BANK_MAX), ("g", Strided),
+        ("coef", ctypes.c_void_p), ("gbias", ctypes.c_void_p),
+    ]
+
+
+class BankReadGrads(ctypes.Structure):
+    _fields_ = [
+        ("dy", Strided), ("dnum", Strided * BANK_MAX), ("dmass", Strided * BANK_MAX), ("dresid", Strided * BANK_MAX),
+        ("dg", Strided), ("dcoef_part", ctypes.c_void_p), ("dgb_part", ctypes.c_void_p),
+    ]
+
+
 class BlendDesc(ctypes.Structure):
     _fields_ = [
         ("B", ctypes.c_int32),
@@ -566,6 +588,9 @@ def load() -> ctypes.CDLL:
         lib.ts_blend_parts.argtypes = [P(BlendDesc), P(ctypes.c_int32)]
         lib.ts_blend_bwd.argtypes = [P(BlendDesc), P(Strided), ctypes.c_void_p, Strided, P(Strided),
                                      ctypes.c_void_p, ctypes.c_void_p]
+        lib.ts_bank_read_fwd.argtypes = [P(BankReadDesc), P(BankReadIO), Strided, ctypes.c_void_p]
+        lib.ts_bank_read_parts.argtypes = [P(BankReadDesc), P(ctypes.c_int32)]
+        lib.ts_bank_read_bwd.argtypes = [P(BankReadDesc), P(BankReadIO), P(BankReadGrads), ctypes.c_void_p]
         lib.ts_gn_write_fwd.argtypes = [P(GnDesc), P(GnIO), ctypes.c_void_p]
         lib.ts_gn_write_bwd.argtypes = [P(GnDesc), P(GnBwdIO), ctypes.c_void_p]
         lib.ts_gn_read_fwd.argtypes = [P(GnReadDesc), P(GnReadIO), ctypes.c_void_p]
