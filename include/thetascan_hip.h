@@ -802,6 +802,38 @@ int ts_blend_parts(const ts_blend_desc* desc, int32_t* nparts);
 int ts_blend_bwd(const ts_blend_desc* desc, const ts_strided* in, const float* coef, ts_strided dy,
                  const ts_strided* din, float* dcoef_part, hipStream_t stream);
 
+/* ------------------------------------------- backward of several retentions */
+
+/* The gradients of ts_scan_views_fwd's views (retention none or static) for
+ * upstream dout_r (and dmass_r of the key mass), summed over the views:
+ *   dq_t = sum_r sum_{i<=t} alpha_r^(t-i) (<dout_r,t, v_i> + dmass_r,t) k_i
+ *   dk_i = sum_r sum_{t>=i} alpha_r^(t-i) (<dout_r,t, v_i> + dmass_r,t) q_t
+ *   dv_i = sum_r sum_{t>=i} alpha_r^(t-i) <q_t, k_i> dout_r,t
+ * One causal and one anti-causal pass; the sums over views are formed in fp32
+ * and rounded once. */
+typedef struct ts_views_bwd_desc {
+  int32_t B, H, T;
+  int32_t m, dv;        /* feature widths: m <= 512, dv <= 64 (multiples of 8) */
+  int32_t dtype;        /* TS_BF16                                             */
+  int32_t n_views;      /* 2 .. TS_MAX_VIEWS                                   */
+  int32_t mass;         /* 1: dmass given for every view                       */
+  int32_t seg_chunks;   /* 64-token tiles per workgroup segment; 0 = auto      */
+} ts_views_bwd_desc;
+
+typedef struct ts_views_bwd_io {
+  ts_strided q, k, v;                   /* [B,H,T,m], [B,H,T,m], [B,H,T,dv]    */
+  ts_strided dout[TS_MAX_VIEWS];        /* [B,H,T,dv]                          */
+  ts_strided dmass[TS_MAX_VIEWS];       /* fp32 [B,H,T] (mass)                 */
+  const float* log_alpha[TS_MAX_VIEWS]; /* [H], NULL: no retention             */
+  ts_strided dq, dk;                    /* [B,H,T,m] (ptr NULL: not wanted)    */
+  void* dv;                             /* contiguous [B,H,T,dv]; with dk      */
+} ts_views_bwd_io;
+
+int ts_views_bwd_workspace_bytes(const ts_views_bwd_desc* desc, size_t* bytes);
+
+int ts_views_bwd(const ts_views_bwd_desc* desc, const ts_views_bwd_io* io, void* workspace, size_t workspace_bytes,
+                 hipStream_t stream);
+
 /* ------------------------------------------------------------- bank read */
 
 #define TS_BANK_MAX 8

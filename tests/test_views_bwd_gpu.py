@@ -1,0 +1,90 @@
+"""ts_views_bwd (the gradients of several retentions' scans in one causal and
+one anti-causal pass) against float64 autograd through the tiled recurrence
+(GPU tests).
+
+Bar: rel 2e-2 of the largest value (bf16 operands; the score sums enter as
+hi + lo, the weighted values and the published states as bf16).  Widths at
+the edges of the 64-column slices, sequences that end inside a tile, one
+segment and several, with and without the key mass, two and three views.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import scans as oracle
+from tests.conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+RATES = (None, (0.9, 0.97), (0.99, 0.5))
+
+
+@pytest.mark.parametrize("n", [2, 3])
+@pytest.mark.parametrize("mass", [False, True])
+@pytest.mark.parametrize("m,dv", [(64, 64), (8, 8), (72, 64), (128, 40), (384, 64)])
+def test_views_backward_matches_float64(cuda, n, mass, m, dv):
+    from thetascan_amd._core.ops import scan_hip
+
+    for T, seg in ((1, 0), (64, 0), (333, 0), (333, 2), (450, 1)):
+        g = torch.Generator().manual_seed(m + dv + T)
+        B, H = 2, 2
+        q, k = ((torch.rand(B, H, T, m, generator=g, dtype=torch.float64) * 2 / m).to(torch.bfloat16) for _ in range(2))
+        # values as the stacked projection holds them: token-major rows
+        v = torch.randn(B, T, H, dv, generator=g, dtype=torch.float64).to(torch.bfloat16).transpose(1, 2)
+        dos = [torch.randn(B, H, T, dv, generator=g, dtype=torch.float64).to(torch.bfloat16) for _ in range(n)]
+        dms = [torch.randn(B, H, T, generator=g, dtype=torch.float64).float() for _ in range(n)] if mass else None
+        las = [None if r is None else torch.log(torch.tensor(r, dtype=torch.float64)) for r in RATES[:n]]
+        leaves = [t.double().requires_grad_(True) for t in (q, k, v)]
+        vx = torch.cat([leaves[2], torch.ones_like(leaves[2][..., :1])], -1) if mass else leaves[2]
+        loss = 0.0
+        for j, la in enumerate(las):
+            out = oracle.linattn_chunk(leaves[0], leaves[1], vx, None if la is None else oracle.as_stream(la, leaves[0]))
+            loss = loss + (out[..., :dv] * dos[j].double()).sum()
+            if mass:
+                loss = loss + (out[..., dv] * dms[j].double()).sum()
+        loss.backward()
+        dev = lambda ts: None if ts is None else [None if t is None else t.to(cuda) for t in ts]  # noqa: E731
+        got = scan_hip.views_bwd_launch(q.to(cuda), k.to(cuda), v.to(cuda), dev(las), dev(dos), dev(dms), need_q=True,
+                                        need_kv=True, seg_chunks=seg)
+        for name, a, e in zip(("dq", "dk", "dv"), got, leaves):
+            assert a.shape == e.shape and a.dtype == torch.bfloat16
+            assert rel_err(a, e.grad) < 2e-2, (name, T, seg)
+        only_q = scan_hip.views_bwd_launch(q.to(cuda), k.to(cuda), v.to(cuda), dev(las), dev(dos), dev(dms),
+                                           need_q=True, need_kv=False, seg_chunks=seg)
+        assert only_q[1] is None and only_q[2] is None and torch.equal(only_q[0], got[0])
+
+
+def test_bank_of_static_views_takes_the_passes(cuda):
+    """The gradients of a bank's views through autograd run in ts_views_bwd,
+    and equal the per-view scans' to bf16 rounding."""
+    from thetascan_amd import _lib
+    from thetascan_amd._core.ops import scan_hip
+
+    g = torch.Generator().manual_seed(3)
+    B, H, T, m, dv = 2, 2, 200, 64, 64
+    base = [torch.rand(B, H, T, m, generator=g).to(cuda, torch.bfloat16) / 32 for _ in range(2)]
+    base.append(torch.randn(B, H, T, dv, generator=g).to(cuda, torch.bfloat16))
+    la = torch.log(torch.tensor([0.9, 0.97], device=cuda))
+    dys = [torch.randn(B, H, T, dv, generator=g).to(cuda, torch.bfloat16) for _ in range(2)]
+
+    def run():
+        ts = [t.clone().requires_grad_(True) for t in base]
+        r = la.clone().requires_grad_(True)
+        with _lib.record_launches() as recs:
+            outs = scan_hip.linattn_views(*ts, (None, r), 64)
+            torch.autograd.backward(outs, dys)
+            torch.cuda.synchronize()
+        return [t.grad for t in ts] + [r.grad], {rec[0] for rec in recs}
+
+    got, names = run()
+    assert "ts_views_bwd" in names and "ts_scan_pair_fwd" not in names
+    real = scan_hip.views_bwd_eligible
+    try:
+        scan_hip.views_bwd_eligible = lambda *a: False
+        want, names = run()
+    finally:
+        scan_hip.views_bwd_eligible = real
+    assert "ts_views_bwd" not in names
+    for a, e in zip(got, want):
+        assert rel_err(a, e) < 1e-2

@@ -452,6 +452,59 @@ def views_eligible(q: torch.Tensor, v: torch.Tensor, kinds) -> bool:
             and q.shape[-1] <= 128 and v.shape[-1] <= 64)
 
 
+def views_bwd_eligible(q: torch.Tensor, v: torch.Tensor, kinds) -> bool:
+    """Whether ts_views_bwd forms these views' gradients: bf16 on the GPU, 2
+    or 3 retentions that are none or static, m <= 512, dv <= 64, and (batch,
+    head) slices of 31-bit offsets."""
+    B, H, T, m = q.shape
+    return (q.is_cuda and q.dtype == torch.bfloat16 and 2 <= len(kinds) <= _lib.MAX_VIEWS
+            and all(k in (_lib.RET_NONE, _lib.RET_STATIC) for k in kinds)
+            and m <= 512 and v.shape[-1] <= 64 and B * H * (-(-m // 64)) <= 65535 and T * 64 * 4 < 1 << 31)
+
+
+def views_bwd_launch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, log_alphas, d_outs, d_mass, *,
+                     need_q: bool, need_kv: bool, seg_chunks: int = 0):
+    """(dq, dk, dv) of every view's scan summed over the views (``log_alphas``:
+    [H] or None per view; ``d_outs`` [B,H,T,dv] per view; ``d_mass`` fp32
+    [B,H,T] per view or None): one causal pass for dq, one anti-causal pass for
+    dk and dv (None where not wanted)."""
+    lib = _lib.load()
+    B, H, T, m = q.shape
+    dv = v.shape[-1]
+    mw, vw = -(-m // 8) * 8, -(-dv // 8) * 8
+    qk, kk, vk = _kernel_view(q, mw), _kernel_view(k.to(q.dtype), mw), _kernel_view(v.to(q.dtype), vw)
+    dos = [_kernel_view(t.to(q.dtype), vw) for t in d_outs]
+    dms = None if d_mass is None else [t.detach().to(torch.float32) for t in d_mass]
+    las = [None if la is None else la.detach().to(device=q.device, dtype=torch.float32).reshape(H).contiguous()
+           for la in log_alphas]
+    n = len(las)
+    desc = _lib.ViewsBwdDesc(B, H, T, mw, vw, _lib.dtype_code(q.dtype), n, int(dms is not None), int(seg_chunks))
+    nb = ctypes.c_size_t()
+    _lib.check(lib.ts_views_bwd_workspace_bytes(ctypes.byref(desc), ctypes.byref(nb)), "views bwd workspace")
+    work = torch.empty(nb.value, dtype=torch.uint8, device=q.device) if nb.value else None
+    gq = torch.empty(B, H, T, mw, dtype=q.dtype, device=q.device) if need_q else None
+    gk = torch.empty(B, H, T, mw, dtype=q.dtype, device=q.device) if need_kv else None
+    gv = torch.empty(B, H, T, vw, dtype=q.dtype, device=q.device) if need_kv else None
+    pad = [_lib.strided(None)] * (_lib.MAX_VIEWS - n)
+    io = _lib.ViewsBwdIO(
+        _lib.strided(qk), _lib.strided(kk), _lib.strided(vk),
+        (_lib.Strided * _lib.MAX_VIEWS)(*[_lib.strided(t) for t in dos], *pad),
+        (_lib.Strided * _lib.MAX_VIEWS)(*[_lib.strided(t) for t in dms or []]),
+        (ctypes.c_void_p * _lib.MAX_VIEWS)(*[None if la is None else la.data_ptr() for la in las]),
+        _lib.strided(gq), _lib.strided(gk), _lib.ptr(gv))
+
+    def traffic():
+        once = _lib.nbytes(vk, *dos, *(dms or []))
+        return (once + _lib.nbytes(kk, gq) if need_q else 0) + (once + _lib.nbytes(qk, kk, gk, gv) if need_kv else 0)
+
+    with _lib.timed("ts_views_bwd", traffic):
+        status = lib.ts_views_bwd(ctypes.byref(desc), ctypes.byref(io), _lib.ptr(work), nb.value,
+                                  _lib.stream_handle(q.device))
+    _lib.check(status, "ts_views_bwd")
+    return (None if gq is None else gq[..., :m], None if gk is None else gk[..., :m],
+            None if gv is None else gv[..., :dv])
+
+
 def scan_views_launch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, log_alphas, *, mass: bool,
                       seg_chunks: int = 0):
     """Forward causal scans of the same q, k, v under several retentions in one
@@ -636,6 +689,16 @@ def _views_backward(q, k, v, retentions, d_outs, d_mass, need_q: bool, need_k: b
         if need_v:
             gv = scan_launch(k, q, dO, **rk, reverse=True)[0][..., :dv]
         return gq, gk, gv, [None]
+    if (views_bwd_eligible(q, v, kinds) and all(d is not None for d in d_outs) and need_k == need_v
+            and (need_q or need_k) and len({d is None for d in d_mass}) == 1):
+        # every view's gradient in one causal and one anti-causal pass; static
+        # retentions' gradients are summed pair by pair
+        dms = None if d_mass[0] is None else list(d_mass)
+        las = [r if kind == _lib.RET_STATIC else None for kind, r in zip(kinds, retentions)]
+        r_grads = [retention_grad(q, k, v, d_outs[j].to(q.dtype), d_mass[j], r).sum(0).to(r.dtype).view_as(r)
+                   if r is not None and need_r[j] else None for j, r in enumerate(retentions)]
+        gq, gk, gv = views_bwd_launch(q, k, v, las, d_outs, dms, need_q=need_q, need_kv=need_k)
+        return gq, None if gk is None else gk.to(k.dtype), None if gv is None else gv.to(v.dtype), r_grads
     # the first scan into each fp32 gradient stores, later ones accumulate;
     # a gradient no scan wrote is zeroed at the end
     dq = torch.empty(B, H, T, -(-dk // _vec(q.dtype)) * _vec(q.dtype), dtype=torch.float32, device=q.device)

@@ -408,6 +408,17 @@ class GnReadBwdIO(ctypes.Structure):
     ]
 
 
+class ViewsBwdDesc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("B", "H", "T", "m", "dv", "dtype", "n_views", "mass", "seg_chunks")]
+
+
+class ViewsBwdIO(ctypes.Structure):
+    _fields_ = [
+        ("q", Strided), ("k", Strided), ("v", Strided), ("dout", Strided * MAX_VIEWS), ("dmass", Strided * MAX_VIEWS),
+        ("log_alpha", ctypes.c_void_p * MAX_VIEWS), ("dq", Strided), ("dk", Strided), ("dv", ctypes.c_void_p),
+    ]
+
+
 BANK_MAX = 8  # views of one ts_bank_read call
 
 
@@ -588,6 +599,8 @@ def load() -> ctypes.CDLL:
         lib.ts_blend_parts.argtypes = [P(BlendDesc), P(ctypes.c_int32)]
         lib.ts_blend_bwd.argtypes = [P(BlendDesc), P(Strided), ctypes.c_void_p, Strided, P(Strided),
                                      ctypes.c_void_p, ctypes.c_void_p]
+        lib.ts_views_bwd_workspace_bytes.argtypes = [P(ViewsBwdDesc), P(ctypes.c_size_t)]
+        lib.ts_views_bwd.argtypes = [P(ViewsBwdDesc), P(ViewsBwdIO), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         lib.ts_bank_read_fwd.argtypes = [P(BankReadDesc), P(BankReadIO), Strided, ctypes.c_void_p]
         lib.ts_bank_read_parts.argtypes = [P(BankReadDesc), P(ctypes.c_int32)]
         lib.ts_bank_read_bwd.argtypes = [P(BankReadDesc), P(BankReadIO), P(BankReadGrads), ctypes.c_void_p]
