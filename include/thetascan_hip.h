@@ -879,6 +879,23 @@ typedef struct ts_bank_read_grads {
 int ts_bank_read_bwd(const ts_bank_read_desc* desc, const ts_bank_read_io* io, const ts_bank_read_grads* grads,
                      hipStream_t stream);
 
+/* A fast bank's parameters (block.py:647-695): log_alpha_j = -softplus(-alpha_j)
+ * ([H] fp32 each, the values rounded to param_dtype and then stream_dtype) and
+ * coef [n+1][H] = (1 - sum_j e_j, e_1 ..), e = eta or tanh(eta); alpha, eta
+ * [n][H] of param_dtype.  The backward takes dlog_alpha_j (entries may be
+ * NULL) and dcoef (or NULL). */
+typedef struct ts_bank_params_desc {
+  int32_t n, H;         /* branches (1 .. TS_BANK_MAX - 1), heads             */
+  int32_t tanh_eta;
+  int32_t param_dtype, stream_dtype;
+} ts_bank_params_desc;
+
+int ts_bank_params_fwd(const ts_bank_params_desc* desc, const void* alpha, const void* eta, float* const* log_alpha,
+                       float* coef, hipStream_t stream);
+int ts_bank_params_bwd(const ts_bank_params_desc* desc, const void* alpha, const void* eta,
+                       const float* const* dlog_alpha, const float* dcoef, void* dalpha, void* deta,
+                       hipStream_t stream);
+
 /* --------------------------------------------------------------- prefixes */
 
 /* Decayed prefix sum along T of an fp32 [B,H,T,F] stream:

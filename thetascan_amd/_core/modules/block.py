@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from ..config import ThetaScanConfig
 from ...state import ThetaScanState, config_fingerprint
-from ..ops import composed, features, fused, gn, interface, maps, prologue, stream
+from ..ops import bankread, composed, features, fused, gn, interface, maps, prologue, stream
 from ..ops.linear import linear, stack_heads
 from ..ops.interface import Accumulator, FadeFast, FadeStale, NullAccumulator, resolve_backend
 from .gates import DecayGate, OutGate
@@ -548,26 +548,25 @@ class ThetaScan(nn.Module):
             if rot:
                 hcos, hsin = rope_cache(T, rot, cfg.rope_base, x.device, x.dtype)
                 hrot = (hcos, hsin, rot)
-        views, etas = self._temporal_views(x, backend)
+        views, coef = self._temporal_views(x, backend)
         weights = self._weights()
         sharp = self.kernel_sharpness()
         controls = self.kernel_controls()
-        request = self._read_gate(x, views, etas)
+        request = self._read_gate(x, views, coef)
         reads = composed.memory_forward(weights, cfg, k, v_w, q, tuple(views), hrot=hrot, gain=sharp,
                                         controls=controls, out_gate=request)
         if request is not None and request.applied:
             return self._project_out(reads[0])
-        return self._blend_and_project(x, reads, etas)
+        return self._blend_and_project(x, reads, coef)
 
-    def _read_gate(self, x: torch.Tensor, views, etas):
+    def _read_gate(self, x: torch.Tensor, views, coef):
         """The blend of a fast bank (block.py:683-695) and the output gate
         (block.py:721-722) as a request that the HIP read epilogue may apply
         (composed.OutputRequest), or None where there is nothing to apply or
         it stays with the caller (a stale bank's views differ in dtype)."""
         cfg = self.cfg
-        if not x.is_cuda or len(views) != 1 + len(etas) or (cfg.read_fade and cfg.read_fade_mode != "fast"):
+        if not x.is_cuda or (cfg.read_fade and cfg.read_fade_mode != "fast"):
             return None
-        coef = maps.fast_coefficients(etas) if cfg.read_fade else None
         if coef is None and self.ogate is None:
             return None
         lin = None if self.ogate is None else self.ogate.g.lin
@@ -583,7 +582,8 @@ class ThetaScan(nn.Module):
     def _temporal_views(self, x: torch.Tensor, backend: str):
         """The memory's temporal views (interface.py:198-327): the accumulator
         (plain sum or the ema stream) and, for a bank, one fast or stale view
-        per recency branch (block.py:647-681), with the branches' blends."""
+        per recency branch (block.py:647-681), with the bank's blend
+        coefficients over the views' reads (block.py:683-717; None otherwise)."""
         cfg = self.cfg
         B, T, _ = x.shape
         H = cfg.n_heads
@@ -592,33 +592,38 @@ class ThetaScan(nn.Module):
             decay_d, decay_m = self.decay(x)
         acc = Accumulator(backend, decay_d=decay_d, decay_m=decay_m, eps=cfg.eps, chunk=cfg.scan_chunk)
         views = [acc]
-        etas = []
-        if cfg.read_fade:
-            alpha_raw = self.fade_alpha
-            eta = self.fade_blends()
-            if alpha_raw.ndim == 1:
-                alpha_raw, eta = alpha_raw.unsqueeze(0), eta.unsqueeze(0)
-            for branch in range(cfg.fade_branches):
-                log_alpha = (-F.softplus(-alpha_raw[branch])).to(dtype=x.dtype)
-                la_s = log_alpha.view(1, H, 1, 1).expand(B, H, T, 1)
-                fast = Accumulator(backend, decay_d=la_s, decay_m=la_s, eps=cfg.eps, chunk=cfg.scan_chunk,
-                                   static_log_alpha=log_alpha)
-                if cfg.read_fade_mode == "fast":
-                    views.append(FadeFast(fast, log_alpha, chunk=cfg.scan_chunk))
-                else:
-                    views.append(FadeStale(acc, fast, log_alpha, cfg.scan_chunk))
-                etas.append(eta[branch].view(1, -1, 1, 1))
-            if cfg.read_fade_mode == "stale":
-                views.append(NullAccumulator())
-        return views, etas
+        if not cfg.read_fade:
+            return views, None
+        fast_bank = cfg.read_fade_mode == "fast"
+        alpha_raw, eta = self.fade_alpha, self.fade_eta
+        if alpha_raw.ndim == 1:
+            alpha_raw, eta = alpha_raw.unsqueeze(0), eta.unsqueeze(0)
+        if fast_bank and bankread.params_eligible(alpha_raw, eta, x.dtype):
+            # retentions and blend in one launch
+            log_alphas, coef = bankread.bank_params(alpha_raw, eta, cfg.fade_blend_mode == "tanh", x.dtype)
+        else:
+            log_alphas = [(-F.softplus(-alpha_raw[j])).to(dtype=x.dtype) for j in range(cfg.fade_branches)]
+            blends = self.fade_blends().reshape(eta.shape)
+            etas = [blends[j].view(1, -1, 1, 1) for j in range(cfg.fade_branches)]
+            coef = maps.fast_coefficients(etas) if fast_bank else maps.stale_coefficients(etas)
+        for log_alpha in log_alphas:
+            la_s = log_alpha.view(1, H, 1, 1).expand(B, H, T, 1)
+            fast = Accumulator(backend, decay_d=la_s, decay_m=la_s, eps=cfg.eps, chunk=cfg.scan_chunk,
+                               static_log_alpha=log_alpha)
+            if fast_bank:
+                views.append(FadeFast(fast, log_alpha, chunk=cfg.scan_chunk))
+            else:
+                views.append(FadeStale(acc, fast, log_alpha, cfg.scan_chunk))
+        if not fast_bank:
+            views.append(NullAccumulator())
+        return views, coef
 
-    def _blend_and_project(self, x: torch.Tensor, reads, etas) -> torch.Tensor:
+    def _blend_and_project(self, x: torch.Tensor, reads, coef) -> torch.Tensor:
         """Bank blend (block.py:683-717), output gate and projection (block.py:721-724)."""
         cfg = self.cfg
         B, T, _ = x.shape
         y = reads[0]
         if cfg.read_fade:
-            coef = maps.fast_coefficients(etas) if cfg.read_fade_mode == "fast" else maps.stale_coefficients(etas)
             if (self.ogate is not None and not torch.is_grad_enabled() and x.is_cuda
                     and all(r.dtype == x.dtype for r in reads) and self.ogate.g.lin.weight.dtype == x.dtype):
                 # inference: the output gate in the blend's epilogue (one
@@ -649,15 +654,15 @@ class ThetaScan(nn.Module):
         tau = self.kernel_relu2_threshold
         phi_k, _ = features.kernel_features(k, W1, None, tau, self._spec, False)
         phi_q, resid = features.kernel_features(q, W1, W2, tau, self._spec, True)
-        views, etas = self._temporal_views(x, backend)
+        views, coef = self._temporal_views(x, backend)
         s = 1.0 / math.sqrt(cfg.depth)
         if cfg.read_norm:
             pairs = interface.scan_views_mass(tuple(views), phi_q, phi_k, v_w, "m")
         else:
             pairs = [(num, None) for num in interface.scan_views(tuple(views), phi_q, phi_k, v_w, "m")]
         nums, masses = [p[0] for p in pairs], [p[1] for p in pairs]
-        request = self._read_gate(x, views, etas)
+        request = self._read_gate(x, views, coef)
         if request is not None and request.fits(nums, masses, [resid]):
             return self._project_out(request.read(nums, masses, [resid], s, cfg.eps))
         reads = [gn.normalized_read(num, mass, resid, s=s, eps=cfg.eps) for num, mass in pairs]
-        return self._blend_and_project(x, reads, etas)
+        return self._blend_and_project(x, reads, coef)

@@ -151,3 +151,80 @@ def bank_read(nums, masses, resids, coef: torch.Tensor, *, s: float = 1.0, eps: 
     ``nums``) the output gate is applied too."""
     mass = [] if masses[0] is None else list(masses)
     return _bank_read_op(list(nums), mass, list(resids), coef, gate, gate_bias, float(s), float(eps))
+
+
+# ------------------------------------------------------------------ parameters
+
+def params_eligible(alpha: torch.Tensor, eta: torch.Tensor, x_dtype: torch.dtype) -> bool:
+    """Whether ts_bank_params forms this bank's retentions and blend."""
+    return (alpha.is_cuda and alpha.shape == eta.shape and alpha.ndim == 2 and alpha.dtype == eta.dtype
+            and alpha.dtype in (torch.bfloat16, torch.float32) and x_dtype in (torch.bfloat16, torch.float32)
+            and 1 <= alpha.shape[0] < _lib.BANK_MAX)
+
+
+def _params_desc(alpha, tanh_eta, stream_code):
+    return _lib.BankParamsDesc(alpha.shape[0], alpha.shape[1], int(tanh_eta), _lib.dtype_code(alpha.dtype), stream_code)
+
+
+def _ptrs(ts):
+    return (ctypes.c_void_p * len(ts))(*[_lib.ptr(t) for t in ts])
+
+
+def _params_forward(alpha: torch.Tensor, eta: torch.Tensor, tanh_eta: bool, stream_code: int) -> list[torch.Tensor]:
+    lib = _lib.load()
+    n, H = alpha.shape
+    a, e = alpha.detach().contiguous(), eta.detach().contiguous()
+    las = [torch.empty(H, dtype=torch.float32, device=a.device) for _ in range(n)]
+    coef = torch.empty(n + 1, H, dtype=torch.float32, device=a.device)
+    status = lib.ts_bank_params_fwd(ctypes.byref(_params_desc(a, tanh_eta, stream_code)), a.data_ptr(), e.data_ptr(),
+                                    _ptrs(las), coef.data_ptr(), _lib.stream_handle(a.device))
+    _lib.check(status, "ts_bank_params_fwd")
+    return las + [coef]
+
+
+def _params_fake(alpha, eta, tanh_eta, stream_code):
+    n, H = alpha.shape
+    return [alpha.new_empty(H, dtype=torch.float32) for _ in range(n)] + [
+        alpha.new_empty(n + 1, H, dtype=torch.float32)]
+
+
+def _params_backward_impl(grads: list[torch.Tensor], alpha: torch.Tensor, eta: torch.Tensor, tanh_eta: bool,
+                          stream_code: int) -> list[torch.Tensor]:
+    lib = _lib.load()
+    a, e = alpha.detach().contiguous(), eta.detach().contiguous()
+    # absent gradients travel as empty placeholders
+    gs = [None if g.numel() == 0 else g.to(torch.float32).contiguous() for g in grads]
+    da, de = torch.empty_like(a), torch.empty_like(e)
+    status = lib.ts_bank_params_bwd(ctypes.byref(_params_desc(a, tanh_eta, stream_code)), a.data_ptr(), e.data_ptr(),
+                                    _ptrs(gs[:-1]), _lib.ptr(gs[-1]), da.data_ptr(), de.data_ptr(),
+                                    _lib.stream_handle(a.device))
+    _lib.check(status, "ts_bank_params_bwd")
+    return [da, de]
+
+
+def _params_backward_fake(grads, alpha, eta, tanh_eta, stream_code):
+    return [torch.empty_like(alpha), torch.empty_like(eta)]
+
+
+def _params_setup(ctx, inputs, output):
+    alpha, eta, *ctx.args = inputs
+    ctx.save_for_backward(alpha, eta)
+
+
+def _params_backward(ctx, grads, bwd):
+    alpha, eta = ctx.saved_tensors
+    da, de = bwd([alpha.new_empty(0) if g is None else g for g in grads], alpha, eta, *ctx.args)
+    return da, de, None, None
+
+
+_bank_params_op = HipOp("bank_params", forward=_params_forward, forward_fake=_params_fake,
+                        backward_impl=_params_backward_impl, backward_fake=_params_backward_fake,
+                        setup=_params_setup, backward=_params_backward)
+
+
+def bank_params(alpha: torch.Tensor, eta: torch.Tensor, tanh_eta: bool, x_dtype: torch.dtype):
+    """(log retentions [H] fp32 per branch, blend coefficients [n+1, H]) of a
+    fast bank with parameters alpha, eta [n, H] (block.py:647-695) for streams
+    of ``x_dtype``: one launch each way."""
+    *las, coef = _bank_params_op(alpha, eta, bool(tanh_eta), _lib.dtype_code(x_dtype))
+    return las, coef

@@ -422,6 +422,10 @@ class ViewsBwdIO(ctypes.Structure):
 BANK_MAX = 8  # views of one ts_bank_read call
 
 
+class BankParamsDesc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("n", "H", "tanh_eta", "param_dtype", "stream_dtype")]
+
+
 class BankReadDesc(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int32) for n in ("B", "H", "T", "d", "n_views", "n_resid", "dtype", "normalize", "gate")] + [
         ("scale", ctypes.c_float), ("eps", ctypes.c_float)]
@@ -601,6 +605,11 @@ def load() -> ctypes.CDLL:
                                      ctypes.c_void_p, ctypes.c_void_p]
         lib.ts_views_bwd_workspace_bytes.argtypes = [P(ViewsBwdDesc), P(ctypes.c_size_t)]
         lib.ts_views_bwd.argtypes = [P(ViewsBwdDesc), P(ViewsBwdIO), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        PP = P(ctypes.c_void_p)
+        lib.ts_bank_params_fwd.argtypes = [P(BankParamsDesc), ctypes.c_void_p, ctypes.c_void_p, PP, ctypes.c_void_p,
+                                           ctypes.c_void_p]
+        lib.ts_bank_params_bwd.argtypes = [P(BankParamsDesc), ctypes.c_void_p, ctypes.c_void_p, PP, ctypes.c_void_p,
+                                           ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
         lib.ts_bank_read_fwd.argtypes = [P(BankReadDesc), P(BankReadIO), Strided, ctypes.c_void_p]
         lib.ts_bank_read_parts.argtypes = [P(BankReadDesc), P(ctypes.c_int32)]
         lib.ts_bank_read_bwd.argtypes = [P(BankReadDesc), P(BankReadIO), P(BankReadGrads), ctypes.c_void_p]

@@ -274,11 +274,92 @@ __global__ __launch_bounds__(256) void bank_read_bwd_kernel(BankReadP p) {
   }
 }
 
+// A fast bank's parameters in one launch each way (block.py:647-695): thread h
+// forms every branch's log retention -softplus(-alpha_raw), rounded through
+// the parameter's and the streams' dtypes as the tensor expression is, and the
+// blend coefficients (1 - sum eta, eta_1 ..), eta through tanh when asked.
+// Latency only: a few dozen numbers, which as tensor expressions took about
+// twenty launches forward and as many backward.
+struct BankParamsP {
+  int n, H, tanh_eta, pbf, xbf;    // pbf / xbf: the parameters / the streams are bf16
+  const void* alpha;               // [n][H]
+  const void* eta;                 // [n][H]
+  float* la[TS_BANK_MAX];          // [H] each
+  float* coef;                     // [n + 1][H]
+  const float* dla[TS_BANK_MAX];   // [H] each or null
+  const float* dcoef;              // [n + 1][H] or null
+  void* dalpha;                    // parameters' dtype
+  void* deta;
+};
+
+__device__ __forceinline__ float bank_param(const void* p, int bf, int i) {
+  return bf ? tof(((const bf16*)p)[i]) : ((const float*)p)[i];
+}
+__device__ __forceinline__ float bank_round(float x, int bf) { return bf ? tof((bf16)x) : x; }
+__device__ __forceinline__ float bank_eta(const BankParamsP& p, int i) {
+  const float e = bank_param(p.eta, p.pbf, i);
+  return p.tanh_eta ? bank_round(tanhf(e), p.pbf) : e;
+}
+
+__global__ void bank_params_fwd_kernel(BankParamsP p) {
+  for (int h = threadIdx.x; h < p.H; h += blockDim.x) {
+    float sum = 0.0f;
+    for (int j = 0; j < p.n; ++j) {
+      const float x = -bank_param(p.alpha, p.pbf, j * p.H + h);
+      const float sp = x > 20.0f ? x : log1pf(expf(x));
+      p.la[j][h] = bank_round(-bank_round(sp, p.pbf), p.xbf);
+      const float e = bank_eta(p, j * p.H + h);
+      p.coef[(j + 1) * p.H + h] = e;
+      sum += e;
+    }
+    p.coef[h] = 1.0f - sum;
+  }
+}
+
+__global__ void bank_params_bwd_kernel(BankParamsP p) {
+  for (int h = threadIdx.x; h < p.H; h += blockDim.x)
+    for (int j = 0; j < p.n; ++j) {
+      const int i = j * p.H + h;
+      const float x = -bank_param(p.alpha, p.pbf, i);
+      // d(-softplus(-a)) / da = sigmoid(-a)
+      const float da = p.dla[j] ? p.dla[j][h] * (x > 20.0f ? 1.0f : 1.0f / (1.0f + expf(-x))) : 0.0f;
+      float de = p.dcoef ? p.dcoef[(j + 1) * p.H + h] - p.dcoef[h] : 0.0f;
+      if (p.tanh_eta) {
+        const float e = bank_eta(p, i);
+        de *= 1.0f - e * e;
+      }
+      if (p.pbf) {
+        ((bf16*)p.dalpha)[i] = (bf16)da;
+        ((bf16*)p.deta)[i] = (bf16)de;
+      } else {
+        ((float*)p.dalpha)[i] = da;
+        ((float*)p.deta)[i] = de;
+      }
+    }
+}
+
 }  // namespace ts
 
 namespace {
 
 using ts::fail;
+
+int fill_params(const ts_bank_params_desc* d, const void* alpha, const void* eta, ts::BankParamsP* p) {
+  if (!d || !alpha || !eta) return fail(TS_ERR_VALUE, "bank params: missing descriptor or parameters");
+  if (d->n < 1 || d->n >= TS_BANK_MAX || d->H < 1) return fail(TS_ERR_VALUE, "bank params: %d branches of %d heads", d->n, d->H);
+  for (int t : {d->param_dtype, d->stream_dtype})
+    if (t != TS_BF16 && t != TS_F32) return fail(TS_ERR_VALUE, "bank params: unknown dtype");
+  memset(p, 0, sizeof(*p));
+  p->n = d->n; p->H = d->H; p->tanh_eta = d->tanh_eta;
+  p->pbf = d->param_dtype == TS_BF16; p->xbf = d->stream_dtype == TS_BF16;
+  p->alpha = alpha; p->eta = eta;
+  return TS_OK;
+}
+
+int params_done() {
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? TS_OK : fail(TS_ERR_RUNTIME, "bank params: launch failed: %s", hipGetErrorString(e));
+}
 
 int chunks_p2(const ts_bank_read_desc* d) {
   const int chunks = d->d / (d->dtype == TS_BF16 ? 8 : 4);
@@ -423,6 +504,31 @@ int ts_bank_read_bwd(const ts_bank_read_desc* d, const ts_bank_read_io* io, cons
   }
   p.dcoef_part = g->dcoef_part;
   return run(d, true, stream, p);
+}
+
+int ts_bank_params_fwd(const ts_bank_params_desc* d, const void* alpha, const void* eta, float* const* log_alpha,
+                       float* coef, hipStream_t stream) {
+  ts::BankParamsP p;
+  int rc = fill_params(d, alpha, eta, &p);
+  if (rc) return rc;
+  if (!log_alpha || !coef) return fail(TS_ERR_VALUE, "bank params: missing outputs");
+  for (int j = 0; j < d->n; ++j)
+    if (!(p.la[j] = log_alpha[j])) return fail(TS_ERR_VALUE, "bank params: missing log retention %d", j);
+  p.coef = coef;
+  hipLaunchKernelGGL(ts::bank_params_fwd_kernel, dim3(1), dim3(64), 0, stream, p);
+  return params_done();
+}
+
+int ts_bank_params_bwd(const ts_bank_params_desc* d, const void* alpha, const void* eta, const float* const* dlog_alpha,
+                       const float* dcoef, void* dalpha, void* deta, hipStream_t stream) {
+  ts::BankParamsP p;
+  int rc = fill_params(d, alpha, eta, &p);
+  if (rc) return rc;
+  if (!dlog_alpha || !dalpha || !deta) return fail(TS_ERR_VALUE, "bank params: missing gradients");
+  for (int j = 0; j < d->n; ++j) p.dla[j] = dlog_alpha[j];
+  p.dcoef = dcoef; p.dalpha = dalpha; p.deta = deta;
+  hipLaunchKernelGGL(ts::bank_params_bwd_kernel, dim3(1), dim3(64), 0, stream, p);
+  return params_done();
 }
 
 }  // extern "C"
