@@ -834,6 +834,45 @@ int ts_views_bwd_workspace_bytes(const ts_views_bwd_desc* desc, size_t* bytes);
 int ts_views_bwd(const ts_views_bwd_desc* desc, const ts_views_bwd_io* io, void* workspace, size_t workspace_bytes,
                  hipStream_t stream);
 
+/* ------------------------------------------------------------- decode step */
+
+/* At most eight tokens per sequence of a depth-1 kernel memory with the plain
+ * sum, continuing a carried state: features, recurrence, read and output gate
+ * in one launch (block.py:595-618, engine.py:117-158, 426-544,
+ * kernel_features.py:73-135, block.py:721-722).  RoPE phases are those of
+ * positions position .. position + T - 1, the position from io->position (an
+ * int64 on the device) where set, else desc->position. */
+typedef struct ts_memory_step_desc {
+  int32_t B, H, T, d, m;          /* d, m: 16, 32, 64 or 128; T <= 8           */
+  int32_t dtype;                  /* of q, k, v, g, y, w1, w2                  */
+  int32_t param_dtype;            /* of tau, gbias                             */
+  int32_t kind;                   /* ts_feature_kind                           */
+  int32_t in_rot, feat_rot;       /* rotated widths                            */
+  int32_t normalize, gate;
+  float gain, resid_scale, eps;
+  int64_t position;
+} ts_memory_step_desc;
+
+typedef struct ts_memory_step_io {
+  ts_strided q, k, v, g, y;       /* [B,H,T,d]; g: gate pre-activation (gate)  */
+  const void* w1;                 /* [H][m][d]                                 */
+  const void* w2;                 /* [H][d][m]                                 */
+  const void* tau;                /* [H] or NULL                               */
+  const void* gbias;              /* [H*d] or NULL                             */
+  const float* inv_in;            /* [in_rot / 2] inverse frequencies          */
+  const float* inv_feat;          /* [feat_rot / 2]                            */
+  const int64_t* position;        /* device counter or NULL                    */
+  const float* init_state;        /* fp32 [B*H][m][d + normalize] or NULL      */
+  float* final_state;             /* same layout (may be init_state) or NULL   */
+} ts_memory_step_io;
+
+int ts_memory_step(const ts_memory_step_desc* desc, const ts_memory_step_io* io, hipStream_t stream);
+
+/* y [n][na + nb] = x [n][k] [wa; wb]^T in bf16 (fp32 accumulation), n <= 64, k
+ * a multiple of 32, na and nb of 16 (nb may be 0); row strides in elements. */
+int ts_skinny_linear(const void* x, int32_t n, int32_t k, int64_t x_stride, const void* wa, int32_t na,
+                     const void* wb, int32_t nb, void* y, int64_t y_stride, hipStream_t stream);
+
 /* ------------------------------------------------------------- bank read */
 
 #define TS_BANK_MAX 8

@@ -1,0 +1,107 @@
+"""ts_memory_step and ts_skinny_linear: a decode step of the one-call kernel
+memory (GPU tests).
+
+A mixer fed a prompt and then pieces of at most eight tokens (the step kernel)
+must continue the sequence that one whole call computes in float64: every
+padded head width and feature count, both maps, both reads, with and without
+the output gate and the learned threshold, RoPE at either placement.  Bars:
+fp32 2e-5 (fp32 sums in another order), bf16 2e-2 (the activations' rounding).
+The skinny product: fp32 accumulation of bf16 products, one rounding (8e-3 of
+the largest value).
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import mixer as oracle_mixer
+from tests.conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(head_dim, mult, feature_map, norm, rope, gate, threshold=False):
+    import thetascan_amd as ts
+
+    return ts.ThetaScanConfig(
+        d_model=2 * head_dim, n_heads=2, memory_multiplier=mult, family="kernel", output_gate=gate,
+        kernel=ts.KernelConfig(feature_map=feature_map, read_normalization=norm,
+                               relu2_threshold_mode="learned_per_head" if threshold else "none"),
+        rope=ts.RoPEConfig() if rope is None else ts.RoPEConfig(mode="partial", fraction=0.5, placement=rope))
+
+
+CASES = [
+    (64, 1, "relu2_ridge", "none", "feature", True, False),
+    (64, 2, "relu2_ridge", "key_mass", "input", True, True),
+    (16, 1, "softmax_partition", "key_mass", None, False, False),
+    (32, 2, "softmax_partition", "none", "feature", True, False),
+    (128, 1, "relu2_ridge", "key_mass", "input", False, True),
+]
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("case", CASES)
+def test_step_continues_the_sequence(cuda, case, dtype, tol):
+    import thetascan_amd as ts
+    from thetascan_amd import _lib
+
+    cfg = _config(*case)
+    torch.manual_seed(1)
+    module = ts.ThetaScan(cfg)
+    g = torch.Generator().manual_seed(2)
+    with torch.no_grad():
+        for _, p in sorted(module.named_parameters()):
+            p.add_(torch.randn(p.shape, generator=g) * 0.05)
+    module = module.to(dtype)
+    B, T = 3, 90
+    x = torch.randn(B, T, cfg.d_model, generator=g).to(dtype)
+    params = {k: v.detach().double() for k, v in module._core.named_parameters()}
+    want = oracle_mixer.forward(oracle_mixer.core_config(cfg.to_dict()), params, x.double(), backend="chunk")
+    module = module.to(cuda)
+    xd, got = x.to(cuda), []
+    with torch.no_grad(), _lib.record_launches() as recs:
+        y, state = module(xd[:, :67], state=module.initial_state())
+        got.append(y)
+        t = 67
+        for n in (1, 8, 3, 1, 8, 2):
+            before = [c.clone() for c in state._tensors()]
+            y, new = module(xd[:, t:t + n], state=state)
+            assert all(torch.equal(a, b) for a, b in zip(state._tensors(), before))  # the given state is unchanged
+            state, t = new, t + n
+            got.append(y)
+        # a first call of few tokens starts from a zero state
+        first, _ = module(xd[:, :5], state=module.initial_state())
+    assert t == T and state.position == T
+    assert sum(r[0] == "ts_memory_step" for r in recs) == 7
+    assert rel_err(torch.cat(got, 1), want) < tol
+    assert rel_err(first, want[:, :5]) < tol
+
+
+@pytest.mark.parametrize("n,k,na,nb", [(1, 512, 1536, 512), (8, 512, 512, 0), (17, 32, 16, 16), (64, 160, 48, 0),
+                                       (5, 1024, 64, 32)])
+def test_skinny_linear(cuda, n, k, na, nb):
+    from thetascan_amd._core.ops import step
+
+    g = torch.Generator().manual_seed(n + k)
+    x, wa, wb = (torch.randn(r, k, generator=g).to(torch.bfloat16) for r in (n, na, max(nb, 1)))
+    want = x.double() @ torch.cat([wa, wb[:nb]]).double().t()
+    got = step._linear(x.to(cuda), wa.to(cuda), wb.to(cuda) if nb else None)
+    assert got.shape == (n, na + nb)
+    assert rel_err(got, want) < 8e-3
+    # rows beyond the kernel's limit take the library product
+    many = step._linear(x.to(cuda).repeat(66, 1), wa.to(cuda), None)
+    assert rel_err(many[:n], want[:, :na]) < 8e-3
+
+
+def test_other_continuations_keep_their_path(cuda):
+    """Nine tokens, and parameters of another dtype than the input's, take the
+    multi-view path."""
+    import thetascan_amd as ts
+    from thetascan_amd import _lib
+
+    cfg = _config(*CASES[0])
+    module = ts.ThetaScan(cfg).to(cuda)
+    x = torch.randn(2, 9, cfg.d_model, device=cuda)
+    with torch.no_grad(), _lib.record_launches() as recs:
+        module(x, state=module.initial_state())
+    assert "ts_memory_step" not in {r[0] for r in recs}

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from ..config import ThetaScanConfig
 from ...state import ThetaScanState, config_fingerprint
-from ..ops import bankread, composed, features, fused, gn, interface, maps, prologue, stream
+from ..ops import bankread, composed, features, fused, gn, interface, maps, prologue, step, stream
 from ..ops.linear import linear, stack_heads
 from ..ops.interface import Accumulator, FadeFast, FadeStale, NullAccumulator, resolve_backend
 from .gates import DecayGate, OutGate
@@ -440,6 +440,19 @@ class ThetaScan(nn.Module):
                                   self.ogate.g.lin.bias if gate else None, W1, W2, self.kernel_relu2_threshold,
                                   self.proj_out.weight, spec, cfg.read_norm, H)
 
+    def _forward_step(self, x: torch.Tensor) -> torch.Tensor | None:
+        """A continuation of at most eight tokens (a decode step) of the
+        one-call memory: three launches, or None where ts_memory_step does not
+        take it."""
+        cfg = self.cfg
+        lin = None if self.ogate is None else self.ogate.g.lin
+        (W1, W2, _), = self._weights()
+        args = (self.proj_qkv.weight, None if lin is None else lin.weight, None if lin is None else lin.bias, W1, W2,
+                self.kernel_relu2_threshold, self.proj_out.weight)
+        if not step.eligible(x, self._spec, cfg.head_dim, args):
+            return None
+        return step.kernel_step(x, *args, self._spec, cfg.read_norm, cfg.n_heads)
+
     def _fingerprint(self) -> str:
         """config_fingerprint(self.cfg), recomputed only when a field changes
         (the configuration's fields are flat values: a shallow snapshot sees
@@ -493,7 +506,9 @@ class ThetaScan(nn.Module):
         with stream.carrying(carry):
             if self.fused_eligible(x):
                 self.last_path = "fused"
-                y = self._forward_views(x, backend)
+                y = self._forward_step(x) if self._fused_cfg else None
+                if y is None:
+                    y = self._forward_views(x, backend)
             else:
                 self.last_path = "composed"
                 y = self._forward_composed(x, backend)

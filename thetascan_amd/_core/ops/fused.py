@@ -32,16 +32,22 @@ from .linear import slot_sum, split_k_outer, weight_grad
 _INV: dict = {}
 
 
+def inverse_frequencies(rot: int, base: float, device) -> torch.Tensor:
+    """fp32 inverse frequencies [rot / 2] (rope.py:7-38), kept for the life of
+    the process: a captured step reads them in place."""
+    key = (rot, float(base), str(device))
+    inv = _INV.get(key)
+    if inv is None:
+        inv = _INV[key] = 1.0 / (base ** (torch.arange(0, rot, 2, device=device, dtype=torch.float32) / rot))
+    return inv
+
+
 def _rope_tables(T: int, rot: int, base: float, device, start=0) -> tuple[torch.Tensor, torch.Tensor]:
     """fp32 cos/sin [T, rot/2] of positions start .. start+T-1 (rope.py:7-38
     phases, kept in fp32).  ``start`` may be an int64 device tensor (a
     captured decode step): the positions are the same exact fp32 integers."""
     if isinstance(start, torch.Tensor):
-        # kept for the life of the process: a captured step reads them in place
-        key = (rot, float(base), str(device))
-        inv = _INV.get(key)
-        if inv is None:
-            inv = _INV[key] = 1.0 / (base ** (torch.arange(0, rot, 2, device=device, dtype=torch.float32) / rot))
+        inv = inverse_frequencies(rot, base, device)
         akey = ("offsets", T, str(device))
         offsets = _INV.get(akey)
         if offsets is None:

@@ -419,6 +419,19 @@ class ViewsBwdIO(ctypes.Structure):
     ]
 
 
+class MemoryStepDesc(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("B", "H", "T", "d", "m", "dtype", "param_dtype", "kind", "in_rot",
+                                              "feat_rot", "normalize", "gate")] + [
+        ("gain", ctypes.c_float), ("resid_scale", ctypes.c_float), ("eps", ctypes.c_float),
+        ("position", ctypes.c_int64)]
+
+
+class MemoryStepIO(ctypes.Structure):
+    _fields_ = [(n, Strided) for n in ("q", "k", "v", "g", "y")] + [
+        (n, ctypes.c_void_p) for n in ("w1", "w2", "tau", "gbias", "inv_in", "inv_feat", "position", "init_state",
+                                       "final_state")]
+
+
 BANK_MAX = 8  # views of one ts_bank_read call
 
 
@@ -605,6 +618,10 @@ def load() -> ctypes.CDLL:
                                      ctypes.c_void_p, ctypes.c_void_p]
         lib.ts_views_bwd_workspace_bytes.argtypes = [P(ViewsBwdDesc), P(ctypes.c_size_t)]
         lib.ts_views_bwd.argtypes = [P(ViewsBwdDesc), P(ViewsBwdIO), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.ts_memory_step.argtypes = [P(MemoryStepDesc), P(MemoryStepIO), ctypes.c_void_p]
+        lib.ts_skinny_linear.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int64,
+                                         ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32,
+                                         ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
         PP = P(ctypes.c_void_p)
         lib.ts_bank_params_fwd.argtypes = [P(BankParamsDesc), ctypes.c_void_p, ctypes.c_void_p, PP, ctypes.c_void_p,
                                            ctypes.c_void_p]
