@@ -1,0 +1,49 @@
+"""GN stages on streams whose token rows are strided, shared or few: the
+kernels address a group's rows through offsets that end after the last token,
+so rows of any stride and one row broadcast over the tokens have to give the
+same bits as contiguous copies of them (the arithmetic is the same)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(B, H, T, w, layout, dtype, dev, g):
+    if layout == "broadcast":
+        return torch.randn(B, H, 1, w, generator=g).to(dev, dtype).expand(B, H, T, w)
+    if layout == "token_major":
+        return torch.randn(B, T, H, w, generator=g).to(dev, dtype).transpose(1, 2)
+    # rows of a wider matrix whose tail would change a sum if it were read
+    return torch.randn(B, H, T, w + 64, generator=g).to(dev, dtype)[..., :w]
+
+
+@pytest.mark.parametrize("nonlin", ["relu2", "tanh", "silu"])
+@pytest.mark.parametrize("dtype,d,m", [(torch.bfloat16, 64, 128), (torch.float32, 32, 48), (torch.bfloat16, 32, 192)])
+@pytest.mark.parametrize("layout", ["broadcast", "token_major", "padded"])
+@pytest.mark.parametrize("T", [1, 65, 130])
+def test_gn_rows_of_any_stride(cuda, dtype, d, m, layout, T, nonlin):
+    from thetascan_amd._core.ops import gn
+
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(7 * d + m + T)
+    w1 = (torch.randn(H, m, d, generator=g) / d ** 0.5).to(cuda, dtype)
+    w2 = (torch.randn(H, d, m, generator=g) * 0.3).to(cuda, dtype)
+    x, v, num = (_rows(B, H, T, w, layout, dtype, cuda, g) for w in (d, d, m))
+    mass = torch.rand(B, H, T, generator=g).to(cuda) + 0.5
+    dys = [_rows(B, H, T, w, layout, dtype, cuda, g) for w in (m, d, m, m, d)]
+
+    def run(x, v, num, dys):
+        x, v, num = (t.detach().requires_grad_(True) for t in (x, v, num))
+        ws = [t.clone().requires_grad_(True) for t in (w1, w2)]
+        out = list(gn.write(x, v, *ws, nonlin=nonlin))
+        out += list(gn.read_stage(x, *ws, None, num, mass, corr=gn.READ_NORMALIZED, want_resid=True, nonlin=nonlin))
+        grads = torch.autograd.grad(out, [x, v, num, *ws], dys)
+        return [*out, *grads]
+
+    got = run(x, v, num, dys)
+    want = run(x.contiguous(), v.contiguous(), num.contiguous(), [t.contiguous() for t in dys])
+    for a, b in zip(got, want):
+        assert torch.isfinite(a).all()
+        assert torch.equal(a, b)

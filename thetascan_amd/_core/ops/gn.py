@@ -44,9 +44,11 @@ def eligible(cfg, weights, k: torch.Tensor, v: torch.Tensor) -> bool:
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
     """A [B,H,T,w] view whose rows the kernel can read: contiguous last axis,
-    16-byte aligned rows (else a contiguous copy)."""
+    16-byte aligned rows, 64 of them within 32-bit offsets (else a contiguous
+    copy)."""
     vec = 16 // t.element_size()
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:3])
+    ok = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:3])
+          and 64 * t.stride(2) * t.element_size() < 1 << 31)
     return t if ok else t.contiguous()
 
 

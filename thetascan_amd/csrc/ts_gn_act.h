@@ -11,8 +11,7 @@
 
 namespace ts {
 
-// sigma(pre); the slope sp = sigma'(pre) is written as a function of h =
-// sigma(pre) for relu2 (2 sqrt(h) = 2 relu(pre)) and tanh (1 - h^2).
+// sigma(pre) and its slope sp = sigma'(pre) (tanh: from h = sigma(pre)).
 __device__ __forceinline__ float gn_sigmoid(float pre) { return 1.f / (1.f + __expf(-pre)); }
 __device__ __forceinline__ float gn_act(int act, float pre) {
   if (act == TS_GN_TANH) return tanhf(pre);
@@ -20,14 +19,14 @@ __device__ __forceinline__ float gn_act(int act, float pre) {
   const float rp = fmaxf(pre, 0.f);
   return rp * rp;
 }
-// sigma'(pre): from h for relu2 and tanh, from pre for SiLU
+// sigma'(pre): 2 relu(pre), from h for tanh (1 - h^2), from pre for SiLU
 // (silu' = sg (1 + pre (1 - sg)), sg = sigmoid(pre)).
 __device__ __forceinline__ float gn_slope(int act, float pre, float hval) {
   if (act == TS_GN_SILU) {
     const float sg = gn_sigmoid(pre);
     return sg * (1.f + pre * (1.f - sg));
   }
-  return act == TS_GN_TANH ? 1.f - hval * hval : 2.f * sqrtf(hval);
+  return act == TS_GN_TANH ? 1.f - hval * hval : 2.f * fmaxf(pre, 0.f);
 }
 // d pre of a term dh * h + dsp * sp: sigma'(pre) dh + sigma''(pre) dsp
 // (relu2: 2 relu(pre) dh + 2 dsp for pre > 0, else 0;

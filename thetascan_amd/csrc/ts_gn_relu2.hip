@@ -1,0 +1,10 @@
+// The GN write and read kernels with a relu2 hidden layer (see ts_gn_kernels.h).
+
+#include "ts_gn_pick.h"
+
+ts::GnKernel ts::gn_relu2_kernel(bool bf16, bool wide, bool fwd, int d, int m) {
+  return gn_kernel<TS_GN_RELU2>(bf16, wide, fwd, d, m);
+}
+ts::GnReadKernel ts::gn_read_relu2_kernel(bool bf16, bool wide, bool fwd, int d, int m) {
+  return gn_read_kernel<TS_GN_RELU2>(bf16, wide, fwd, d, m);
+}
