@@ -13,26 +13,34 @@
 // of terms about T / (1 - alpha) times larger, which bf16 scans cannot
 // resolve; this kernel sums the pair terms themselves instead.
 //
-// A workgroup walks one segment of seg_tiles 64-token tiles of one (b, h);
-// wave w owns value block w (16 columns; the last block of a call with a mass
-// column holds that column).  Per tile:
+// A workgroup walks one segment of seg_tiles 64-token tiles of one (b, h).
+// The [dk][values] states split into 16x16 blocks: wave w owns key block
+// w % NKB for every S-th value block (S waves a key block, so that narrow keys
+// too run eight waves; the last value block of a call with a mass column holds
+// that column).  Per tile:
 //   * pairs inside the tile: the ten causal 16x16 blocks of S = Q K^T, each
-//     formed once by one wave on MFMA, against G = D V^T of every value
-//     block, summed with the weights d alpha^d, d = t - i >= 0;
-//   * pairs with i in earlier tiles of the segment, through the states
-//     M = sum_{i<t0} alpha^(t0-1-i) k_i v_i^T and M' = sum (t0-1-i) alpha^(..) k_i v_i^T:
-//     sum_t alpha^(tau+1) [(tau+1) q_t^T M dO_t + q_t^T M' dO_t], tau = t - t0.
-//     Each wave holds its value block of M and M' in MFMA accumulators, and
-//     they enter the next MFMAs from registers (the accumulator rows are the
-//     contraction order of the query fragments), with no LDS copy.
-// Operands formed inside the kernel (the states and the weighted value and
-// gradient rows) enter the MFMAs as bf16 pairs hi + lo, hi = bf16(x),
-// lo = bf16(x - hi): with the bf16 inputs exact, every product then carries
-// about 16 bits, as the fp32 sums need.
+//     formed once by one wave on MFMA, times G = D V^T (summed over the values
+//     by its MFMAs), with the weights d alpha^d, d = t - i >= 0;
+//   * pairs with i in earlier tiles of the segment: with the states
+//     M = sum_{i<t0} alpha^(t0-1-i) k_i v_i^T and M' = sum (t0-1-i) alpha^(..) k_i v_i^T
+//     and the tile's query sums A = sum_t (tau+1) alpha^(tau+1) q_t dO_t^T,
+//     B = sum_t alpha^(tau+1) q_t dO_t^T (tau = t - t0), they are
+//     <M, A> + <M', B>: all four are fp32 MFMA accumulators of one layout, so
+//     the products are element by element in registers.
+// The weighted keys and queries enter the MFMAs as bf16 pairs hi + lo,
+// hi = bf16(x), lo = bf16(x - hi), against the exact bf16 values and
+// gradients: every product then carries about 16 bits, as the fp32 sums need.
+// The kernel is bound by vector and matrix issue (per key and value block and
+// tile 16 MFMAs and 40 vector instructions, and 290 a key block for the
+// weighted pairs: vector units 52 %, MFMA 26 % busy), so every wave has a block
+// and no work is repeated.  An
+// earlier split by value blocks (five of eight waves busy at 64 values with a
+// mass column, the query products formed against split copies of the states)
+// took 163 us where this takes 97 us: B8 H8 T4096, dk 128, dv 64 + mass.
 // Pairs across segments need the state entering the segment, which is not
 // known here; each segment therefore also leaves its own forward summaries
-// M_s, M'_s and the query-side sums A_s = sum_t (n+1) alpha^(n+1) q_t dO_t^T,
-// B_s = sum_t alpha^(n+1) q_t dO_t^T (n = t - segment start), and a combine
+// M_s, M'_s and the query-side sums A_s, B_s with n = t - segment start in the
+// place of tau (summed from the tiles' A and B), and a combine
 // kernel adds <M_in, A_s> + <M'_in, B_s> with M_in, M'_in the prefix of the
 // summaries (M'_in composes as alpha^L (M'_in + L M_in) + M'_s).
 
@@ -45,7 +53,7 @@
 namespace ts {
 
 struct RetP {
-  int B, H, T, dk, dv, nvr, has_mass, seg_tiles, nseg, vw, nw;  // nvr: real value blocks; vw: padded width
+  int B, H, T, dk, dv, nvr, has_mass, seg_tiles, nseg, vw;  // nvr: real value blocks; vw: padded width
   ts_strided q, k, v, dout, dm;
   uint32_t q_rec, k_rec, v_rec, o_rec, dm_rec;
   const float* log_alpha;
@@ -67,12 +75,10 @@ constexpr int kTabRB = 192;   // [64] alpha^(tau+1)
 constexpr int kTabPow = 256;  // [68] alpha^d, d = 0..64
 constexpr int kTabWM = 324;   // [64] this tile's alpha^(len-1-tok), 0 past len
 constexpr int kTabWMp = 388;  // [64] (len-1-tok) alpha^(len-1-tok)
-constexpr int kTabWA = 452;   // [64] (n+1) alpha^(n+1), n from the segment start
-constexpr int kTabWB = 516;   // [64] alpha^(n+1)
-constexpr int kTabRed = 580;  // [8]
-constexpr int kTabFloats = 588;
+constexpr int kTabRed = 452;  // [8]
+constexpr int kTabFloats = 460;
 
-__host__ __device__ inline RetLayout ret_layout(int DK, int vw) {
+__host__ __device__ constexpr RetLayout ret_layout(int DK, int vw) {
   RetLayout L{};
   L.qp = DK + 8;
   L.vp = vw + 8;
@@ -107,51 +113,47 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8& hi, bf16x8& 
   lo = __builtin_bit_cast(bf16x8, make_uint4(l[0], l[1], l[2], l[3]));
 }
 
-// Accumulator fragments a, b (the eight k-values of one lane) as hi + lo.
-__device__ __forceinline__ void split_acc(floatx4 a, floatx4 b, bf16x8& hi, bf16x8& lo) {
-  const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-  split8(x, hi, lo);
-}
-__device__ __forceinline__ void split_acc4(floatx4 a, bf16x4& hi, bf16x4& lo) {
-  const uint32_t h0 = pk2(a[0], a[1]), h1 = pk2(a[2], a[3]);
-  const uint32_t l0 = pk2(a[0] - __uint_as_float(h0 << 16), a[1] - __uint_as_float(h0 & 0xffff0000u));
-  const uint32_t l1 = pk2(a[2] - __uint_as_float(h1 << 16), a[3] - __uint_as_float(h1 & 0xffff0000u));
-  hi = __builtin_bit_cast(bf16x4, make_uint2(h0, h1));
-  lo = __builtin_bit_cast(bf16x4, make_uint2(l0, l1));
-}
-
 // bf16 element e of a fragment as float
 __device__ __forceinline__ float elt(bf16x8 v, int e) { return tof(v[e]); }
 
-// Eight table entries at the tokens of a col8 fragment (kp, lane group g).
-__device__ __forceinline__ void tab8(const float* t, int kp, int g, float (&w)[8]) {
+// The eight tokens of a col8 fragment x (kp, lane group g) times a table's
+// weights, as hi + lo.
+__device__ __forceinline__ void weigh8(bf16x8 x, const float* t, int kp, int g, bf16x8& hi, bf16x8& lo) {
   const floatx4 a = *(const floatx4*)(t + 32 * kp + 4 * g);
   const floatx4 b = *(const floatx4*)(t + 32 * kp + 16 + 4 * g);
+  float y[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    w[i] = a[i];
-    w[4 + i] = b[i];
+    y[i] = elt(x, i) * a[i];
+    y[4 + i] = elt(x, 4 + i) * b[i];
   }
+  split8(y, hi, lo);
 }
 
 // (query block, key block) pairs of the causal tile, key block <= query block
 __constant__ int kPairs[10][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}, {3, 0}, {3, 1}, {3, 2}, {3, 3}};
 
-template <int DK>
-__global__ __launch_bounds__(512) void retention_grad_kernel(RetP p) {
+// Waves that share a key block: as many as keep a workgroup at eight waves.
+constexpr int ret_share(int dk) { return 128 / dk; }
+
+template <int DK, int NVB>
+__global__ __launch_bounds__(64 * (DK / 16) * ret_share(DK)) void retention_grad_kernel(RetP p) {
   typedef bf16 E;
   typedef Tok<E> TK;
   constexpr int NK32 = DK / 32;
   constexpr bool KTAIL = (DK % 32) != 0;
   constexpr int NKB = DK / 16;
   constexpr int QC = DK / 8;  // 16-byte chunks per key row
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, l16 = lane & 15;
-  const int bd = blockDim.x, nwave = bd >> 6;
+  constexpr int S = ret_share(DK), nwave = NKB * S, bd = 64 * nwave;
+  constexpr int NQ = (C * QC + bd - 1) / bd;                // chunks of a query or key tile per thread
+  constexpr int NW = NVB * S, vw = NW * 16;                 // value blocks (the host rounds up; the rest are zeros)
+  constexpr int NV = (C * 2 * NW + bd - 1) / bd;            // chunks of a value or gradient tile per thread
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
+            l16 = lane & 15;
+  const int kb = w % NKB, vs = w / NKB;  // this wave's blocks: keys kb, values vs, vs + S, ..
   const int seg = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int bh = b * p.H + h;
-  const int vw = p.vw, nw = p.nw;
-  const bool owner = w < nw;  // owns value block w; later waves only load and form tile pairs
-  const RetLayout L = ret_layout(DK, vw);
+  constexpr RetLayout L = ret_layout(DK, vw);
   extern __shared__ __align__(16) unsigned char smem[];
   E* base = (E*)smem;
   E* Qs = base + L.qs;
@@ -183,47 +185,35 @@ __global__ __launch_bounds__(512) void retention_grad_kernel(RetP p) {
   const rsrc_t dm_rs = make_rsrc(bh_base(p.dm, b, h, 4), p.dm_rec);
   const int vr = p.nvr * 16;  // real (padded) value columns; the mass block follows
 
-  // tile loads: at most two 16-byte chunks of each tile per thread (the host
-  // launches max(value blocks, DK/16) waves); rows and columns fixed per tile
-  int v_row[2], v_col[2];
+  // the states and the segment's query sums, rows (keys) kb*16 + 4g + i,
+  // column (value) (vs + n S)*16 + l16
+  floatx4 M[NVB], Mp[NVB], A[NVB], Bq[NVB];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int idx = tid + r * bd;
-    v_row[r] = idx < C * (vw / 8) ? idx / (vw / 8) : -1;
-    v_col[r] = idx < C * (vw / 8) ? (idx % (vw / 8)) * 8 : 0;
-  }
-
-  // this wave's value block w: the states and query-side sums, rows (keys)
-  // kb*16 + 4g + i, column (value) w*16 + l16
-  floatx4 M[NKB], Mp[NKB], A[NKB], Bq[NKB];
-#pragma unroll
-  for (int kb = 0; kb < NKB; ++kb) M[kb] = Mp[kb] = A[kb] = Bq[kb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int n = 0; n < NVB; ++n) M[n] = Mp[n] = A[n] = Bq[n] = floatx4{0.f, 0.f, 0.f, 0.f};
   float acc = 0.f;
 
   // tile c's loads go to registers while tile c - 1 is computed
-  uint4 rq[2], rk[2], rv[2], rd[2];
-  float rdm[2];
+  uint4 rq[NQ], rk[NQ], rv[NV], rd[NV];
+  float rdm[NV];
   auto fetch = [&](int c) {
     const int t0 = c * C;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < NQ; ++r) {
       const int idx = tid + r * bd;
-      rq[r] = rk[r] = rv[r] = rd[r] = make_uint4(0u, 0u, 0u, 0u);
-      rdm[r] = 0.f;
-      if (idx < C * QC) {
-        const int row = idx / QC, col = (idx % QC) * 8;
-        rq[r] = bld16(q_rs, (uint32_t)((t0 + row) * q_st + col * 2));
-        rk[r] = bld16(k_rs, (uint32_t)((t0 + row) * k_st + col * 2));
-      }
-      const int row = v_row[r], col = v_col[r];
-      if (row >= 0 && col < vr) {
-        const uint32_t ov = col < p.dv ? (uint32_t)((t0 + row) * v_st + col * 2) : kOOB;
-        const uint32_t oo = col < p.dv ? (uint32_t)((t0 + row) * o_st + col * 2) : kOOB;
-        rv[r] = bld16(v_rs, ov);
-        rd[r] = bld16(o_rs, oo);
-      } else if (row >= 0 && col == vr && p.has_mass && t0 + row < p.T) {
-        rdm[r] = bldf(dm_rs, (uint32_t)((t0 + row) * (int)p.dm.st * 4));
-      }
+      const int row = idx / QC, col = (idx % QC) * 8;
+      const bool on = idx < C * QC;
+      rq[r] = bld16(q_rs, on ? (uint32_t)((t0 + row) * q_st + col * 2) : kOOB);
+      rk[r] = bld16(k_rs, on ? (uint32_t)((t0 + row) * k_st + col * 2) : kOOB);
+    }
+#pragma unroll
+    for (int r = 0; r < NV; ++r) {
+      const int idx = tid + r * bd;
+      const int row = idx / (2 * NW), col = (idx % (2 * NW)) * 8;
+      const bool in = idx < C * 2 * NW, on = in && col < p.dv;
+      rv[r] = bld16(v_rs, on ? (uint32_t)((t0 + row) * v_st + col * 2) : kOOB);
+      rd[r] = bld16(o_rs, on ? (uint32_t)((t0 + row) * o_st + col * 2) : kOOB);
+      const bool mass = in && col == vr && p.has_mass && t0 + row < p.T;
+      rdm[r] = bldf(dm_rs, mass ? (uint32_t)((t0 + row) * (int)p.dm.st * 4) : kOOB);
     }
   };
   if (c0 < c1) fetch(c0);
@@ -234,15 +224,19 @@ __global__ __launch_bounds__(512) void retention_grad_kernel(RetP p) {
     __syncthreads();  // the previous tile's operands and tables are consumed
     {
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
+      for (int r = 0; r < NQ; ++r) {
         const int idx = tid + r * bd;
         if (idx < C * QC) {
           const int row = idx / QC, col = (idx % QC) * 8;
           *(uint4*)(Qs + row * L.qp + col) = rq[r];
           *(uint4*)(Ks + row * L.qp + col) = rk[r];
         }
-        const int row = v_row[r], col = v_col[r];
-        if (row >= 0) {
+      }
+#pragma unroll
+      for (int r = 0; r < NV; ++r) {
+        const int idx = tid + r * bd;
+        const int row = idx / (2 * NW), col = (idx % (2 * NW)) * 8;
+        if (idx < C * 2 * NW) {
           uint4 vv = rv[r], dd = rd[r];
           if (col == vr && p.has_mass) {
             // two unit V columns against dm as bf16 hi + lo
@@ -263,188 +257,86 @@ __global__ __launch_bounds__(512) void retention_grad_kernel(RetP p) {
         const float pw = d >= 0 ? tab[kTabPow + max(d, 0)] : 0.f;
         tab[kTabWM + tok] = pw;
         tab[kTabWMp + tok] = (float)d * pw;
-        const float n1 = (float)((c - c0) * C + tok + 1);
-        const float a = expf(la * n1);
-        tab[kTabWA + tok] = n1 * a;
-        tab[kTabWB + tok] = a;
       }
     }
     __syncthreads();
     if (c + 1 < c1) fetch(c + 1);
 
-    // ---- pairs inside the tile: each score block once, against every value block
+    // ---- pairs inside the tile: each score block once, against D V^T
     for (int pi = w; pi < 10; pi += nwave) {
       const int tb = kPairs[pi][0], ib = kPairs[pi][1];
-      floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+      floatx4 sc = {0.f, 0.f, 0.f, 0.f}, gg = sc;
 #pragma unroll
       for (int j = 0; j < NK32; ++j)
         sc = mma32(frow8<E>(Qs, L.qp, tb * 16 + l16, j, g), frow8<E>(Ks, L.qp, ib * 16 + l16, j, g), sc);
       if (KTAIL) sc = mma16(frow4<E>(Qs, L.qp, tb * 16 + l16, NK32, g), frow4<E>(Ks, L.qp, ib * 16 + l16, NK32, g), sc);
+#pragma unroll
+      for (int j = 0; j < NW / 2; ++j)
+        gg = mma32(frow8<E>(Ds, L.vp, tb * 16 + l16, j, g), frow8<E>(Vs, L.vp, ib * 16 + l16, j, g), gg);
+      if (NW & 1)
+        gg = mma16(frow4<E>(Ds, L.vp, tb * 16 + l16, NW / 2, g), frow4<E>(Vs, L.vp, ib * 16 + l16, NW / 2, g), gg);
       // rows (queries) tb*16 + 4g + i, columns (keys) ib*16 + l16; d = t - i
       const float* dt = tab + kTabD + 64 + (tb - ib) * 16 + 4 * g - l16;
-      float wd[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wd[i] = dt[i] * sc[i];
-      // value blocks four at a time: their operand reads and products issue
-      // together before the sums consume them
-      for (int vb0 = 0; vb0 < nw; vb0 += 4) {
-        floatx4 gg[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          gg[u] = floatx4{0.f, 0.f, 0.f, 0.f};
-          const int vb = vb0 + u;
-          if (vb < nw)
-            gg[u] = mma16(frow4<E>(Ds + vb * 16, L.vp, tb * 16 + l16, 0, g),
-                          frow4<E>(Vs + vb * 16, L.vp, ib * 16 + l16, 0, g), gg[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc += wd[i] * gg[u][i];
-      }
+      for (int i = 0; i < 4; ++i) acc += dt[i] * sc[i] * gg[i];
     }
 
-    if (owner) {
-      const E* Dw = Ds + w * 16;
-      const E* Vw = Vs + w * 16;
-      bf16x8 d8[2];
-#pragma unroll
-      for (int kp = 0; kp < 2; ++kp) d8[kp] = TK::col8(Dw, L.vp, 0, kp, lane);
-      // ---- pairs with keys in earlier tiles of the segment, through the
-      // states (B operand from the accumulators: column = value, contraction
-      // over keys in the accumulator order), as bf16 hi + lo
-      if (c > c0) {
-        // rows of the products: queries tau = tb*16 + 4g + i; the gradient
-        // entries of those rows in this value column are d8[tb / 2] elements
-        // (tb % 2)*4 + i
-        auto add_rows = [&](int tb, floatx4 qm, floatx4 qmp) {
-          const floatx4 ra = *(const floatx4*)(tab + kTabRA + tb * 16 + 4 * g);
-          const floatx4 rb = *(const floatx4*)(tab + kTabRB + tb * 16 + 4 * g);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc += (ra[i] * qm[i] + rb[i] * qmp[i]) * elt(d8[tb >> 1], (tb & 1) * 4 + i);
-        };
-        bf16x4 th, tl, tph, tpl;
-        if (KTAIL) {
-          split_acc4(M[NKB - 1], th, tl);
-          split_acc4(Mp[NKB - 1], tph, tpl);
-        }
-        if constexpr (NK32 <= 2) {
-          // narrow keys: every state fragment split once, one query block at a time
-          constexpr int NJ = NK32 > 0 ? NK32 : 1;
-          bf16x8 mh[NJ], ml[NJ], mph[NJ], mpl[NJ];
-#pragma unroll
-          for (int j = 0; j < NK32; ++j) {
-            split_acc(M[2 * j], M[2 * j + 1], mh[j], ml[j]);
-            split_acc(Mp[2 * j], Mp[2 * j + 1], mph[j], mpl[j]);
-          }
-#pragma unroll
-          for (int tb = 0; tb < 4; ++tb) {
-            floatx4 qm = {0.f, 0.f, 0.f, 0.f}, qmp = qm;
-#pragma unroll
-            for (int j = 0; j < NK32; ++j) {
-              const auto qf = frow8<E>(Qs, L.qp, tb * 16 + l16, j, g);
-              qm = mma32(qf, mh[j], qm);
-              qm = mma32(qf, ml[j], qm);
-              qmp = mma32(qf, mph[j], qmp);
-              qmp = mma32(qf, mpl[j], qmp);
-            }
-            if (KTAIL) {
-              const auto qf = frow4<E>(Qs, L.qp, tb * 16 + l16, NK32, g);
-              qm = mma16(qf, th, qm);
-              qm = mma16(qf, tl, qm);
-              qmp = mma16(qf, tph, qmp);
-              qmp = mma16(qf, tpl, qmp);
-            }
-            add_rows(tb, qm, qmp);
-          }
-        } else {
-          // wide keys: one state fragment split at a time, all query blocks
-          floatx4 qm[4], qmp[4];
-#pragma unroll
-          for (int tb = 0; tb < 4; ++tb) qm[tb] = qmp[tb] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < NK32; ++j) {
-            bf16x8 mh, ml, mph, mpl;
-            split_acc(M[2 * j], M[2 * j + 1], mh, ml);
-            split_acc(Mp[2 * j], Mp[2 * j + 1], mph, mpl);
-#pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
-              const auto qf = frow8<E>(Qs, L.qp, tb * 16 + l16, j, g);
-              qm[tb] = mma32(qf, mh, qm[tb]);
-              qm[tb] = mma32(qf, ml, qm[tb]);
-              qmp[tb] = mma32(qf, mph, qmp[tb]);
-              qmp[tb] = mma32(qf, mpl, qmp[tb]);
-            }
-          }
-          if (KTAIL) {
-#pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
-              const auto qf = frow4<E>(Qs, L.qp, tb * 16 + l16, NK32, g);
-              qm[tb] = mma16(qf, th, qm[tb]);
-              qm[tb] = mma16(qf, tl, qm[tb]);
-              qmp[tb] = mma16(qf, tph, qmp[tb]);
-              qmp[tb] = mma16(qf, tpl, qmp[tb]);
-            }
-          }
-#pragma unroll
-          for (int tb = 0; tb < 4; ++tb) add_rows(tb, qm[tb], qmp[tb]);
-        }
-      }
-      // ---- query-side sums A, B
+    // ---- this tile's query sums against the states of the earlier tiles, and
+    // into the segment's (their weights start at the segment: off tokens back)
+    {
+      bf16x8 ah[2], al[2], bh8[2], bl8[2];
 #pragma unroll
       for (int kp = 0; kp < 2; ++kp) {
-        float wa[8], wb[8], xa[8], xb[8];
-        tab8(tab + kTabWA, kp, g, wa);
-        tab8(tab + kTabWB, kp, g, wb);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = elt(d8[kp], e);
-          xa[e] = x * wa[e];
-          xb[e] = x * wb[e];
-        }
-        bf16x8 ah, al, bh8, bl8;
-        split8(xa, ah, al);
-        split8(xb, bh8, bl8);
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-          const auto qc = TK::col8(Qs, L.qp, kb * 16, kp, lane);
-          A[kb] = mma32(qc, ah, A[kb]);
-          A[kb] = mma32(qc, al, A[kb]);
-          Bq[kb] = mma32(qc, bh8, Bq[kb]);
-          Bq[kb] = mma32(qc, bl8, Bq[kb]);
-        }
+        const bf16x8 q8 = TK::col8(Qs, L.qp, kb * 16, kp, lane);
+        weigh8(q8, tab + kTabRA, kp, g, ah[kp], al[kp]);
+        weigh8(q8, tab + kTabRB, kp, g, bh8[kp], bl8[kp]);
       }
-      // ---- states after this tile (relative to its last token)
-      const float dec = tab[kTabPow + len];
+      const float off = (float)((c - c0) * C), aoff = expf(la * off), aoff1 = aoff * off;
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb)
+      for (int n = 0; n < NVB; ++n) {
+        const int vb = vs + n * S;
+        floatx4 at = {0.f, 0.f, 0.f, 0.f}, bt = at;
+#pragma unroll
+        for (int kp = 0; kp < 2; ++kp) {
+          const bf16x8 d8 = TK::col8(Ds + vb * 16, L.vp, 0, kp, lane);
+          at = mma32(ah[kp], d8, at);
+          at = mma32(al[kp], d8, at);
+          bt = mma32(bh8[kp], d8, bt);
+          bt = mma32(bl8[kp], d8, bt);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          Mp[kb][i] = dec * (Mp[kb][i] + (float)len * M[kb][i]);
-          M[kb][i] *= dec;
+          acc += M[n][i] * at[i] + Mp[n][i] * bt[i];
+          A[n][i] += aoff * at[i] + aoff1 * bt[i];
+          Bq[n][i] += aoff * bt[i];
         }
+      }
+    }
+    // ---- states after this tile (relative to its last token)
+    {
+      bf16x8 mh[2], ml[2], mph[2], mpl[2];
 #pragma unroll
       for (int kp = 0; kp < 2; ++kp) {
-        float wm[8], wmp[8], xa[8], xb[8];
-        tab8(tab + kTabWM, kp, g, wm);
-        tab8(tab + kTabWMp, kp, g, wmp);
-        const bf16x8 v8 = TK::col8(Vw, L.vp, 0, kp, lane);
+        const bf16x8 k8 = TK::col8(Ks, L.qp, kb * 16, kp, lane);
+        weigh8(k8, tab + kTabWM, kp, g, mh[kp], ml[kp]);
+        weigh8(k8, tab + kTabWMp, kp, g, mph[kp], mpl[kp]);
+      }
+      const float dec = tab[kTabPow + len], dec1 = dec * (float)len;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = elt(v8, e);
-          xa[e] = x * wm[e];
-          xb[e] = x * wmp[e];
+      for (int n = 0; n < NVB; ++n) {
+        const int vb = vs + n * S;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          Mp[n][i] = dec * Mp[n][i] + dec1 * M[n][i];
+          M[n][i] *= dec;
         }
-        bf16x8 mh, ml, mph, mpl;
-        split8(xa, mh, ml);
-        split8(xb, mph, mpl);
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-          const auto kc = TK::col8(Ks, L.qp, kb * 16, kp, lane);
-          M[kb] = mma32(kc, mh, M[kb]);
-          M[kb] = mma32(kc, ml, M[kb]);
-          Mp[kb] = mma32(kc, mph, Mp[kb]);
-          Mp[kb] = mma32(kc, mpl, Mp[kb]);
+        for (int kp = 0; kp < 2; ++kp) {
+          const bf16x8 v8 = TK::col8(Vs + vb * 16, L.vp, 0, kp, lane);
+          M[n] = mma32(mh[kp], v8, M[n]);
+          M[n] = mma32(ml[kp], v8, M[n]);
+          Mp[n] = mma32(mph[kp], v8, Mp[n]);
+          Mp[n] = mma32(mpl[kp], v8, Mp[n]);
         }
       }
     }
@@ -461,20 +353,23 @@ __global__ __launch_bounds__(512) void retention_grad_kernel(RetP p) {
     for (int i = 0; i < nwave; ++i) s += red[i];
     p.part[(size_t)bh * p.nseg + seg] = s;
   }
-  if (owner) {
-    const size_t nel = (size_t)p.dk * vw;
-    float* out = p.sums + ((size_t)bh * p.nseg + seg) * 4 * nel;
+  // the first segment has no state before it, the last no segment after it
+  const size_t nel = (size_t)p.dk * vw;
+  float* out = p.sums + ((size_t)bh * p.nseg + seg) * 4 * nel;
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
+  for (int n = 0; n < NVB; ++n)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const size_t e = (size_t)(kb * 16 + 4 * g + i) * vw + w * 16 + l16;
-        out[e] = M[kb][i];
-        out[nel + e] = Mp[kb][i];
-        out[2 * nel + e] = A[kb][i];
-        out[3 * nel + e] = Bq[kb][i];
+    for (int i = 0; i < 4; ++i) {
+      const size_t e = (size_t)(kb * 16 + 4 * g + i) * vw + (vs + n * S) * 16 + l16;
+      if (seg + 1 < p.nseg) {
+        out[e] = M[n][i];
+        out[nel + e] = Mp[n][i];
       }
-  }
+      if (seg > 0) {
+        out[2 * nel + e] = A[n][i];
+        out[3 * nel + e] = Bq[n][i];
+      }
+    }
 }
 
 __global__ void retention_zero_kernel(float* out, int n) {
@@ -496,13 +391,14 @@ __global__ __launch_bounds__(256) void retention_combine_kernel(RetP p, float* p
   float acc = 0.f;
   if (e < nel) {
     float m = 0.f, mp = 0.f;
-    for (int s = 0; s < p.nseg; ++s) {
-      const float* base = p.sums + ((size_t)bh * p.nseg + s) * 4 * nel;
-      if (s > 0) acc += m * base[2 * nel + e] + mp * base[3 * nel + e];
-      const int len = min(seg_len, p.T - s * seg_len);
-      const float aL = expf(la * (float)len);
-      mp = aL * (mp + (float)len * m) + base[nel + e];
-      m = aL * m + base[e];
+    // every segment but the last is whole
+    const float aL = expf(la * (float)seg_len);
+#pragma unroll 4
+    for (int s = 1; s < p.nseg; ++s) {
+      const float* base = p.sums + ((size_t)bh * p.nseg + s - 1) * 4 * nel + e;
+      mp = aL * (mp + (float)seg_len * m) + base[nel];
+      m = aL * m + base[0];
+      acc += m * base[6 * nel] + mp * base[7 * nel];
     }
   }
   __shared__ float red[4];
@@ -531,16 +427,31 @@ using ts::fail;
 
 typedef void (*RetFn)(ts::RetP);
 
-RetFn pick_ret(int dk) {
+// Value blocks of a kernel with room for nw: 4, 5 (64 values and a mass
+// column) or 8, in whole multiples of the waves that share a key block.
+int ret_blocks(int dk, int nw) {
+  const int S = ts::ret_share(dk), n = nw <= 4 ? 4 : nw <= 5 ? 5 : 8;
+  return (n + S - 1) / S * S;
+}
+
+template <int DK>
+RetFn pick_ret_dk(int nw) {
+  constexpr int S = ts::ret_share(DK);
+  return nw <= (4 + S - 1) / S * S   ? ts::retention_grad_kernel<DK, (4 + S - 1) / S>
+         : nw <= (5 + S - 1) / S * S ? ts::retention_grad_kernel<DK, (5 + S - 1) / S>
+                                     : ts::retention_grad_kernel<DK, 8 / S>;
+}
+
+RetFn pick_ret(int dk, int nw) {
   switch (dk) {
-    case 16: return ts::retention_grad_kernel<16>;
-    case 32: return ts::retention_grad_kernel<32>;
-    case 48: return ts::retention_grad_kernel<48>;
-    case 64: return ts::retention_grad_kernel<64>;
-    case 80: return ts::retention_grad_kernel<80>;
-    case 96: return ts::retention_grad_kernel<96>;
-    case 112: return ts::retention_grad_kernel<112>;
-    case 128: return ts::retention_grad_kernel<128>;
+    case 16: return pick_ret_dk<16>(nw);
+    case 32: return pick_ret_dk<32>(nw);
+    case 48: return pick_ret_dk<48>(nw);
+    case 64: return pick_ret_dk<64>(nw);
+    case 80: return pick_ret_dk<80>(nw);
+    case 96: return pick_ret_dk<96>(nw);
+    case 112: return pick_ret_dk<112>(nw);
+    case 128: return pick_ret_dk<128>(nw);
   }
   return nullptr;
 }
@@ -561,20 +472,25 @@ int ret_plan(const ts_retention_desc* d, RetPlan* P) {
                 "retention grad: dk a multiple of 16 up to 128, dv a multiple of 8 (split wider keys)");
   P->dkp = d->dk;
   P->nvr = (d->dv + 15) / 16;
-  P->vw = (P->nvr + (d->has_mass ? 1 : 0)) * 16;
-  P->nw = P->vw / 16;
+  P->nw = P->nvr + (d->has_mass ? 1 : 0);
   if (P->nw > 8) return fail(TS_ERR_NOT_IMPLEMENTED, "retention grad: at most 8 value blocks per call (split wider values)");
-  // enough waves that every thread loads at most two chunks of each tile
-  P->waves = P->nw > d->dk / 16 ? P->nw : d->dk / 16;
+  P->nw = ret_blocks(d->dk, P->nw);
+  P->vw = P->nw * 16;
+  P->waves = d->dk / 16 * ts::ret_share(d->dk);
   if (ts::ret_layout(P->dkp, P->vw).bytes > ts::kLdsPerCU)
     return fail(TS_ERR_NOT_IMPLEMENTED, "retention grad: tiles of dk=%d and %d value columns exceed LDS (split the values)",
                 P->dkp, P->vw);
   const int tiles = (d->T + ts::C - 1) / ts::C;
   int st = d->seg_tiles;
   if (st <= 0) {
-    // about 512 workgroups, segments of at least two tiles
+    // at most 256 workgroups, one per CU, since more and shorter segments cost
+    // more in summaries than they hide (B8 H8 T4096, dk 128, 64 values + mass:
+    // 97 us against 117 us at 512; dk 32: 70 against 77); 512 for 16 keys,
+    // whose summaries are small and several of whose workgroups share a CU
+    // (56 us against 61 us).  Segments of at least two tiles.
+    const long most = d->dk <= 16 ? 512 : 256;
     st = 2;
-    while (st < tiles && (long)d->B * d->H * ((tiles + st - 1) / st) > 512) st *= 2;
+    while (st < tiles && (long)d->B * d->H * ((tiles + st - 1) / st) > most) st *= 2;
   }
   P->seg_tiles = st;
   P->nseg = tiles > 0 ? (tiles + st - 1) / st : 0;
@@ -648,13 +564,13 @@ int ts_retention_grad(const ts_retention_desc* d, const ts_retention_io* io, flo
   ts::RetP p;
   memset(&p, 0, sizeof(p));
   p.B = d->B; p.H = d->H; p.T = d->T; p.dk = P.dkp; p.dv = d->dv; p.nvr = P.nvr; p.has_mass = d->has_mass;
-  p.seg_tiles = P.seg_tiles; p.nseg = P.nseg; p.vw = P.vw; p.nw = P.nw;
+  p.seg_tiles = P.seg_tiles; p.nseg = P.nseg; p.vw = P.vw;
   p.q = io->q; p.k = io->k; p.v = io->v; p.dout = io->dout; p.dm = io->dmass;
   p.q_rec = rec[0]; p.k_rec = rec[1]; p.v_rec = rec[2]; p.o_rec = rec[3]; p.dm_rec = rec[4];
   p.log_alpha = io->log_alpha;
   p.part = (float*)workspace;
   p.sums = (float*)((char*)workspace + (P.part_bytes + 255) / 256 * 256);
-  RetFn fn = pick_ret(P.dkp);
+  RetFn fn = pick_ret(P.dkp, P.nw);
   if (!fn) return fail(TS_ERR_NOT_IMPLEMENTED, "retention grad: no kernel for dk=%d", P.dkp);
   const ts::RetLayout L = ts::ret_layout(P.dkp, P.vw);
   if (L.bytes > 65536) {
