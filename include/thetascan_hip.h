@@ -1115,6 +1115,34 @@ int ts_contract_tokens(const ts_contract_desc* desc, const void* a, int64_t a_sg
                        int64_t b_sg, int64_t b_sn, float* out, void* workspace, size_t ws_bytes,
                        hipStream_t stream);
 
+/* Several contractions over the same groups and tokens in one launch, and
+ * outputs formed from them: sum i is c_i = sum over its nterms[i] terms of
+ * sum_n a[g, n, :]^T b[g, n, :] ([G, p[i], q[i]], widths multiples of 16 up to
+ * 512), and an output is c_sum (+ scale * w o c_w_sum with w [G, p, q] of
+ * `dtype`), formed in fp32 and rounded once to out_dtype.  The terms of all
+ * sums follow each other in `terms`. */
+#define TS_CONTRACT_SUMS 4
+#define TS_CONTRACT_TERMS 2
+typedef struct ts_contract_sums_desc {
+  int32_t G, N, dtype, nsums;
+  int32_t p[TS_CONTRACT_SUMS], q[TS_CONTRACT_SUMS], nterms[TS_CONTRACT_SUMS];
+} ts_contract_sums_desc;
+typedef struct ts_contract_term {
+  const void* a;
+  const void* b;
+  int64_t a_sg, a_sn, b_sg, b_sn; /* element strides: group, token */
+} ts_contract_term;
+typedef struct ts_contract_out {
+  void* out;      /* [G, p, q] of out_dtype                 */
+  const void* w;  /* NULL: no scaled sum                    */
+  int32_t sum, w_sum;
+  float scale;
+  int32_t pad;
+} ts_contract_out;
+int ts_contract_sums_workspace_bytes(const ts_contract_sums_desc* desc, size_t* bytes);
+int ts_contract_sums(const ts_contract_sums_desc* desc, const ts_contract_term* terms, const ts_contract_out* outs,
+                     int32_t nouts, int32_t out_dtype, void* workspace, size_t ws_bytes, hipStream_t stream);
+
 /* ------------------------------------------------ depth-1 kernel memory */
 
 /* Everything between the input and the output projection of a depth-1

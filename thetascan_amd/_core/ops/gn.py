@@ -89,6 +89,39 @@ def contract_tokens(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return parts.view(H, S, p, q).sum(1, dtype=torch.float32)
 
 
+def _contract_sums(sums, outs, dtypes) -> list[torch.Tensor]:
+    """Weight gradients from several token contractions in one
+    ts_contract_sums call.  ``sums``: each a list of products ``(a, b)``
+    (head-major tiles [H, N, p] and [H, N, q]) that add; ``outs``: each
+    ``(sum, scaled)`` with ``scaled`` None or ``(w, sum, scale)`` for
+    + scale * w o (that sum); ``dtypes``: the outputs' dtypes."""
+    lib = _lib.load()
+    a0 = sums[0][0][0]
+    H, N = a0.shape[:2]
+    desc = _lib.ContractSumsDesc(H, N, _lib.dtype_code(a0.dtype), len(sums))
+    terms = (_lib.ContractTerm * sum(len(ts) for ts in sums))()
+    n = 0
+    for i, ts in enumerate(sums):
+        desc.p[i], desc.q[i], desc.nterms[i] = ts[0][0].shape[-1], ts[0][1].shape[-1], len(ts)
+        for a, b in ts:
+            terms[n] = _lib.ContractTerm(a.data_ptr(), b.data_ptr(), a.stride(0), a.stride(1), b.stride(0), b.stride(1))
+            n += 1
+    dt = dtypes[0] if len(set(dtypes)) == 1 and dtypes[0] in (torch.bfloat16, torch.float32) else torch.float32
+    res = [torch.empty(H, desc.p[i], desc.q[i], dtype=dt, device=a0.device) for i, _ in outs]
+    io = (_lib.ContractOut * len(outs))()
+    for j, (i, scaled) in enumerate(outs):
+        w, k, scale = scaled or (None, 0, 0.0)
+        io[j] = _lib.ContractOut(res[j].data_ptr(), _lib.ptr(w), i, k, scale, 0)
+    ws = ctypes.c_size_t()
+    _lib.check(lib.ts_contract_sums_workspace_bytes(ctypes.byref(desc), ctypes.byref(ws)), "contract workspace")
+    work = torch.empty(ws.value, dtype=torch.uint8, device=a0.device)
+    with _lib.timed("ts_contract_sums", lambda: _lib.nbytes(*(t for ts in sums for ab in ts for t in ab), *res)):
+        status = lib.ts_contract_sums(ctypes.byref(desc), terms, io, len(outs), _lib.dtype_code(dt), work.data_ptr(),
+                                      ws.value, _lib.stream_handle(a0.device))
+    _lib.check(status, "ts_contract_sums")
+    return [r if r.dtype == d else r.to(d) for r, d in zip(res, dtypes)]
+
+
 def _gn_write_forward(x: torch.Tensor, v: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, tau: torch.Tensor | None,
                  s: float, inv_depth: float, eps: float, act: int, damping: float) -> list[torch.Tensor]:
     lib = _lib.load()
@@ -152,13 +185,12 @@ def _gn_write_backward_impl(dh: torch.Tensor | None, dlam: torch.Tensor | None, 
         status = lib.ts_gn_write_bwd(ctypes.byref(desc), ctypes.byref(io), _lib.stream_handle(xk.device))
     _lib.check(status, "ts_gn_write_bwd")
     # dW1 = da^T x;  dW2 = lam^T dz + du^T h + 2 W2 o (drq^T s2);  dtau = -sum dpre
-    dw1 = contract_tokens(tm[2], td[2])
-    dw2 = contract_tokens(td[0], tm[0]) + contract_tokens(td[1], tm[1])
-    dw2 = dw2 + 2.0 * w2c.to(torch.float32) * contract_tokens(td[3], tm[3])
+    dw1, dw2 = _contract_sums([[(tm[2], td[2])], [(td[0], tm[0]), (td[1], tm[1])], [(td[3], tm[3])]],
+                              [(0, None), (1, (w2c, 2, 2.0))], [w1.dtype, w2.dtype])
     dtau = x.new_empty(0)
     if has_tau and need_tau:
         dtau = (-tm[4].sum(1, dtype=torch.float32)).to(tau.dtype)
-    return [dx, dv, dw1.to(w1.dtype), dw2.to(w2.dtype), dtau]
+    return [dx, dv, dw1, dw2, dtau]
 
 
 def _gn_write_backward_fake(dh, dlam, dg, x, v, w1, w2, tau, s, inv_depth, eps, act, damping, need_tau):
@@ -277,8 +309,10 @@ def _gn_read_backward_impl(dh: torch.Tensor | None, dresid: torch.Tensor | None,
     with _lib.timed("ts_gn_read_bwd", lambda: _lib.nbytes(qk, nk, mk, dh, dresid, dq, dnum, dmass, tm, td)):
         status = lib.ts_gn_read_bwd(ctypes.byref(desc), ctypes.byref(io), _lib.stream_handle(qk.device))
     _lib.check(status, "ts_gn_read_bwd")
-    dw1 = contract_tokens(tm[0], td[0]).to(w1.dtype)
-    dw2 = contract_tokens(td[1], tm[1]).to(w2.dtype) if want_resid else q.new_empty(0)
+    if want_resid:
+        dw1, dw2 = _contract_sums([[(tm[0], td[0])], [(td[1], tm[1])]], [(0, None), (1, None)], [w1.dtype, w2.dtype])
+    else:
+        (dw1,), dw2 = _contract_sums([[(tm[0], td[0])]], [(0, None)], [w1.dtype]), q.new_empty(0)
     dtau = (-tm[2].sum(1, dtype=torch.float32)).to(tau.dtype) if (has_tau and need_tau) else q.new_empty(0)
     dnum = q.new_empty(0) if dnum is None else dnum.to(num.dtype)
     dmass = q.new_empty(0) if dmass is None else dmass.to(mass.dtype)

@@ -210,6 +210,25 @@ class ContractDesc(ctypes.Structure):
                 ("dtype", ctypes.c_int32)]
 
 
+CONTRACT_SUMS, CONTRACT_TERMS = 4, 2
+
+
+class ContractSumsDesc(ctypes.Structure):
+    _fields_ = [("G", ctypes.c_int32), ("N", ctypes.c_int32), ("dtype", ctypes.c_int32), ("nsums", ctypes.c_int32),
+                ("p", ctypes.c_int32 * CONTRACT_SUMS), ("q", ctypes.c_int32 * CONTRACT_SUMS),
+                ("nterms", ctypes.c_int32 * CONTRACT_SUMS)]
+
+
+class ContractTerm(ctypes.Structure):
+    _fields_ = [("a", ctypes.c_void_p), ("b", ctypes.c_void_p), ("a_sg", ctypes.c_int64), ("a_sn", ctypes.c_int64),
+                ("b_sg", ctypes.c_int64), ("b_sn", ctypes.c_int64)]
+
+
+class ContractOut(ctypes.Structure):
+    _fields_ = [("out", ctypes.c_void_p), ("w", ctypes.c_void_p), ("sum", ctypes.c_int32), ("w_sum", ctypes.c_int32),
+                ("scale", ctypes.c_float), ("pad", ctypes.c_int32)]
+
+
 class ReadBwdIO(ctypes.Structure):
     _fields_ = [
         ("num", Strided),
@@ -590,6 +609,9 @@ def load() -> ctypes.CDLL:
         lib.ts_contract_tokens.argtypes = [P(ContractDesc), ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
                                            ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p,
                                            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        lib.ts_contract_sums_workspace_bytes.argtypes = [P(ContractSumsDesc), P(ctypes.c_size_t)]
+        lib.ts_contract_sums.argtypes = [P(ContractSumsDesc), P(ContractTerm), P(ContractOut), ctypes.c_int32,
+                                         ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         lib.ts_qknorm_fwd.argtypes = [P(QkNormDesc), Strided, Strided, ctypes.c_void_p, ctypes.c_void_p,
                                       ctypes.c_void_p]
         lib.ts_qknorm_bwd.argtypes = [P(QkNormDesc), Strided, Strided, Strided, ctypes.c_void_p, ctypes.c_void_p,
