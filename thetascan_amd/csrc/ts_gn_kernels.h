@@ -30,7 +30,7 @@
 // element, with tanh's code inlined at each) and rows are addressed with a
 // bound instead of a test (GnTok).  B8 H8 T2048 d64 m128, bf16: write forward
 // 98 -> 43 us, backward 305 -> 172 us (about 2 TB/s), read backward
-// 85 -> 73 us; hidden width 192 (B4 H16 T3001): write backward 447 -> 205 us,
+// 85 -> 73 us; hidden width 192 (B4 H8 T3001): write backward 447 -> 205 us,
 // read backward 187 -> 129 us.
 
 #pragma once
@@ -1027,8 +1027,10 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
   }
 }
 
+// Two waves per SIMD (237 registers, two workgroups' LDS on a CU): 205 -> 166 us
+// at B4 H8 T3001 d64 m192.
 template <int ACT, int D, int MB>
-__global__ __launch_bounds__(256) void gn_write_bwd_wide_kernel(GnP p) {
+__global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
   typedef bf16 E;
   constexpr int M = MB * 16;
   constexpr int NC = MB / 4;
