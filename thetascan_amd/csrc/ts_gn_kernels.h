@@ -25,15 +25,20 @@
 // are LDS weight rows and accumulator fragments of the previous product.
 //
 // What bounds these kernels is the chain per token group (products, row sums,
-// the nonlinearity), not memory, so it is kept free of branches: the
-// nonlinearity is a compile-time choice (a runtime one cost a compare per
-// element, with tanh's code inlined at each) and rows are addressed with a
-// bound instead of a test (GnTok).  B8 H8 T2048 d64 m128, bf16: write forward
-// 98 -> 43 us, backward 305 -> 172 us (about 2 TB/s), read backward
-// 85 -> 73 us; hidden width 192 (B4 H8 T3001): write backward 447 -> 205 us,
-// read backward 187 -> 129 us.
+// the nonlinearity) and the loads it waits for, at one or two waves per SIMD,
+// so the chain is kept free of branches -- the nonlinearity is a compile-time
+// choice (a runtime one cost a compare per element, with tanh's code inlined at
+// each) and rows are addressed with a bound instead of a test (GnTok) -- and a
+// group's loads go before its stores (GnAhead, GnRing).  B8 H8 T2048 d64 m128,
+// bf16: write forward 98 -> 42 us, backward 305 -> 137 us (2.6 TB/s), read
+// backward 85 -> 59 us; hidden width 192 (B4 H8 T3001): write backward
+// 447 -> 161 us, read forward 54 -> 36 us, backward 187 -> 104 us.  Of these
+// the order of loads and stores gave 173 -> 137 us of the write backward and
+// 128 -> 104 us of the wide read backward.
 
 #pragma once
+
+#include <type_traits>
 
 #include "ts_common.h"
 #include "ts_gn_act.h"
@@ -61,6 +66,7 @@ struct GnP {
 struct GnLayout {
   int xp, mp;
   int xs, w1, w2, w1t, w2t;
+  int tau;  // fp32 [m]
   int end;
 };
 __host__ __device__ constexpr GnLayout gn_layout(int esize, int d, int m, bool fwd, bool w_lds) {
@@ -77,6 +83,7 @@ __host__ __device__ constexpr GnLayout gn_layout(int esize, int d, int m, bool f
     L.w2t = off; off += m * L.xp;
     if (!fwd) { L.w1t = off; off += d * L.mp; }
   }
+  L.tau = off; off += m * 4 / esize;
   L.end = off;
   return L;
 }
@@ -100,6 +107,7 @@ __host__ __device__ constexpr GnLayout gn_read_layout(int esize, int d, int m, b
       L.w2t = off; off += m * L.xp;
     }
   }
+  L.tau = off; off += m * 4 / esize;
   L.end = off;
   return L;
 }
@@ -177,6 +185,64 @@ __device__ __forceinline__ void st4_tile(void* base, int64_t n0, const GnTok& tk
   gn_st<E>(make_rsrc((E*)base + n0 * w, kGnRowsEnd), gn_off(tk, (uint32_t)(tk.row * w + c) * (uint32_t)sizeof(E)), v);
 }
 
+// Row blocks c0 + 16 i of a stream, loaded ahead of their use and kept as
+// loaded.  Vector memory completes in order, so a load issued after stores is
+// waited for together with them: a group's loads go first, before its stores.
+// ON = false (the widest rows and fp32, where the registers are short): each
+// block is loaded where it is used.
+template <typename E, int NB, bool ON>
+struct GnAhead {
+  typedef typename std::conditional<sizeof(E) == 2, uint2, uint4>::type Raw;
+  Raw r[ON ? NB : 1];
+  __device__ __forceinline__ void load(const Str& s, int b, int h, const GnTok& tk, int c0) {
+    if constexpr (ON) {
+      const rsrc_t rs = gn_rows<E>(s, b, h, tk);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const uint32_t off = gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c0 + 16 * i) * (uint32_t)sizeof(E));
+        if constexpr (sizeof(E) == 2) r[i] = bld8(rs, off);
+        else r[i] = bld16(rs, off);
+      }
+    }
+  }
+  __device__ __forceinline__ void step(const Str&, int, int, const GnTok&, int, int) {}
+  __device__ __forceinline__ void get(const Str& s, int b, int h, const GnTok& tk, int c0, int i, float* o) const {
+    if constexpr (ON) {
+      if constexpr (sizeof(E) == 2) {
+        const bf16x4 v = __builtin_bit_cast(bf16x4, r[i]);
+        o[0] = tof(v[0]); o[1] = tof(v[1]); o[2] = tof(v[2]); o[3] = tof(v[3]);
+      } else {
+        const floatx4 v = __builtin_bit_cast(floatx4, r[i]);
+        o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
+      }
+    } else {
+      ld4_row<E>(s, b, h, tk, c0 + 16 * i, o);
+    }
+  }
+};
+
+// The chunked kernels' form of it: 64 features (four blocks) of a stream, the
+// next chunk loaded before the present one's stores.
+struct GnRing {
+  uint2 cur[4], nxt[4];
+  __device__ __forceinline__ void load(const Str& s, int b, int h, const GnTok& tk, int g, int c) {
+    const rsrc_t rs = gn_rows<bf16>(s, b, h, tk);
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+      nxt[f] = bld8(rs, gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c * 64 + f * 16 + 4 * g) * 2u));
+  }
+  // the loaded chunk becomes the present one; chunk c is loaded
+  __device__ __forceinline__ void step(const Str& s, int b, int h, const GnTok& tk, int g, int c) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) cur[f] = nxt[f];
+    load(s, b, h, tk, g, c);
+  }
+  __device__ __forceinline__ void get(const Str&, int, int, const GnTok&, int, int i, float* o) const {
+    const bf16x4 v = __builtin_bit_cast(bf16x4, cur[i & 3]);
+    o[0] = tof(v[0]); o[1] = tof(v[1]); o[2] = tof(v[2]); o[3] = tof(v[3]);
+  }
+};
+
 // out[db] = (Wt o Wt) reg: gemm_back with every weight squared on its way
 // into the MFMA (the reference squares W2 elementwise, engine.py:244).
 template <typename E, int D, int MB>
@@ -215,8 +281,9 @@ struct GnToken {
   float rinv, xx, hh;
 };
 
-template <int ACT, typename E, int D, int MB>
-__device__ __forceinline__ void gn_forward_token(const GnP& p, int b, int h, const GnTok& tk, int l16, int g,
+template <int ACT, typename E, int D, int MB, typename V>
+__device__ __forceinline__ void gn_forward_token(const GnP& p, int b, int h, const GnTok& tk, const V& v_a, int l16,
+                                                 int g,
                                                  const E* xrow, const E* xs_w, int xp, const E* w1, int wp1,
                                                  const E* w2, int wp2, const float* tau, GnToken<E, D, MB>& k,
                                                  floatx4* hv, floatx4* s2v) {
@@ -224,7 +291,7 @@ __device__ __forceinline__ void gn_forward_token(const GnP& p, int b, int h, con
 #pragma unroll
   for (int db = 0; db < D / 16; ++db) {
     ld4f<E>(xrow + db * 16 + 4 * g, k.xr[db]);
-    ld4_row<E>(p.v, b, h, tk, db * 16 + 4 * g, k.vr[db]);
+    v_a.get(p.v, b, h, tk, 4 * g, db, k.vr[db]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) xx += k.xr[db][i] * k.xr[db][i];
   }
@@ -270,8 +337,8 @@ __device__ __forceinline__ void gn_forward_token(const GnP& p, int b, int h, con
 }
 
 // Two waves per SIMD for the bf16 forward up to 64-wide tokens and 128 hidden
-// features (216 registers at the largest; B8 T2048 H8: 43 us).  The backward
-// at that width needs 500.
+// features (212 registers at the largest; B8 T2048 H8: 42 us).  The backward
+// at that width needs 480.
 template <int ACT, typename E, int D, int MB>
 __global__ __launch_bounds__(256, (sizeof(E) == 2 && D <= 64 && MB <= 8 ? 2 : 1)) void gn_write_fwd_kernel(GnP p) {
   constexpr int M = MB * 16;
@@ -296,7 +363,9 @@ __global__ __launch_bounds__(256, (sizeof(E) == 2 && D <= 64 && MB <= 8 ? 2 : 1)
     wp1 = L.xp;
     wp2 = L.mp;
   }
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const Rows<E> xsrc = rows_of<E>(p.x, b, h);
   RowTile<E, D> ldx;
   ldx.init(D, tid);
@@ -307,14 +376,16 @@ __global__ __launch_bounds__(256, (sizeof(E) == 2 && D <= 64 && MB <= 8 ? 2 : 1)
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();       // weights staged; previous group consumed
     ldx.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    GnAhead<E, D / 16, sizeof(E) == 2 && MB <= 8> v_a;
+    v_a.load(p.v, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     GnToken<E, D, MB> k;
     floatx4 hv[MB], s2v[MB];
-    gn_forward_token<ACT, E, D, MB>(p, b, h, tk, l16, g, xs + row * L.xp, xs + w * 16 * L.xp, L.xp, w1, wp1, w2,
+    gn_forward_token<ACT, E, D, MB>(p, b, h, tk, v_a, l16, g, xs + row * L.xp, xs + w * 16 * L.xp, L.xp, w1, wp1, w2,
                                wp2, tau, k, hv, s2v);
     floatx4 z[MB];
     gemm_back<E, M, D / 16>(w2t, wp1, k.lam, l16, g, D / 16, z);
@@ -368,7 +439,9 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
     wpd = L.xp;
     wpm = L.mp;
   }
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const int64_t N = (int64_t)p.B * p.T;
   // slot-major tiles: slot k of head h starts at k * H * N * w + h * N * w
   E* tm = (E*)p.tm + (int64_t)h * N * M;  // dz, h, da, s2 (, dpre)
@@ -384,15 +457,22 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldx.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    constexpr bool AHEAD = sizeof(E) == 2 && MB <= 8;
+    GnAhead<E, MB, AHEAD> dg_a, dh_a;
+    GnAhead<E, D / 16, AHEAD> v_a, dlam_a;
+    v_a.load(p.v, b, h, tk, 4 * g);
+    dg_a.load(p.dg, b, h, tk, 4 * g);
+    dlam_a.load(p.dlam, b, h, tk, 4 * g);
+    dh_a.load(p.dh, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     const int64_t n0 = (int64_t)b * p.T + t0;
     GnToken<E, D, MB> k;
     floatx4 hv[MB], s2v[MB];
-    gn_forward_token<ACT, E, D, MB>(p, b, h, tk, l16, g, xs + row * L.xp, xs + w * 16 * L.xp, L.xp, w1, wpd, w2,
+    gn_forward_token<ACT, E, D, MB>(p, b, h, tk, v_a, l16, g, xs + row * L.xp, xs + w * 16 * L.xp, L.xp, w1, wpd, w2,
                                wpm, tau, k, hv, s2v);
     // tiles known after the forward: h, s2, lam, x
 #pragma unroll
@@ -417,7 +497,7 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
 #pragma unroll
       for (int fb = 0; fb < MB; ++fb) {
         float dgv[4], tv[4];
-        ld4_row<E>(p.dg, b, h, tk, fb * 16 + 4 * g, dgv);
+        dg_a.get(p.dg, b, h, tk, 4 * g, fb, dgv);
         tau4(tau, p.has_tau, fb, g, tv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -440,7 +520,7 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
 #pragma unroll
       for (int db = 0; db < D / 16; ++db) {
         float dlv[4];
-        ld4_row<E>(p.dlam, b, h, tk, db * 16 + 4 * g, dlv);
+        dlam_a.get(p.dlam, b, h, tk, 4 * g, db, dlv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float dl = p.s * dlv[i] + wdz[db][i];
@@ -500,7 +580,7 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
 #pragma unroll
       for (int fb = 0; fb < MB; ++fb) {
         float dhv[4];
-        ld4_row<E>(p.dh, b, h, tk, fb * 16 + 4 * g, dhv);
+        dh_a.get(p.dh, b, h, tk, 4 * g, fb, dhv);
         float tv[4] = {0.f, 0.f, 0.f, 0.f};
         if (p.has_tau) {
           const floatx4 t4 = *(const floatx4*)(tau + fb * 16 + 4 * g);
@@ -532,8 +612,8 @@ __global__ __launch_bounds__(256) void gn_write_bwd_kernel(GnP p) {
     gemm_back<E, D, MB>(w1t, wpm, da, l16, g, MB, wda);
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
-      float dxi[4], o[4];
-      ld4_row<E>(p.dxin, b, h, tk, db * 16 + 4 * g, dxi);
+      float dxi[4] = {0.f, 0.f, 0.f, 0.f}, o[4];
+      if (p.dxin.ptr) ld4_row<E>(p.dxin, b, h, tk, db * 16 + 4 * g, dxi);
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = dxi[i] - dr[db][i] + 2.f * k.xr[db][i] * dxx + wda[db][i];
       st4_row<E>(p.dx, b, h, tk, db * 16 + 4 * g, o);
@@ -569,18 +649,26 @@ struct GnReadP {
   void* td;  // [2, H, B*T, d]: q, s dresid
 };
 
-template <typename E, int D, int MB>
-__device__ __forceinline__ float gn_read_preact(const GnReadP& p, int b, int h, const GnTok& tk, int l16, int g,
-                                                const E* xs_w, int xp, const E* w1, int wp1, floatx4* a,
+// Feature blocks up to which the chunked read kernels keep a group's streams.
+constexpr int kGnAheadWide = 12;
+
+// The key mass of a token (1 where none is read).
+__device__ __forceinline__ float gn_mass(const GnReadP& p, int b, int h, const GnTok& tk) {
+  return p.corr == 2 && tk.valid() ? p.mass[b * p.msb + h * p.msh + (int64_t)tk.t() * p.mst] : 1.f;
+}
+
+template <typename E, int D, int MB, typename Num>
+__device__ __forceinline__ float gn_read_preact(const GnReadP& p, int b, int h, const GnTok& tk, const Num& num,
+                                                float mass, int l16, int g, const E* xs_w, int xp, const E* w1, int wp1, floatx4* a,
                                                 float& cinv) {
   gemm_a<E, D, MB>(w1, wp1, xs_w, xp, l16, g, MB, a);
   cinv = 1.f;
   if (p.corr) {
-    if (p.corr == 2) cinv = tk.valid() ? 1.f / (p.mass[b * p.msb + h * p.msh + (int64_t)tk.t() * p.mst] + p.eps) : 0.f;
+    if (p.corr == 2) cinv = tk.valid() ? 1.f / (mass + p.eps) : 0.f;
 #pragma unroll
     for (int fb = 0; fb < MB; ++fb) {
       float c[4];
-      ld4_row<E>(p.num, b, h, tk, fb * 16 + 4 * g, c);
+      num.get(p.num, b, h, tk, 4 * g, fb, c);
 #pragma unroll
       for (int i = 0; i < 4; ++i) a[fb][i] += c[i] * cinv;
     }
@@ -623,7 +711,9 @@ __global__ __launch_bounds__(256) void gn_read_fwd_kernel(GnReadP p) {
     wp1 = L.xp;
     wp2 = L.mp;
   }
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const Rows<E> qsrc = rows_of<E>(p.q, b, h);
   RowTile<E, D> ldq;
   ldq.init(D, tid);
@@ -634,14 +724,16 @@ __global__ __launch_bounds__(256) void gn_read_fwd_kernel(GnReadP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldq.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
-    const bool valid = tk.valid();
+    GnAhead<E, MB, sizeof(E) == 2 && MB <= 8> num_a;
+    const float mass = gn_mass(p, b, h, tk);
+    if (p.corr) num_a.load(p.num, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
+    __syncthreads();
     floatx4 a[MB], hv[MB];
     float cinv;
-    const float rinv = gn_read_preact<E, D, MB>(p, b, h, tk, l16, g, xs + w * 16 * L.xp, L.xp, w1, wp1, a,
+    const float rinv = gn_read_preact<E, D, MB>(p, b, h, tk, num_a, mass, l16, g, xs + w * 16 * L.xp, L.xp, w1, wp1, a,
                                                 cinv);
 #pragma unroll
     for (int fb = 0; fb < MB; ++fb) {
@@ -671,7 +763,7 @@ __global__ __launch_bounds__(256) void gn_read_fwd_kernel(GnReadP p) {
 }
 
 template <int ACT, typename E, int D, int MB>
-__global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
+__global__ __launch_bounds__(256, (sizeof(E) == 2 && D <= 64 && MB <= 8 ? 2 : 1)) void gn_read_bwd_kernel(GnReadP p) {
   constexpr int M = MB * 16;
   constexpr bool WL = gn_read_weights_in_lds<E, D, MB, false>();
   const int b = blockIdx.z, h = blockIdx.y;
@@ -694,7 +786,9 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
     wpd = L.xp;
     wpm = L.mp;
   }
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const int64_t N = (int64_t)p.B * p.T;
   // slot-major tiles: slot k of head h starts at k * H * N * w + h * N * w
   E* tm = (E*)p.tm + (int64_t)h * N * M;  // da, h (, dpre)
@@ -710,15 +804,22 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldq.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    constexpr bool AHEAD = sizeof(E) == 2 && MB <= 8;
+    GnAhead<E, MB, AHEAD> num_a, dh_a;
+    GnAhead<E, D / 16, AHEAD> dres_a;
+    const float mass = gn_mass(p, b, h, tk);
+    if (p.corr) num_a.load(p.num, b, h, tk, 4 * g);
+    dres_a.load(p.dresid, b, h, tk, 4 * g);
+    dh_a.load(p.dh, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     const int64_t n0 = (int64_t)b * p.T + t0;
     floatx4 a[MB];
     float cinv;
-    const float rinv = gn_read_preact<E, D, MB>(p, b, h, tk, l16, g, xs + w * 16 * L.xp, L.xp, w1, wpd, a,
+    const float rinv = gn_read_preact<E, D, MB>(p, b, h, tk, num_a, mass, l16, g, xs + w * 16 * L.xp, L.xp, w1, wpd, a,
                                                 cinv);
     float dres[D / 16][4], qv[D / 16][4];
     floatx4 dres4[D / 16];
@@ -726,7 +827,7 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
       ld4f<E>(qrow + db * 16 + 4 * g, qv[db]);
-      ld4_row<E>(p.dresid, b, h, tk, db * 16 + 4 * g, dres[db]);
+      dres_a.get(p.dresid, b, h, tk, 4 * g, db, dres[db]);
       float sd[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -749,7 +850,7 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
     for (int fb = 0; fb < MB; ++fb) {
       float tv[4], dhv[4], hvv[4], dpv[4];
       tau_of<MB>(tau, fb, g, p.has_tau, tv);
-      ld4_row<E>(p.dh, b, h, tk, fb * 16 + 4 * g, dhv);
+      dh_a.get(p.dh, b, h, tk, 4 * g, fb, dhv);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float pre = a[fb][i] * rinv - tv[i];
@@ -769,7 +870,7 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
     for (int fb = 0; fb < MB; ++fb) {
       float o[4], dn[4];
       float c[4] = {0.f, 0.f, 0.f, 0.f};
-      if (p.corr == 2) ld4_row<E>(p.num, b, h, tk, fb * 16 + 4 * g, c);
+      if (p.corr == 2) num_a.get(p.num, b, h, tk, 4 * g, fb, c);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         da[fb][i] = da[fb][i] * rinv - c3 * a[fb][i];
@@ -811,6 +912,7 @@ __global__ __launch_bounds__(256) void gn_read_bwd_kernel(GnReadP p) {
 struct GnWideLayout {
   int xp, mp;
   int xs, w1, w2;  // element offsets; w2 holds W2 [d][mp] or W2^T [m][xp]
+  int tau;  // fp32 [m]
   int end;
 };
 // w2_rows: 0 (no W2), 1 (W2 as [d][m + 8]), 2 (W2^T as [m][d + 8])
@@ -824,6 +926,7 @@ __host__ __device__ constexpr GnWideLayout gn_wide_layout(int d, int m, int w2_r
   L.w2 = -1;
   if (w2_rows == 1) { L.w2 = off; off += d * L.mp; }
   if (w2_rows == 2) { L.w2 = off; off += m * L.xp; }
+  L.tau = off; off += m * 2;
   L.end = off;
   return L;
 }
@@ -962,7 +1065,9 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
   E* w2s = base + L.w2;
   stage_matrix<E>((const E*)p.w1 + (size_t)h * M * D, M, D, w1s, L.xp, tid);
   stage_matrix<E>((const E*)p.w2 + (size_t)h * D * M, D, M, w2s, L.mp, tid);
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const Rows<E> xsrc = rows_of<E>(p.x, b, h);
   RowTile<E, D> ldx;
   ldx.init(D, tid);
@@ -973,10 +1078,12 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();       // weights staged; previous group consumed
     ldx.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    GnAhead<E, D / 16, true> v_a;
+    v_a.load(p.v, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     const E* xs_w = xs + w * 16 * L.xp;
     float xr[D / 16][4], vr[D / 16][4];
@@ -984,7 +1091,7 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
       ld4f<E>(xs + row * L.xp + db * 16 + 4 * g, xr[db]);
-      ld4_row<E>(p.v, b, h, tk, db * 16 + 4 * g, vr[db]);
+      v_a.get(p.v, b, h, tk, 4 * g, db, vr[db]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) xx += xr[db][i] * xr[db][i];
     }
@@ -1027,8 +1134,8 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
   }
 }
 
-// Two waves per SIMD (237 registers, two workgroups' LDS on a CU): 205 -> 166 us
-// at B4 H8 T3001 d64 m192.
+// Two waves per SIMD (two workgroups' LDS fit a CU): 205 -> 166 us at B4 H8 T3001
+// d64 m192 when it was given them.
 template <int ACT, int D, int MB>
 __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
   typedef bf16 E;
@@ -1044,7 +1151,9 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
   E* w2s = base + L.w2;
   stage_matrix<E>((const E*)p.w1 + (size_t)h * M * D, M, D, w1s, L.xp, tid);
   stage_matrix<E>((const E*)p.w2 + (size_t)h * D * M, D, M, w2s, L.mp, tid);
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const int64_t N = (int64_t)p.B * p.T;
   // slot-major tiles: slot k of head h starts at k * H * N * w + h * N * w
   E* tm = (E*)p.tm + (int64_t)h * N * M;  // dz, h, da, s2 (, dpre)
@@ -1060,10 +1169,15 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldx.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    GnAhead<E, D / 16, true> v_a, dlam_a;
+    v_a.load(p.v, b, h, tk, 4 * g);
+    dlam_a.load(p.dlam, b, h, tk, 4 * g);
+    GnRing dg_a, dh_a;
+    dg_a.load(p.dg, b, h, tk, g, 0);
+    if (grp + 1 < p.groups) ldx.fetch(xsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     const int64_t n0 = (int64_t)b * p.T + t0;
     const E* xs_w = xs + w * 16 * L.xp;
@@ -1072,7 +1186,7 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
       ld4f<E>(xs + row * L.xp + db * 16 + 4 * g, xr[db]);
-      ld4_row<E>(p.v, b, h, tk, db * 16 + 4 * g, vr[db]);
+      v_a.get(p.v, b, h, tk, 4 * g, db, vr[db]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) xx += xr[db][i] * xr[db][i];
     }
@@ -1103,13 +1217,15 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
 #pragma unroll 1
     for (int c = 0; c < NC; ++c) {
       floatx4 a[4], z[4], dz[4];
+      dg_a.step(p.dg, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
+      if (c + 1 == NC) dh_a.load(p.dh, b, h, tk, g, 0);
       gnw_a<D>(w1s, L.xp, xs_w, c, l16, g, a);
       gnw_w2t<D, false>(w2s, L.mp, c, lam, lane, z);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         float tv[4], dgv[4];
         tau_of<MB>(tau, 4 * c + f, g, p.has_tau, tv);
-        ld4_row<E>(p.dg, b, h, tk, c * 64 + f * 16 + 4 * g, dgv);
+        dg_a.get(p.dg, b, h, tk, 4 * g, f, dgv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float pre = a[f][i] * rinv - tv[i];
@@ -1129,7 +1245,7 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
       float dlv[4];
-      ld4_row<E>(p.dlam, b, h, tk, db * 16 + 4 * g, dlv);
+      dlam_a.get(p.dlam, b, h, tk, 4 * g, db, dlv);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float dl = p.s * dlv[i] + wdz[db][i];
@@ -1161,6 +1277,8 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
     // dsp = s dg z rinv + 2 sp rinv ((W2 o W2)^T drq) rinv; adds the chunk's share to drinv
     auto dpre_chunk = [&](int c, floatx4* a, floatx4* dpre, float& drv) {
       floatx4 z[4], ds2[4], dhu[4];
+      dg_a.step(p.dg, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
+      dh_a.step(p.dh, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
       gnw_a<D>(w1s, L.xp, xs_w, c, l16, g, a);
       gnw_w2t<D, false>(w2s, L.mp, c, lam, lane, z);
       gnw_w2t<D, true>(w2s, L.mp, c, drq, lane, ds2);
@@ -1169,8 +1287,8 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
       for (int f = 0; f < 4; ++f) {
         float tv[4], dgv[4], dhv[4];
         tau_of<MB>(tau, 4 * c + f, g, p.has_tau, tv);
-        ld4_row<E>(p.dg, b, h, tk, c * 64 + f * 16 + 4 * g, dgv);
-        ld4_row<E>(p.dh, b, h, tk, c * 64 + f * 16 + 4 * g, dhv);
+        dg_a.get(p.dg, b, h, tk, 4 * g, f, dgv);
+        dh_a.get(p.dh, b, h, tk, 4 * g, f, dhv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float pre = a[f][i] * rinv - tv[i];
@@ -1222,8 +1340,8 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
     }
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
-      float dxi[4], o[4];
-      ld4_row<E>(p.dxin, b, h, tk, db * 16 + 4 * g, dxi);
+      float dxi[4] = {0.f, 0.f, 0.f, 0.f}, o[4];
+      if (p.dxin.ptr) ld4_row<E>(p.dxin, b, h, tk, db * 16 + 4 * g, dxi);
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = dxi[i] - dr[db][i] + 2.f * xr[db][i] * dxx + wda[db][i];
       st4_row<E>(p.dx, b, h, tk, db * 16 + 4 * g, o);
@@ -1232,31 +1350,32 @@ __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
 }
 
 // a + correction of chunk c for the read stage (c = num or num / (mass + eps))
-template <int D>
-__device__ __forceinline__ void gnw_read_a(const GnReadP& p, int b, int h, const GnTok& tk, const bf16* w1s, int xp,
-                                           const bf16* xs_w, int c, int l16, int g, float cinv, floatx4* a) {
+template <int D, typename Num>
+__device__ __forceinline__ void gnw_read_a(const GnReadP& p, int b, int h, const GnTok& tk, const Num& num,
+                                           const bf16* w1s, int xp, const bf16* xs_w, int c, int l16, int g, float cinv, floatx4* a) {
   gnw_a<D>(w1s, xp, xs_w, c, l16, g, a);
   if (p.corr) {
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       float cv[4];
-      ld4_row<bf16>(p.num, b, h, tk, c * 64 + f * 16 + 4 * g, cv);
+      num.get(p.num, b, h, tk, 4 * g, 4 * c + f, cv);
 #pragma unroll
       for (int i = 0; i < 4; ++i) a[f][i] += cv[i] * cinv;
     }
   }
 }
 
-template <int D, int MB>
-__device__ __forceinline__ float gnw_read_rinv(const GnReadP& p, int b, int h, const GnTok& tk, const bf16* w1s,
-                                               int xp, const bf16* xs_w, int l16, int g, float& cinv) {
+template <int D, int MB, typename Num>
+__device__ __forceinline__ float gnw_read_rinv(const GnReadP& p, int b, int h, const GnTok& tk, Num& num,
+                                               float mass, const bf16* w1s, int xp, const bf16* xs_w, int l16, int g, float& cinv) {
   cinv = 1.f;
-  if (p.corr == 2) cinv = tk.valid() ? 1.f / (p.mass[b * p.msb + h * p.msh + (int64_t)tk.t() * p.mst] + p.eps) : 0.f;
+  if (p.corr == 2) cinv = tk.valid() ? 1.f / (mass + p.eps) : 0.f;
   float ss = 0.f;
-#pragma unroll 1
+#pragma unroll (std::is_same<Num, GnRing>::value || MB > kGnAheadWide ? 1 : MB / 4)
   for (int c = 0; c < MB / 4; ++c) {
     floatx4 a[4];
-    gnw_read_a<D>(p, b, h, tk, w1s, xp, xs_w, c, l16, g, cinv, a);
+    if (p.corr) num.step(p.num, b, h, tk, g, c + 1 < MB / 4 ? c + 1 : 0);
+    gnw_read_a<D>(p, b, h, tk, num, w1s, xp, xs_w, c, l16, g, cinv, a);
 #pragma unroll
     for (int f = 0; f < 4; ++f)
 #pragma unroll
@@ -1270,6 +1389,7 @@ __global__ __launch_bounds__(256) void gn_read_fwd_wide_kernel(GnReadP p) {
   typedef bf16 E;
   constexpr int M = MB * 16;
   constexpr int NC = MB / 4;
+  constexpr bool AHEAD = MB <= kGnAheadWide;
   const int b = blockIdx.z, h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, g = lane >> 4;
   const GnWideLayout L = gn_wide_layout(D, M, p.want_resid ? 1 : 0);
@@ -1280,7 +1400,9 @@ __global__ __launch_bounds__(256) void gn_read_fwd_wide_kernel(GnReadP p) {
   E* w2s = base + L.w2;
   stage_matrix<E>((const E*)p.w1 + (size_t)h * M * D, M, D, w1s, L.xp, tid);
   if (p.want_resid) stage_matrix<E>((const E*)p.w2 + (size_t)h * D * M, D, M, w2s, L.mp, tid);
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const Rows<E> qsrc = rows_of<E>(p.q, b, h);
   RowTile<E, D> ldq;
   ldq.init(D, tid);
@@ -1291,21 +1413,23 @@ __global__ __launch_bounds__(256) void gn_read_fwd_wide_kernel(GnReadP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldq.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
-    const bool valid = tk.valid();
+    GnAhead<E, MB, AHEAD> num_a;
+    const float mass = gn_mass(p, b, h, tk);
+    if (p.corr) num_a.load(p.num, b, h, tk, 4 * g);
+    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
+    __syncthreads();
     const E* xs_w = xs + w * 16 * L.xp;
     float cinv;
-    const float rinv = gnw_read_rinv<D, MB>(p, b, h, tk, w1s, L.xp, xs_w, l16, g, cinv);
+    const float rinv = gnw_read_rinv<D, MB>(p, b, h, tk, num_a, mass, w1s, L.xp, xs_w, l16, g, cinv);
     floatx4 u[D / 16];
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) u[db] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
+#pragma unroll (AHEAD ? NC : 1)
     for (int c = 0; c < NC; ++c) {
       floatx4 a[4], hv[4];
-      gnw_read_a<D>(p, b, h, tk, w1s, L.xp, xs_w, c, l16, g, cinv, a);
+      gnw_read_a<D>(p, b, h, tk, num_a, w1s, L.xp, xs_w, c, l16, g, cinv, a);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         float tv[4], o[4];
@@ -1334,7 +1458,7 @@ __global__ __launch_bounds__(256) void gn_read_fwd_wide_kernel(GnReadP p) {
 }
 
 template <int ACT, int D, int MB>
-__global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
+__global__ __launch_bounds__(256, 2) void gn_read_bwd_wide_kernel(GnReadP p) {
   typedef bf16 E;
   typedef LdsIO<E> IO;
   constexpr int M = MB * 16;
@@ -1349,7 +1473,9 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
   E* w2ts = base + L.w2;  // W2^T [m][xp]
   stage_matrix<E>((const E*)p.w1 + (size_t)h * M * D, M, D, w1s, L.xp, tid);
   if (p.want_resid) stage_matrix<E>((const E*)p.w2t + (size_t)h * M * D, M, D, w2ts, L.xp, tid);
-  const float* tau = p.has_tau ? p.tau + h * M : nullptr;
+  float* tau = (float*)(base + L.tau);
+  if (p.has_tau)
+    for (int i = tid; i < M; i += 256) tau[i] = p.tau[h * M + i];
   const int64_t N = (int64_t)p.B * p.T;
   E* tm = (E*)p.tm + (int64_t)h * N * M;  // da, h (, dpre)
   E* td = (E*)p.td + (int64_t)h * N * D;  // q, s dresid
@@ -1364,15 +1490,21 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
     if (t0 >= p.T) break;  // uniform over the workgroup
     __syncthreads();
     ldq.store(xs, L.xp);
-    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
-    __syncthreads();
     const int row = w * 16 + l16;
     const GnTok tk{t0, row, p.T};
+    GnRing num_a, dh_a;
+    GnAhead<E, D / 16, true> dres_a;
+    const float mass = gn_mass(p, b, h, tk);
+    if (p.corr) num_a.load(p.num, b, h, tk, g, 0);
+    dres_a.load(p.dresid, b, h, tk, 4 * g);
+    dh_a.load(p.dh, b, h, tk, g, 0);
+    if (grp + 1 < p.groups) ldq.fetch(qsrc, t0 + TT, p.T);
+    __syncthreads();
     const bool valid = tk.valid();
     const int64_t n0 = (int64_t)b * p.T + t0;
     const E* xs_w = xs + w * 16 * L.xp;
     float cinv;
-    const float rinv = gnw_read_rinv<D, MB>(p, b, h, tk, w1s, L.xp, xs_w, l16, g, cinv);
+    const float rinv = gnw_read_rinv<D, MB>(p, b, h, tk, num_a, mass, w1s, L.xp, xs_w, l16, g, cinv);
     float dres[D / 16][4];
     floatx4 dres4[D / 16];
     const E* qrow = xs + row * L.xp;
@@ -1380,7 +1512,7 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
     for (int db = 0; db < D / 16; ++db) {
       float qv[4], sd[4];
       ld4f<E>(qrow + db * 16 + 4 * g, qv);
-      ld4_row<E>(p.dresid, b, h, tk, db * 16 + 4 * g, dres[db]);
+      dres_a.get(p.dresid, b, h, tk, 4 * g, db, dres[db]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         dres4[db][i] = dres[db][i];
@@ -1403,12 +1535,12 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
                            IO::from_acc(dres4[2 * kk], dres4[2 * kk + 1]), dhr[f]);
         }
       }
-      gnw_read_a<D>(p, b, h, tk, w1s, L.xp, xs_w, c, l16, g, cinv, a);
+      gnw_read_a<D>(p, b, h, tk, num_a, w1s, L.xp, xs_w, c, l16, g, cinv, a);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         float tv[4], dhv[4];
         tau_of<MB>(tau, 4 * c + f, g, p.has_tau, tv);
-        ld4_row<E>(p.dh, b, h, tk, c * 64 + f * 16 + 4 * g, dhv);
+        dh_a.get(p.dh, b, h, tk, 4 * g, 4 * c + f, dhv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float pre = a[f][i] * rinv - tv[i];
@@ -1421,6 +1553,8 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
 #pragma unroll 1
     for (int c = 0; c < NC; ++c) {
       floatx4 a[4], dpre[4];
+      if (p.corr) num_a.step(p.num, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
+      dh_a.step(p.dh, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
       dpre_chunk(c, a, dpre);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
@@ -1445,12 +1579,14 @@ __global__ __launch_bounds__(256) void gn_read_bwd_wide_kernel(GnReadP p) {
 #pragma unroll 1
     for (int c = 0; c < NC; ++c) {
       floatx4 a[4], da[4];
+      if (p.corr) num_a.step(p.num, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
+      dh_a.step(p.dh, b, h, tk, g, c + 1 < NC ? c + 1 : 0);
       dpre_chunk(c, a, da);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         float o[4], dn[4];
         float cv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (p.corr == 2) ld4_row<E>(p.num, b, h, tk, c * 64 + f * 16 + 4 * g, cv);
+        if (p.corr == 2) num_a.get(p.num, b, h, tk, 4 * g, 4 * c + f, cv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           da[f][i] = da[f][i] * rinv - c3 * a[f][i];
