@@ -1,9 +1,9 @@
-"""Feature widths of 192 and 384 on the chunked feature kernels (GPU tests).
+"""Feature widths of 192 and 384 on the wide feature kernels (GPU tests).
 
 The published expanded kernel preset has m = 384 (192 trainable projection
 rows, sign-expanded twice); a memory multiplier of 3 at head width 64, or of
-6 at head width 32, gives m = 192.  These widths run the chunked kernels in
-bf16 (the feature axis walked 64 features at a time).  Each mixer below runs
+6 at head width 32, gives m = 192.  These widths run the wide kernels in
+bf16 (a token's whole feature row in registers).  Each mixer below runs
 them on the multi-view path and is checked against the float64 oracle, across
 both feature maps, input and feature RoPE, the learned ReLU^2 threshold,
 shared key/query, banks, the ema stream and the plain sum, with a ragged last
@@ -87,7 +87,7 @@ def test_wide_feature_mixer_matches_float64_oracle(cuda, name):
 
 
 def test_wide_widths_stay_on_the_composed_path_in_fp32(cuda):
-    """The chunked kernels are bf16 only: an fp32 mixer at m = 384 takes the
+    """The wide kernels are bf16 only: an fp32 mixer at m = 384 takes the
     composed path and still matches the oracle at the fp32 bar."""
     pub = _preset()
     module = build_module(pub, cuda, torch.float32)
@@ -100,3 +100,76 @@ def test_wide_widths_stay_on_the_composed_path_in_fp32(cuda):
     y = module(x.to(cuda, torch.float32))
     assert module._core.last_path == "composed"
     assert rel_err(y, y64) < 1e-3
+
+
+@pytest.mark.parametrize("T", [1, 63, 65, 257])
+@pytest.mark.parametrize("kind,m,d,feat_rot", [("relu2", 384, 64, 0), ("relu2", 192, 32, 64), ("softmax", 384, 64, 128),
+                                               ("softmax", 192, 64, 0)])
+def test_wide_features_at_tile_edges(cuda, T, kind, m, d, feat_rot):
+    """Features, the query's residual read and every gradient at the edges of
+    the 64-token groups, rows of a strided view, keys (no residual) and
+    queries, against float64 autograd of the definition on the same bf16
+    inputs.  The bf16 rounding of xn (2^-9 per entry) and of the outputs puts
+    a ReLU^2 feature off by about 2 * 2^-8, a softmax one of sharpness 8 by 8
+    times its pre-activation's error: 2-norm bars of 2e-2 and 4e-2; the
+    gradients add dphi's and da's roundings (3e-2 and 6e-2)."""
+    from thetascan_amd._core.ops.features import kernel_features
+    from thetascan_amd._core.ops.fused import FeatureSpec
+    from thetascan_amd import _lib
+
+    B, H, eps = 2, 3, 1e-6
+    g = torch.Generator().manual_seed(T + m + d)
+    x = torch.randn(B, T, H, d, generator=g).bfloat16()
+    w1 = (torch.randn(H, m, d, generator=g)).bfloat16()
+    w2 = (torch.randn(H, d, m, generator=g) * 0.3).bfloat16()
+    tau = torch.randn(H, generator=g) * 0.1
+    dphi = torch.randn(B, H, T, m, generator=g).bfloat16()
+    dres = torch.randn(B, H, T, d, generator=g).bfloat16()
+    in_rot = d // 2
+
+    def turn(v, rot):
+        inv = 1.0 / (10_000.0 ** (torch.arange(0, rot, 2, dtype=torch.float64) / rot))
+        f = torch.outer(torch.arange(T, dtype=torch.float64), inv)
+        a, b = v[..., :rot:2], v[..., 1:rot:2]
+        r = torch.stack((a * f.cos() - b * f.sin(), a * f.sin() + b * f.cos()), -1).flatten(-2)
+        return torch.cat((r, v[..., rot:]), -1)
+
+    for resid in (False, True):
+        leaves = [t.double().clone().requires_grad_(True) for t in (x, w1, w2, tau)]
+        lx, l1, l2, lt = leaves
+        xr = turn(lx.transpose(1, 2), in_rot)
+        xn = xr / xr.norm(dim=-1, keepdim=True).clamp_min(eps)
+        a = xn @ l1.transpose(-1, -2)
+        pre = a * torch.rsqrt(a.square().mean(-1, keepdim=True) + eps) - lt.view(1, H, 1, 1)
+        if kind == "relu2":
+            f = torch.relu(pre).square()
+            h = f / f.sum(-1, keepdim=True)
+        else:
+            h = torch.softmax(8.0 * pre, -1)
+        phi = turn(h, feat_rot) if feat_rot else h
+        r64 = xn + h @ l2.transpose(-1, -2)
+        loss = (phi * dphi.double()).sum() + ((r64 * dres.double()).sum() if resid else 0.0)
+        loss.backward()
+
+        dev = [t.to(cuda).requires_grad_(True) for t in (x, w1, w2, tau)]
+        spec = FeatureSpec(_lib.FEAT_RELU2 if kind == "relu2" else _lib.FEAT_SOFTMAX, m, 8.0, in_rot, feat_rot,
+                           10_000.0, 1.0, eps)
+        got, base = kernel_features(dev[0].transpose(1, 2), dev[1], dev[2] if resid else None, dev[3], spec, resid)
+        out = (got.float() * dphi.to(cuda).float()).sum()
+        if resid:
+            out = out + (base.float() * dres.to(cuda).float()).sum()
+        out.backward()
+        torch.cuda.synchronize()
+
+        def err(t, ref):
+            return float((t.double().cpu() - ref).norm() / ref.norm())
+
+        bar, gbar = (2e-2, 3e-2) if kind == "relu2" else (4e-2, 6e-2)
+        errs = {"phi": err(got.detach(), phi.detach())}
+        if resid:
+            errs["resid"] = err(base.detach(), r64.detach())
+        grads = {n: err(t.grad, l.grad) for n, t, l in zip(("dx", "dw1", "dw2", "dtau"), dev, leaves)
+                 if l.grad is not None and (n != "dtau" or kind == "relu2")}  # (a shift leaves a softmax as it is)
+        print(f"wide {kind} m={m} d={d} T={T} resid={resid}: {errs} {grads}", flush=True)
+        assert all(e < bar for e in errs.values()), errs
+        assert all(e < gbar for e in grads.values()), grads

@@ -37,7 +37,7 @@ _EXPANSION_FINGERPRINT_SCHEMA_VERSION = 1
 
 FUSED_HEAD_DIMS = (16, 32, 64, 128)
 FUSED_FEATURE_WIDTHS = (16, 32, 64, 128, 256)
-# widths the chunked feature kernels take: bf16 streams, head widths 32 and 64
+# widths the wide feature kernels take: bf16 streams, head widths 32 and 64
 WIDE_FEATURE_WIDTHS = (192, 384)
 WIDE_HEAD_DIMS = (32, 64)
 

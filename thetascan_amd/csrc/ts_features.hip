@@ -733,36 +733,35 @@ __global__ __launch_bounds__(256, (sizeof(E) == 2 && D <= 64 && MB <= 4 ? (RESID
 
 // ------------------------------------------------------------------ wide maps
 //
-// Feature widths of 192 and 384 (bf16, head widths 32 and 64): the per-lane
-// feature arrays of the kernels above would not fit in registers, so these
-// walk the feature axis 64 features at a time, re-forming the chunk's
-// a^T = W1 xn^T on MFMA in every pass that needs it (RMSNorm sum, mass or
-// softmax max/sum, then h; in the backward dh . h, sum dp and dp . a, then
-// da).  W1 (and W2) are staged in LDS once per workgroup; W1^T and W2^T
-// operands are transposing LDS reads of the staged rows.  The backward
-// writes da, xn, h and dtau per token for the weight-gradient GEMMs (no
-// fused weight-gradient partials at these widths).
+// Feature widths of 192 and 384 (bf16, head widths 32 and 64).  W1 (and W2)
+// are staged in LDS once per workgroup, which leaves one or two waves per
+// SIMD, and a wave then has 512 or 256 registers per lane: a token's whole
+// feature row (96 floats per lane at 384) and, in the backward, its gradient
+// beside it stay in registers, so a^T = W1 xn^T is formed once and dphi is
+// read once.  (Walking the axis 64 features at a time and re-forming a in
+// every pass over it took three to five times the MFMAs, with two barriers
+// or three exposed reads of dphi per chunk.  B8 H8 T4096 d64 m384: forward,
+// mean of keys and queries, 157 -> 86 us, backward 255 -> 191 us for keys and
+// 465 -> 275 us for queries.)  Bound by the rows: 0.2 GB of phi, or 0.4 to 0.65 GB of dphi, da
+// and h.  Every wave loads, computes and stores its own 16 tokens of a group,
+// so the group loop has no barrier.  The backward writes da, xn, h and dtau
+// per token for the weight-gradient GEMMs (no fused weight-gradient partials
+// at these widths).
 
 struct WideLayout {
-  int xp, cp, mp;
-  int xs, cs, rs, os, w1, w2;  // element offsets
+  int xp, mp;
+  int xs, rs, w1, w2;  // element offsets
   int end;
 };
 
 __host__ __device__ constexpr WideLayout wide_layout(int d, int m, bool fwd, bool resid) {
   WideLayout L{};
   L.xp = d + 8;
-  L.cp = 64 + 8;
   L.mp = m + 8;
   int off = 0;
   L.xs = off; off += TT * L.xp;
-  L.cs = L.rs = L.os = -1;
-  if (fwd) {
-    L.cs = off; off += TT * L.cp;
-  } else {
-    if (resid) { L.rs = off; off += TT * L.xp; }
-    L.os = off; off += TT * L.xp;
-  }
+  L.rs = -1;
+  if (!fwd && resid) { L.rs = off; off += TT * L.xp; }
   L.w1 = off; off += m * L.xp;
   L.w2 = -1;
   if (resid) { L.w2 = off; off += d * L.mp; }
@@ -770,98 +769,14 @@ __host__ __device__ constexpr WideLayout wide_layout(int d, int m, bool fwd, boo
   return L;
 }
 
-// a^T of feature chunk c (blocks 4c..4c+3) for this wave's 16 tokens.
-template <int D>
-__device__ __forceinline__ void wide_a(const bf16* w1s, int xp, const bf16* xs_w, int c, int l16, int g, floatx4* a) {
-  gemm_a<bf16, D, 4>(w1s + c * 64 * xp, xp, xs_w, xp, l16, g, 4, a);
-}
-
-// Per-token statistics over the whole width: rinv (RMSNorm) and the
-// normalizer (ReLU^2 mass, or the softmax max mx and sum).
-template <int D, int KIND, int NC>
-__device__ __forceinline__ void wide_stats(const FeatP& p, float tau, const bf16* w1s, int xp, const bf16* xs_w,
-                                           int l16, int g, float& rinv, float& mass, float& mx) {
-  float ss = 0.f;
-#pragma unroll 1
-  for (int c = 0; c < NC; ++c) {
-    floatx4 a[4];
-    wide_a<D>(w1s, xp, xs_w, c, l16, g, a);
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ss += a[f][i] * a[f][i];
-  }
-  rinv = rsqrtf(sum_g(ss) * p.inv_m + p.eps);
-  mx = 0.f;
-  if constexpr (KIND == TS_FEAT_RELU2) {
-    float sf = 0.f;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4];
-      wide_a<D>(w1s, xp, xs_w, c, l16, g, a);
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pre = fmaxf(a[f][i] * rinv - tau, 0.f);
-          sf += pre * pre;
-        }
-    }
-    mass = sum_g(sf);
-  } else {
-    float m_ = -INFINITY;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4];
-      wide_a<D>(w1s, xp, xs_w, c, l16, g, a);
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m_ = fmaxf(m_, p.gain * (a[f][i] * rinv - tau));
-    }
-    mx = max_g(m_);
-    float se = 0.f;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4];
-      wide_a<D>(w1s, xp, xs_w, c, l16, g, a);
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) se += __expf(p.gain * (a[f][i] * rinv - tau) - mx);
-    }
-    mass = sum_g(se);
-  }
-}
-
-// h of one chunk from its a and the statistics.
-template <int KIND>
-__device__ __forceinline__ void wide_h(const FeatP& p, float tau, const floatx4* a, float rinv, float mass, float mx,
-                                       floatx4* hc) {
-  if constexpr (KIND == TS_FEAT_RELU2) {
-    const bool ok = mass > p.eps;
-    const float inv = ok ? rcp(mass) : 0.f;
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pre = fmaxf(a[f][i] * rinv - tau, 0.f);
-        hc[f][i] = ok ? pre * pre * inv : p.inv_m;
-      }
-  } else {
-    const float inv = rcp(mass);
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) hc[f][i] = __expf(p.gain * (a[f][i] * rinv - tau) - mx) * inv;
-  }
-}
-
+// The rows of W1 are fed to the MFMAs in the order that leaves eight
+// consecutive features in a lane (blocks 2j and 2j + 1: features 32j + 8g + i
+// and 32j + 8g + 4 + i), so phi is stored from registers in 16-byte vectors
+// and W2 is read from LDS in 16-byte vectors.
 template <int D, int MB, int KIND>
-__global__ __launch_bounds__(256) void feature_fwd_wide_kernel(FeatP p) {
+__global__ __launch_bounds__(256, 2) void feature_fwd_wide_kernel(FeatP p) {
   typedef bf16 E;
   typedef LdsIO<E> IO;
-  constexpr int NC = MB / 4;
   constexpr int m = MB * 16;
   const int b = blockIdx.z, h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, g = lane >> 4;
@@ -870,7 +785,6 @@ __global__ __launch_bounds__(256) void feature_fwd_wide_kernel(FeatP p) {
   extern __shared__ __align__(16) unsigned char smem[];
   E* base = (E*)smem;
   E* xs = base + L.xs;
-  E* cs = base + L.cs;
   E* w1s = base + L.w1;
   E* w2s = base + L.w2;
   stage_matrix<E>((const E*)p.w1 + (size_t)h * m * D, m, D, w1s, L.xp, tid);
@@ -879,84 +793,94 @@ __global__ __launch_bounds__(256) void feature_fwd_wide_kernel(FeatP p) {
   const Rows<E> xsrc = rows_of<E>(p.x, b, h);
   const Rows<E> phi = rows_of<E>(p.phi, b, h);
 
-  RowTile<E, D> ldx;
-  ldx.init(D, tid);
   const int g0 = blockIdx.x * p.groups;
-  ldx.fetch(xsrc, g0 * TT, p.T);
   const int ng = min(p.groups, (p.T + TT - 1) / TT - g0);
+  WaveRows<E, D> ldx;
+  ldx.init(D, w, lane);
+  ldx.fetch_all(xsrc, g0 * TT, p.T);
+  __syncthreads();  // weights staged
   for (int grp = 0; grp < ng; ++grp) {
     const int t0 = (g0 + grp) * TT;
-    __syncthreads();  // weights staged; previous group's rows written out
-    ldx.store(xs, L.xp);
+    wave_lds_sync();  // the previous group's rows written out
+    ldx.store_valid(xs, L.xp, t0, p.T);
     const int row = w * 16 + l16;
     const int t = t0 + row;
     const bool valid = t < p.T;
     RopeRegs<D / 16> ir;
     ir.fetch(p.in_rot, p.in_cos, p.in_sin, t, valid, g);
-    ldx.fetch(xsrc, t0 + TT, grp + 1 < ng ? p.T : 0);
-    __syncthreads();
+    // (past the last group: the last rows again, cached and never stored)
+    ldx.fetch_all(xsrc, t0 + TT, p.T);
+    wave_lds_sync();
 
     E* xrow = xs + row * L.xp;
-    const E* xs_w = xs + w * 16 * L.xp;
     float xr[D / 16][4];
     bool big;
     const float inv =
         load_xn<E, D>(p, [&](float* v, int db) { ir.apply(v, db, p.in_rot, g, false); }, g, xrow, xr, big);
     wave_lds_sync();  // this wave's xn rows complete before they feed its MFMAs
 
-    float rinv, mass, mx;
-    wide_stats<D, KIND, NC>(p, tau, w1s, L.xp, xs_w, l16, g, rinv, mass, mx);
-    floatx4 rb[D / 16];
+    floatx4 hv[MB];
+    {
+      const E* xl = xs + (w * 16 + l16) * L.xp + 8 * g;
+      const E* wl = w1s + (8 * (l16 >> 2) + (l16 & 3)) * L.xp + 8 * g;
 #pragma unroll
-    for (int db = 0; db < D / 16; ++db) rb[db] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4], hc[4];
-      wide_a<D>(w1s, L.xp, xs_w, c, l16, g, a);
-      wide_h<KIND>(p, tau, a, rinv, mass, mx, hc);
-      if (want_resid) {
+      for (int fb = 0; fb < MB; ++fb) {
+        const E* wrow = wl + ((fb >> 1) * 32 + (fb & 1) * 4) * L.xp;
+        hv[fb] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int db = 0; db < D / 16; ++db) {
-          const E* wrow = w2s + (db * 16 + l16) * L.mp + c * 64;
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-            rb[db] = mma32(IO::cat(IO::ld4(wrow + 32 * jj + 4 * g), IO::ld4(wrow + 32 * jj + 16 + 4 * g)),
-                           IO::from_acc(hc[2 * jj], hc[2 * jj + 1]), rb[db]);
-        }
+        for (int kk = 0; kk < D / 32; ++kk)
+          hv[fb] = mma32(IO::ld8(wrow + kk * 32), IO::ld8(xl + kk * 32), hv[fb]);
       }
-      E* crow = cs + row * L.cp;
+    }
+    float rinv, mass;
+    feature_map<KIND, MB>(p, tau, hv, MB, hv, rinv, mass);  // in place
+    E* prow = phi.at(valid ? t : 0);
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        float v[4] = {hc[f][0], hc[f][1], hc[f][2], hc[f][3]};
-        const int col = c * 64 + f * 16 + 4 * g;
-        if (c * 64 + f * 16 < p.feat_rot)
-          rope4(v, col, p.feat_rot, p.f_cos, p.f_sin, t, valid && col < p.feat_rot, false);
-        st4f<E>(crow + f * 16 + 4 * g, v);
+    for (int j = 0; j < MB / 2; ++j) {
+      const int col = 32 * j + 8 * g;
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = hv[2 * j][i];
+        v[4 + i] = hv[2 * j + 1][i];
       }
-      __syncthreads();
-      write_rows<E>(cs, L.cp, Rows<E>{phi.base + c * 64, phi.st}, t0, p.T, 64, tid);
-      __syncthreads();
+      if (32 * j < p.feat_rot) {
+        rope4(v, col, p.feat_rot, p.f_cos, p.f_sin, t, valid && col < p.feat_rot, false);
+        rope4(v + 4, col + 4, p.feat_rot, p.f_cos, p.f_sin, t, valid && col + 4 < p.feat_rot, false);
+      }
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (bf16)v[i];
+      if (valid) *(uint4*)(prow + col) = __builtin_bit_cast(uint4, o);
     }
     if (want_resid) {
 #pragma unroll
       for (int db = 0; db < D / 16; ++db) {
+        floatx4 r = {0.f, 0.f, 0.f, 0.f};
+        const E* wrow = w2s + (db * 16 + l16) * L.mp + 8 * g;
+#pragma unroll
+        for (int j = 0; j < MB / 2; ++j)
+          r = mma32(IO::ld8(wrow + 32 * j), IO::from_acc(hv[2 * j], hv[2 * j + 1]), r);
         float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = xr[db][i] * inv + p.s * rb[db][i];
-        st4f<E>(xrow + db * 16 + 4 * g, v);
+        for (int i = 0; i < 4; ++i) v[i] = xr[db][i] * inv + p.s * r[i];
+        st4f<E>(xrow + db * 16 + 4 * g, v);  // resid over this lane's own xn entries
       }
-      __syncthreads();
-      write_rows<E>(xs, L.xp, rows_of<E>(p.resid, b, h), t0, p.T, D, tid);
+      wave_lds_sync();
+      write_rows_wave<E>(xs, L.xp, rows_of<E>(p.resid, b, h), t0, p.T, D, w, lane);
     }
   }
 }
 
+// One wave per SIMD with up to 512 registers: a token's a and dh take 192, and
+// at 256 the kernel spills.  In place of a second wave, the next group's rows
+// (its dphi too, once this group's is unpacked) are in flight while a group
+// is computed.
 template <int D, int MB, bool RESID, int KIND>
-__global__ __launch_bounds__(256) void feature_bwd_wide_kernel(FeatP p) {
+__global__ __launch_bounds__(256, 1) void feature_bwd_wide_kernel(FeatP p) {
   typedef bf16 E;
   typedef LdsIO<E> IO;
   typedef TokFrag<E> TF;
-  constexpr int NC = MB / 4;
   constexpr int m = MB * 16;
   const int b = blockIdx.z, h = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, g = lane >> 4;
@@ -965,7 +889,6 @@ __global__ __launch_bounds__(256) void feature_bwd_wide_kernel(FeatP p) {
   E* base = (E*)smem;
   E* xs = base + L.xs;
   E* rs = base + L.rs;
-  E* os = base + L.os;
   E* w1s = base + L.w1;
   E* w2s = base + L.w2;
   stage_matrix<E>((const E*)p.w1 + (size_t)h * m * D, m, D, w1s, L.xp, tid);
@@ -975,147 +898,166 @@ __global__ __launch_bounds__(256) void feature_bwd_wide_kernel(FeatP p) {
   const Rows<E> rsrc = rows_of<E>(p.dresid, b, h);
   const Rows<E> psrc = rows_of<E>(p.dphi, b, h);
 
-  RowTile<E, D> ldx, ldr;
-  ldx.init(D, tid);
-  ldr.init(RESID ? D : 0, tid);
   const int g0 = blockIdx.x * p.groups;
-  ldx.fetch(xsrc, g0 * TT, p.T);
-  if (RESID) ldr.fetch(rsrc, g0 * TT, p.T);
   const int ng = min(p.groups, (p.T + TT - 1) / TT - g0);
+  WaveRows<E, D> ldx, ldr;
+  ldx.init(D, w, lane);
+  ldx.fetch_all(xsrc, g0 * TT, p.T);
+  if (RESID) {
+    ldr.init(D, w, lane);
+    ldr.fetch_all(rsrc, g0 * TT, p.T);
+  }
+  // a token's dphi row (tokens past T read the last row; their gradients are
+  // zeroed where they are used)
+  uint2 dpr[MB];
+  auto fetch_dphi = [&](int t) {
+    const E* prow = psrc.at(min(t, p.T - 1)) + 4 * g;
+#pragma unroll
+    for (int fb = 0; fb < MB; ++fb) dpr[fb] = *(const uint2*)(prow + fb * 16);
+  };
+  fetch_dphi(g0 * TT + w * 16 + l16);
+  __syncthreads();  // weights staged
   for (int grp = 0; grp < ng; ++grp) {
     const int t0 = (g0 + grp) * TT;
-    __syncthreads();  // weights staged; previous group fully consumed
-    ldx.store(xs, L.xp);
-    if (RESID) ldr.store(rs, L.xp);
+    wave_lds_sync();  // the previous group's rows consumed
+    ldx.store_valid(xs, L.xp, t0, p.T);
+    if (RESID) ldr.store_valid(rs, L.xp, t0, p.T);
     const int row = w * 16 + l16;
     const int t = t0 + row;
     const bool valid = t < p.T;
     RopeRegs<D / 16> ir;
     ir.fetch(p.in_rot, p.in_cos, p.in_sin, t, valid, g);
-    const int next_T = grp + 1 < ng ? p.T : 0;
-    ldx.fetch(xsrc, t0 + TT, next_T);
-    if (RESID) ldr.fetch(rsrc, t0 + TT, next_T);
-    __syncthreads();
+    // (past the last group: the last rows again, cached and never stored)
+    ldx.fetch_all(xsrc, t0 + TT, p.T);
+    if (RESID) ldr.fetch_all(rsrc, t0 + TT, p.T);
+    wave_lds_sync();
 
-    const E* prow = psrc.at(valid ? t : 0);
     E* xrow = xs + row * L.xp;
-    const E* xs_w = xs + w * 16 * L.xp;
     float xr[D / 16][4];
     bool big;
     const float inv =
         load_xn<E, D>(p, [&](float* v, int db) { ir.apply(v, db, p.in_rot, g, false); }, g, xrow, xr, big);
     wave_lds_sync();  // this wave's xn rows complete before they feed its MFMAs
 
-    float rinv, mass, mx;
-    wide_stats<D, KIND, NC>(p, tau, w1s, L.xp, xs_w, l16, g, rinv, mass, mx);
-    const E* rrow = rs + row * L.xp;
-    // a, h and dh = rotate^T(dphi) + s W2^T dresid of chunk c
-    auto chunk = [&](int c, floatx4* a, floatx4* hc, floatx4* dh) {
-      uint2 dpr[4];
+    floatx4 a[MB], dh[MB];
+    gemm_a<E, D, MB>(w1s, L.xp, xs + w * 16 * L.xp, L.xp, l16, g, MB, a);
+    // statistics over the width: RMSNorm, then the ReLU^2 mass, or the softmax max and sum
+    float ss = 0.f;
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
-        dpr[f] = valid ? *(const uint2*)(prow + c * 64 + f * 16 + 4 * g) : make_uint2(0u, 0u);
-      wide_a<D>(w1s, L.xp, xs_w, c, l16, g, a);
-      wide_h<KIND>(p, tau, a, rinv, mass, mx, hc);
+    for (int fb = 0; fb < MB; ++fb)
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        dh[f] = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (RESID) {
+      for (int i = 0; i < 4; ++i) ss += a[fb][i] * a[fb][i];
+    const float rinv = rsqrtf(sum_g(ss) * p.inv_m + p.eps);
+    float mass = 0.f, mx = 0.f;
+    if constexpr (KIND == TS_FEAT_RELU2) {
 #pragma unroll
-          for (int kk = 0; kk < D / 32; ++kk)
-            dh[f] = mma32(TF::get(w2s, L.mp, c * 64 + f * 16, kk, lane),
-                          IO::cat(IO::ld4(rrow + 32 * kk + 4 * g), IO::ld4(rrow + 32 * kk + 16 + 4 * g)), dh[f]);
+      for (int fb = 0; fb < MB; ++fb)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) dh[f][i] *= p.s;
+        for (int i = 0; i < 4; ++i) {
+          const float pre = fmaxf(a[fb][i] * rinv - tau, 0.f);
+          mass += pre * pre;
         }
-        float v[4] = {__uint_as_float(dpr[f].x << 16), __uint_as_float(dpr[f].x & 0xffff0000u),
-                      __uint_as_float(dpr[f].y << 16), __uint_as_float(dpr[f].y & 0xffff0000u)};
-        const int col = c * 64 + f * 16 + 4 * g;
-        if (c * 64 + f * 16 < p.feat_rot)
-          rope4(v, col, p.feat_rot, p.f_cos, p.f_sin, t, valid && col < p.feat_rot, true);
+    } else {
+      mx = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dh[f][i] += v[i];
+      for (int fb = 0; fb < MB; ++fb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, p.gain * (a[fb][i] * rinv - tau));
+      mx = max_g(mx);
+#pragma unroll
+      for (int fb = 0; fb < MB; ++fb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mass += __expf(p.gain * (a[fb][i] * rinv - tau) - mx);
+    }
+    mass = sum_g(mass);
+    const bool ok = KIND == TS_FEAT_SOFTMAX || mass > p.eps;
+    const float minv = ok ? rcp(mass) : 0.f;
+    // h of one a.  `r` is rinv, made opaque anew by each pass below: what a
+    // pass forms from a is formed again in the next one, not kept in another
+    // 96 registers that would spill.
+    auto h_of = [&](float av, float r) {
+      if constexpr (KIND == TS_FEAT_RELU2) {
+        const float pre = fmaxf(av * r - tau, 0.f);
+        return ok ? pre * pre * minv : p.inv_m;
+      } else {
+        return __expf(p.gain * (av * r - tau) - mx) * minv;
       }
     };
-    // pass 1: sdh = dh . h
+    float r1 = rinv;
+    asm volatile("" : "+v"(r1));
+
+    // dh = rotate^T(dphi) + s W2^T dresid, and sdh = dh . h
+    const E* rrow = rs + row * L.xp;
     float sdh = 0.f;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4], hc[4], dh[4];
-      chunk(c, a, hc, dh);
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+    for (int fb = 0; fb < MB; ++fb) {
+      dh[fb] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (RESID) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sdh += dh[f][i] * hc[f][i];
+        for (int kk = 0; kk < D / 32; ++kk)
+          dh[fb] = mma32(TF::get(w2s, L.mp, fb * 16, kk, lane),
+                         IO::cat(IO::ld4(rrow + 32 * kk + 4 * g), IO::ld4(rrow + 32 * kk + 16 + 4 * g)), dh[fb]);
+      }
+      const uint2 dp = valid ? dpr[fb] : make_uint2(0u, 0u);
+      float v[4] = {__uint_as_float(dp.x << 16), __uint_as_float(dp.x & 0xffff0000u), __uint_as_float(dp.y << 16),
+                    __uint_as_float(dp.y & 0xffff0000u)};
+      const int col = fb * 16 + 4 * g;
+      if (fb * 16 < p.feat_rot)
+        rope4(v, col, p.feat_rot, p.f_cos, p.f_sin, t, valid && col < p.feat_rot, true);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dh[fb][i] = RESID ? fmaf(dh[fb][i], p.s, v[i]) : v[i];
+        sdh += dh[fb][i] * h_of(a[fb][i], r1);
+      }
     }
+    fetch_dphi(t + TT);
     sdh = sum_g(sdh);
-    const float scale = KIND == TS_FEAT_RELU2 ? (mass > p.eps ? 2.0f * rcp(mass) : 0.f) : p.gain;
-    // dp of a chunk (left in dh)
-    auto dp_of = [&](const floatx4* a, const floatx4* hc, floatx4* dh) {
+    // dp over dh; sum dp and dp . a
+    const float scale = KIND == TS_FEAT_RELU2 ? 2.0f * minv : p.gain;
+    float sdp = 0.f, sda = 0.f, r2 = rinv;
+    asm volatile("" : "+v"(r2));
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+    for (int fb = 0; fb < MB; ++fb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (KIND == TS_FEAT_RELU2)
-            dh[f][i] = (dh[f][i] - sdh) * scale * fmaxf(a[f][i] * rinv - tau, 0.f);
-          else
-            dh[f][i] = scale * hc[f][i] * (dh[f][i] - sdh);
-        }
-    };
-    // pass 2: sum dp, dp . a
-    float sdp = 0.f, sda = 0.f;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4], hc[4], dh[4];
-      chunk(c, a, hc, dh);
-      dp_of(a, hc, dh);
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sdp += dh[f][i];
-          sda += dh[f][i] * a[f][i];
-        }
-    }
+      for (int i = 0; i < 4; ++i) {
+        const float f = KIND == TS_FEAT_RELU2 ? fmaxf(a[fb][i] * r2 - tau, 0.f) : h_of(a[fb][i], r2);
+        const float dp = (dh[fb][i] - sdh) * scale * f;
+        dh[fb][i] = dp;
+        sdp += dp;
+        sda += dp * a[fb][i];
+      }
     sdp = sum_g(sdp);
     sda = sum_g(sda);
     if (g == 0 && valid && p.dtau.ptr) *rows_of<float>(p.dtau, b, h).at(t) = -sdp;
     const float c3 = rinv * rinv * rinv * sda * p.inv_m;
-    // pass 3: da = rinv dp - c3 a per chunk -> dxn^T += W1^T da^T; da and h out
+    // da = rinv dp - c3 a; dxn^T = W1^T da^T; da and h out
     floatx4 dxn[D / 16];
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) dxn[db] = floatx4{0.f, 0.f, 0.f, 0.f};
-    E* da_out = valid && p.da.ptr ? rows_of<E>(p.da, b, h).at(t) : nullptr;
-    E* h_out = valid && p.h.ptr ? rows_of<E>(p.h, b, h).at(t) : nullptr;
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      floatx4 a[4], hc[4], da[4];
-      chunk(c, a, hc, da);
-      dp_of(a, hc, da);
+    E* da_out = valid && p.da.ptr ? rows_of<E>(p.da, b, h).at(t) + 4 * g : nullptr;
+    E* h_out = valid && p.h.ptr ? rows_of<E>(p.h, b, h).at(t) + 4 * g : nullptr;
+    float r3 = rinv;
+    asm volatile("" : "+v"(r3));
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+    for (int j = 0; j < MB / 2; ++j) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) da[f][i] = rinv * da[f][i] - c3 * a[f][i];
+      for (int f = 2 * j; f < 2 * j + 2; ++f) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dh[f][i] = rinv * dh[f][i] - c3 * a[f][i];
+        if (da_out) {
+          float v[4] = {dh[f][0], dh[f][1], dh[f][2], dh[f][3]};
+          st4f<E>(da_out + f * 16, v);
+        }
+        if (h_out) {
+          float v[4] = {h_of(a[f][0], r3), h_of(a[f][1], r3), h_of(a[f][2], r3), h_of(a[f][3], r3)};
+          st4f<E>(h_out + f * 16, v);
+        }
+      }
+      const auto fa = IO::from_acc(dh[2 * j], dh[2 * j + 1]);
 #pragma unroll
       for (int db = 0; db < D / 16; ++db)
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-          dxn[db] = mma32(TF::get(w1s + c * 64 * L.xp, L.xp, db * 16, jj, lane),
-                          IO::from_acc(da[2 * jj], da[2 * jj + 1]), dxn[db]);
-      if (da_out) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          float v[4] = {da[f][0], da[f][1], da[f][2], da[f][3]};
-          st4f<E>(da_out + c * 64 + f * 16 + 4 * g, v);
-        }
-      }
-      if (h_out) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          float u[4] = {hc[f][0], hc[f][1], hc[f][2], hc[f][3]};
-          st4f<E>(h_out + c * 64 + f * 16 + 4 * g, u);
-        }
-      }
+        dxn[db] = mma32(TF::get(w1s, L.xp, db * 16, j, lane), fa, dxn[db]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     if (valid && p.xn.ptr) {
       E* xn_out = rows_of<E>(p.xn, b, h).at(t);
@@ -1142,19 +1084,16 @@ __global__ __launch_bounds__(256) void feature_bwd_wide_kernel(FeatP p) {
     }
     dot = sum_g(dot);  // every lane takes part in the cross-lane sum
     dot = big ? dot * inv * inv : 0.f;
-    {
-      E* orow = os + row * L.xp;
+    // dx straight from registers: four consecutive dims per lane
+    E* dxrow = valid ? rows_of<E>(p.dx, b, h).at(t) : nullptr;
 #pragma unroll
-      for (int db = 0; db < D / 16; ++db) {
-        float v[4];
+    for (int db = 0; db < D / 16; ++db) {
+      float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (dxn[db][i] - xr[db][i] * dot) * inv;
-        if (db * 16 < p.in_rot) ir.apply(v, db, p.in_rot, g, true);
-        st4f<E>(orow + db * 16 + 4 * g, v);
-      }
+      for (int i = 0; i < 4; ++i) v[i] = (dxn[db][i] - xr[db][i] * dot) * inv;
+      if (db * 16 < p.in_rot) ir.apply(v, db, p.in_rot, g, true);
+      if (valid) st4f<E>(dxrow + db * 16 + 4 * g, v);
     }
-    __syncthreads();  // dx rows of all four waves complete
-    write_rows<E>(os, L.xp, rows_of<E>(p.dx, b, h), t0, p.T, D, tid);
   }
 }
 
@@ -1311,7 +1250,8 @@ size_t lds_bytes(int es, int d, int m, bool fwd, bool resid, bool wgrad) {
 
 // Launch plan of one call: fused weight gradients when a kernel exists for
 // the shape and its tiles fit in LDS.  Forward: enough 64-token groups per
-// workgroup to leave about four resident workgroups per CU.  Backward: the
+// workgroup to leave about four resident workgroups per CU.  Backward, and
+// the wide forward (up to 105 KB of weights to stage per workgroup): the
 // groups of each (batch, head) split over as many workgroups as the device
 // holds at once (the occupancy calculator's count for the kernel), so that
 // one wave of workgroups covers the call.
@@ -1324,10 +1264,10 @@ int plan_feature(const ts_feature_desc* d, bool fwd, bool resid, bool want_wgrad
   if (P->lds > (size_t)ts::kLdsMax) return fail(TS_ERR_NOT_IMPLEMENTED, "feature: tiles need %zu bytes of LDS", P->lds);
   const int tiles = (d->T + ts::TT - 1) / ts::TT;
   int groups = 1;
-  if (fwd) {
+  if (fwd && !is_wide(d)) {
     while (groups < 16 && (long)((tiles + 2 * groups - 1) / (2 * groups)) * d->H * d->B >= 1024) groups *= 2;
   } else {
-    long slots = ts::resident_workgroups((const void*)pick(d, false, P->wgrad, resid), (int)P->lds);
+    long slots = ts::resident_workgroups((const void*)pick(d, fwd, P->wgrad, resid), (int)P->lds);
     if (slots <= 0) slots = 512;  // two per CU on 256 CUs
     const long per_bh = slots / ((long)d->H * d->B) > 1 ? slots / ((long)d->H * d->B) : 1;
     const long g = (tiles + per_bh - 1) / per_bh;
