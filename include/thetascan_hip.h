@@ -1015,6 +1015,14 @@ int ts_rownorm_fwd(const ts_rownorm_desc* desc, ts_strided x, const float* cos, 
 int ts_rownorm_bwd(const ts_rownorm_desc* desc, ts_strided x, ts_strided dy, const float* cos, const float* sin,
                    const float* gain, const float* rstd, void* dx, float* dg_row, hipStream_t stream);
 
+/* The same with the outputs as [B,H,T,W] views of any 16-byte aligned row
+ * strides (the calls above write contiguous ones). */
+int ts_rownorm_fwd_to(const ts_rownorm_desc* desc, ts_strided x, const float* cos, const float* sin,
+                      const float* gain, ts_strided y, float* rstd, hipStream_t stream);
+
+int ts_rownorm_bwd_to(const ts_rownorm_desc* desc, ts_strided x, ts_strided dy, const float* cos, const float* sin,
+                      const float* gain, const float* rstd, ts_strided dx, float* dg_row, hipStream_t stream);
+
 /* ------------------------------------------------ host LM row glue */
 
 /* Contiguous [rows, W] tensors of ts_dtype `dtype` (W a multiple of 8, every
@@ -1032,6 +1040,12 @@ typedef struct ts_rows_desc {
  * training script, which this build does not have). */
 int ts_scale_add_fwd(const ts_rows_desc* desc, const void* x, const void* u, const void* a, const void* b,
                      void* y, hipStream_t stream);
+
+/* ts_scale_add_fwd and the RMS norm of its rows in one pass: y as above,
+ * n = y r and r = (mean(y^2) + eps)^-1/2 per row (rstd, fp32 [rows]) from the
+ * stored (rounded) y, as ts_rownorm_fwd forms them.  W = 8, 16, 32, ... 512. */
+int ts_scale_add_norm_fwd(const ts_rows_desc* desc, const void* x, const void* u, const void* a, const void* b,
+                          float eps, void* y, void* n, float* rstd, hipStream_t stream);
 
 /* Number P of fp32 column-sum partials [P][W] that ts_scale_add_bwd writes
  * (W at most 2048). */

@@ -156,3 +156,34 @@ def test_softcap_cross_entropy_flags_targets_out_of_range(cuda):
                                             reduction="none")
     assert torch.allclose(loss[[0, 2]].double(), ref[[0, 2]], rtol=1e-5)
     assert rowglue.xent_supported(z, target)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(3, 77, 512), (1, 1, 8), (2, 5, 64), (1, 33, 256)])
+def test_scale_add_norm_equals_the_two_launches(cuda, dtype, shape):
+    """y and its RMS norm, and every gradient (through both outputs, and
+    through either alone), bit for bit as scale_add followed by rms_rows."""
+    from thetascan_amd._core.ops import rowglue, rownorm
+
+    g = torch.Generator().manual_seed(shape[1])
+    W = shape[-1]
+    x, u, gy, gn = (torch.randn(shape, generator=g).to(cuda, dtype) for _ in range(4))
+    a, b = ((torch.randn(W, generator=g) + 1).to(cuda, dtype) for _ in range(2))
+    for fa, fb in ((a, b), (None, b)):
+        for use in ((True, True), (True, False), (False, True)):
+            res = []
+            for fused in (True, False):
+                leaves = [None if t is None else t.clone().requires_grad_(True) for t in (x, u, fa, fb)]
+                if fused:
+                    assert rowglue.add_norm_supported(*leaves)
+                    y, n = rowglue.scale_add_norm(*leaves)
+                else:
+                    y = rowglue.scale_add(*leaves)
+                    n = rownorm.rms_rows(y.unsqueeze(1)).squeeze(1)
+                outs = [(t, d) for t, d, w in zip((y, n), (gy, gn), use) if w]
+                torch.autograd.backward([t for t, _ in outs], [d for _, d in outs])
+                res.append([y, n] + [t.grad for t in leaves if t is not None])
+            torch.cuda.synchronize()
+            assert all(torch.equal(p, q) for p, q in zip(*res)), (fa is None, use)
+    z = torch.zeros(2, 24, device=cuda, dtype=dtype)  # no power of two of eight-column groups
+    assert rowglue.supported(z, z) and not rowglue.add_norm_supported(z, z, None, None)

@@ -119,3 +119,24 @@ def test_hybrid_lm_uses_the_row_kernel(cuda):
         y = attn(lm._rms(x))
         ref = attn.proj(o.transpose(1, 2).reshape(B, T, D))
     assert rel_err(y.float(), ref.float()) < 5e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_keep_their_memory_order(cuda, dtype):
+    """Outputs and gradients of a projection's heads are token-major like
+    their input, and equal the contiguous rows' bit for bit."""
+    from thetascan_amd._core.ops import rownorm
+
+    B, H, T, W = 2, 4, 37, 64
+    base = torch.randn(B, T, H, W, generator=torch.Generator().manual_seed(3)).to(cuda, dtype)
+    dy = torch.randn(B, H, T, W, generator=torch.Generator().manual_seed(4)).to(cuda, dtype)
+    ang = torch.rand(T, W // 2, generator=torch.Generator().manual_seed(5)).to(cuda)
+    got = []
+    for x in (base.transpose(1, 2), base.transpose(1, 2).contiguous()):
+        x = x.detach().requires_grad_(True)
+        y = rownorm.rms_rows(x, ang.cos(), ang.sin())
+        (dx,) = torch.autograd.grad(y, x, dy)
+        got.append((y, dx))
+    torch.cuda.synchronize()
+    assert got[0][0].transpose(1, 2).is_contiguous() and got[1][0].is_contiguous()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

@@ -17,6 +17,7 @@ import ctypes
 import torch
 
 from ... import _lib
+from . import rownorm
 from .dispatch import HipOp
 from .linear import slot_sum
 
@@ -125,6 +126,78 @@ def scale_add(x: torch.Tensor, u: torch.Tensor, a: torch.Tensor | None = None,
         return _scale_add_op(x, u, a, b)
     ax = x if a is None else a.to(x.dtype) * x
     return ax + (u if b is None else b.to(u.dtype) * u)
+
+
+# ---------------------------------------------------------------- scale-add and norm
+
+def _add_norm_forward(x: torch.Tensor, u: torch.Tensor, a: torch.Tensor | None, b: torch.Tensor | None,
+                      eps: float) -> list[torch.Tensor]:
+    lib = _lib.load()
+    y, n = torch.empty_like(x), torch.empty_like(x)
+    rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
+    fa, fb = _factor(a, x), _factor(b, x)
+    with _lib.timed("ts_scale_add_norm_fwd", lambda: _lib.nbytes(x, u, y, n, rstd)):
+        status = lib.ts_scale_add_norm_fwd(ctypes.byref(_desc(x)), x.data_ptr(), u.data_ptr(), _lib.ptr(fa),
+                                           _lib.ptr(fb), eps, y.data_ptr(), n.data_ptr(), rstd.data_ptr(),
+                                           _lib.stream_handle(x.device))
+    _lib.check(status, "ts_scale_add_norm_fwd")
+    return [y, n, rstd]
+
+
+def _add_norm_fake(x, u, a, b, eps):
+    return [torch.empty_like(x), torch.empty_like(x), x.new_empty(x.shape[:-1], dtype=torch.float32)]
+
+
+def _add_norm_backward_impl(gy: torch.Tensor | None, gn: torch.Tensor | None, x: torch.Tensor, u: torch.Tensor,
+                            a: torch.Tensor | None, b: torch.Tensor | None, y: torch.Tensor, rstd: torch.Tensor,
+                            eps: float, need: list[bool]) -> list[torch.Tensor]:
+    g = gy
+    if gn is not None:
+        rows = (1, 1, -1, y.shape[-1])
+        d = rownorm._backward_impl(gn.reshape(rows), y.view(rows), None, None, None, rstd.view(rows[:3]), False, eps,
+                                   False)[0].view(y.shape)
+        g = d if gy is None else gy + d
+    return _scale_add_backward_impl(g, x, u, a, b, need)
+
+
+def _add_norm_backward_fake(gy, gn, x, u, a, b, y, rstd, eps, need):
+    return _scale_add_backward_fake(gy, x, u, a, b, need)
+
+
+def _add_norm_setup(ctx, inputs, output):
+    x, u, a, b, eps = inputs
+    ctx.eps = eps
+    ctx.need = [x.requires_grad, u.requires_grad, a is not None and a.requires_grad,
+                b is not None and b.requires_grad]
+    ctx.save_for_backward(x, u, a, b, output[0], output[2])
+
+
+def _add_norm_backward(ctx, grads, bwd):
+    x, u, a, b, y, rstd = ctx.saved_tensors
+    if grads[0] is None and grads[1] is None:
+        return None, None, None, None, None
+    dx, du, da, db = bwd(grads[0], grads[1], x, u, a, b, y, rstd, ctx.eps, ctx.need)
+    return *(t if w else None for t, w in zip((dx, du, da, db), ctx.need)), None
+
+
+_add_norm_op = HipOp("scale_add_norm", forward=_add_norm_forward, forward_fake=_add_norm_fake,
+                     backward_impl=_add_norm_backward_impl, backward_fake=_add_norm_backward_fake,
+                     setup=_add_norm_setup, backward=_add_norm_backward)
+
+
+def add_norm_supported(x: torch.Tensor, u: torch.Tensor, a: torch.Tensor | None, b: torch.Tensor | None) -> bool:
+    """Whether :func:`scale_add_norm` takes these tensors (a host query)."""
+    W = x.shape[-1]
+    return supported(x, u) and W in rownorm.WIDTHS and all(f is None or (f.shape == (W,) and f.is_cuda)
+                                                           for f in (a, b))
+
+
+def scale_add_norm(x: torch.Tensor, u: torch.Tensor, a: torch.Tensor | None = None,
+                   b: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """:func:`scale_add` and the RMS norm of its rows (F.rms_norm's eps), one
+    HIP launch forward: bit for bit what the two launches give."""
+    y, n, _ = _add_norm_op(x, u, a, b, float(torch.finfo(torch.float32).eps))
+    return y, n
 
 
 # ---------------------------------------------------------------- relu^2

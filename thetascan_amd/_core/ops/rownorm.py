@@ -33,6 +33,16 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
     return x if ok else x.contiguous()
 
 
+def _like(x: torch.Tensor) -> torch.Tensor:
+    """An output for x's rows in x's own order: token-major memory for the
+    heads of a projection, so that what follows reads or reshapes it without
+    a copy; contiguous otherwise."""
+    B, H, T, W = x.shape
+    if H > 1 and T > 1 and x.stride(1) < x.stride(2):
+        return x.new_empty(B, T, H, W).transpose(1, 2)
+    return x.new_empty(B, H, T, W)
+
+
 def _f32(t: torch.Tensor | None) -> torch.Tensor | None:
     return None if t is None else t.detach().to(torch.float32).contiguous()
 
@@ -43,18 +53,18 @@ def _forward(x: torch.Tensor, cos: torch.Tensor | None, sin: torch.Tensor | None
     x4 = _rows(x)
     B, H, T, W = x4.shape
     c, s, g = _f32(cos), _f32(sin), _f32(gain)
-    y = torch.empty(B, H, T, W, dtype=x.dtype, device=x.device)
+    y = _like(x)
     rstd = torch.empty(B, H, T, dtype=torch.float32, device=x.device)
     desc = _desc(x4, rope, eps)
     with _lib.timed("ts_rownorm_fwd", lambda: _lib.nbytes(x4, y, rstd)):
-        status = lib.ts_rownorm_fwd(ctypes.byref(desc), _lib.strided(x4), _lib.ptr(c), _lib.ptr(s), _lib.ptr(g),
-                                    y.data_ptr(), rstd.data_ptr(), _lib.stream_handle(x.device))
+        status = lib.ts_rownorm_fwd_to(ctypes.byref(desc), _lib.strided(x4), _lib.ptr(c), _lib.ptr(s), _lib.ptr(g),
+                                       _lib.strided(y), rstd.data_ptr(), _lib.stream_handle(x.device))
     _lib.check(status, "ts_rownorm_fwd")
     return [y, rstd]
 
 
 def _forward_fake(x, cos, sin, gain, rope, eps):
-    return [x.new_empty(x.shape), x.new_empty(x.shape[:3], dtype=torch.float32)]
+    return [_like(x), x.new_empty(x.shape[:3], dtype=torch.float32)]
 
 
 def _backward_impl(dy: torch.Tensor, x: torch.Tensor, cos: torch.Tensor | None, sin: torch.Tensor | None,
@@ -64,20 +74,20 @@ def _backward_impl(dy: torch.Tensor, x: torch.Tensor, cos: torch.Tensor | None, 
     x4 = _rows(x)
     d4 = _rows(dy.to(x.dtype))
     c, s, g = _f32(cos), _f32(sin), _f32(gain)
-    dx = torch.empty(x4.shape, dtype=x.dtype, device=x.device)
+    dx = _like(x)
     dg_row = torch.empty(x4.shape[:3], dtype=torch.float32, device=x.device) if need_gain else None
     desc = _desc(x4, rope, eps)
     with _lib.timed("ts_rownorm_bwd", lambda: _lib.nbytes(x4, d4, rstd, dx)):
-        status = lib.ts_rownorm_bwd(ctypes.byref(desc), _lib.strided(x4), _lib.strided(d4), _lib.ptr(c),
-                                    _lib.ptr(s), _lib.ptr(g), rstd.data_ptr(), dx.data_ptr(), _lib.ptr(dg_row),
-                                    _lib.stream_handle(x.device))
+        status = lib.ts_rownorm_bwd_to(ctypes.byref(desc), _lib.strided(x4), _lib.strided(d4), _lib.ptr(c),
+                                       _lib.ptr(s), _lib.ptr(g), rstd.data_ptr(), _lib.strided(dx), _lib.ptr(dg_row),
+                                       _lib.stream_handle(x.device))
     _lib.check(status, "ts_rownorm_bwd")
     dgain = dg_row.sum(dim=(0, 2)).to(gain.dtype) if need_gain else x.new_empty(0)
     return [dx, dgain]
 
 
 def _backward_fake(dy, x, cos, sin, gain, rstd, rope, eps, need_gain):
-    return [x.new_empty(x.shape), gain.new_empty(gain.shape) if need_gain else x.new_empty(0)]
+    return [_like(x), gain.new_empty(gain.shape) if need_gain else x.new_empty(0)]
 
 
 def _setup(ctx, inputs, output):

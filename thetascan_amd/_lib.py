@@ -666,6 +666,11 @@ def load() -> ctypes.CDLL:
         lib.ts_rownorm_bwd.argtypes = [P(RowNormDesc), Strided, Strided, ctypes.c_void_p, ctypes.c_void_p,
                                        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                        ctypes.c_void_p]
+        lib.ts_rownorm_fwd_to.argtypes = [P(RowNormDesc), Strided, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                          Strided, ctypes.c_void_p, ctypes.c_void_p]
+        lib.ts_rownorm_bwd_to.argtypes = [P(RowNormDesc), Strided, Strided, ctypes.c_void_p, ctypes.c_void_p,
+                                          ctypes.c_void_p, ctypes.c_void_p, Strided, ctypes.c_void_p,
+                                          ctypes.c_void_p]
         lib.ts_gn_act_fwd.argtypes = [P(GnActDesc), Strided, Strided, ctypes.c_void_p, Strided, Strided, Strided,
                                       ctypes.c_void_p]
         lib.ts_gn_act_bwd.argtypes = [P(GnActDesc), Strided, Strided, ctypes.c_void_p] + [Strided] * 6 + [
@@ -680,6 +685,8 @@ def load() -> ctypes.CDLL:
                                           ctypes.c_size_t, ctypes.c_void_p]
         lib.ts_stack_heads.argtypes = [P(StackDesc), P(Strided), ctypes.c_void_p, ctypes.c_void_p]
         lib.ts_scale_add_fwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 6
+        lib.ts_scale_add_norm_fwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 4 + [ctypes.c_float] + [
+            ctypes.c_void_p] * 4
         lib.ts_scale_add_parts.argtypes = [P(RowsDesc), P(ctypes.c_int32)]
         lib.ts_scale_add_bwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 10
         lib.ts_relu2_fwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 3

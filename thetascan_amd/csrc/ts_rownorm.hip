@@ -31,8 +31,7 @@ struct RowNormP {
   int B, H, T, W, rope, lanes;  // lanes per row = W / 8
   float eps;
   ts_strided x, dy;             // [B,H,T,W] views (feature axis contiguous)
-  void* y;                      // out: contiguous [B,H,T,W]
-  void* dx;                     // out: contiguous [B,H,T,W]
+  ts_strided y, dx;             // out: [B,H,T,W] views (feature axis contiguous)
   float* rstd;                  // [B*H*T]
   float* dg_row;                // [B*H*T] or null
   const float* cos;             // [T, W/2]
@@ -143,7 +142,7 @@ __global__ __launch_bounds__(256) void rownorm_fwd_kernel(RowNormP p) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] *= g;
   if (w.valid) {
-    rn_st8<E>((E*)p.y + w.r * p.W + w.c0, o);
+    rn_st8<E>((E*)p.y.ptr + w.b * p.y.sb + w.h * p.y.sh + (int64_t)w.t * p.y.st + w.c0, o);
     if (w.c0 == 0) p.rstd[w.r] = r;
   }
 }
@@ -194,7 +193,7 @@ __global__ __launch_bounds__(256) void rownorm_bwd_kernel(RowNormP p) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = r * dn[e] - c3 * v[e];
   if (w.valid) {
-    rn_st8<E>((E*)p.dx + w.r * p.W + w.c0, o);
+    rn_st8<E>((E*)p.dx.ptr + w.b * p.dx.sb + w.h * p.dx.sh + (int64_t)w.t * p.dx.st + w.c0, o);
     if (p.dg_row && w.c0 == 0) p.dg_row[w.r] = dg;
   }
 }
@@ -237,7 +236,16 @@ int rn_launch(const ts::RowNormP& p, hipStream_t stream) {
   return TS_OK;
 }
 
-bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
+// Rows of 16-byte alignment at every stride.
+bool aligned_rows(const ts_strided& s, int dtype) {
+  const int vec = dtype == TS_BF16 ? 8 : 4;
+  return s.ptr && ((uintptr_t)s.ptr & 15u) == 0 && s.sb % vec == 0 && s.sh % vec == 0 && s.st % vec == 0;
+}
+
+ts_strided contiguous_rows(const ts_rownorm_desc* d, void* ptr) {
+  if (!d) return ts_strided{ptr, 0, 0, 0};
+  return ts_strided{ptr, (int64_t)d->H * d->T * d->W, (int64_t)d->T * d->W, d->W};
+}
 
 }  // namespace
 
@@ -245,10 +253,20 @@ extern "C" {
 
 int ts_rownorm_fwd(const ts_rownorm_desc* d, ts_strided x, const float* cos, const float* sin, const float* gain,
                    void* y, float* rstd, hipStream_t stream) {
+  return ts_rownorm_fwd_to(d, x, cos, sin, gain, contiguous_rows(d, y), rstd, stream);
+}
+
+int ts_rownorm_bwd(const ts_rownorm_desc* d, ts_strided x, ts_strided dy, const float* cos, const float* sin,
+                   const float* gain, const float* rstd, void* dx, float* dg_row, hipStream_t stream) {
+  return ts_rownorm_bwd_to(d, x, dy, cos, sin, gain, rstd, contiguous_rows(d, dx), dg_row, stream);
+}
+
+int ts_rownorm_fwd_to(const ts_rownorm_desc* d, ts_strided x, const float* cos, const float* sin, const float* gain,
+                      ts_strided y, float* rstd, hipStream_t stream) {
   ts::RowNormP p;
   int rc = rn_prepare(d, x, cos, sin, &p);
   if (rc) return rc;
-  if (!y || !aligned16(y) || !rstd) return fail(TS_ERR_VALUE, "row norm: missing or unaligned output");
+  if (!aligned_rows(y, d->dtype) || !rstd) return fail(TS_ERR_VALUE, "row norm: missing or unaligned output");
   if (d->T == 0) return TS_OK;
   p.y = y;
   p.rstd = rstd;
@@ -256,15 +274,13 @@ int ts_rownorm_fwd(const ts_rownorm_desc* d, ts_strided x, const float* cos, con
   return d->dtype == TS_BF16 ? rn_launch<ts::bf16, true>(p, stream) : rn_launch<float, true>(p, stream);
 }
 
-int ts_rownorm_bwd(const ts_rownorm_desc* d, ts_strided x, ts_strided dy, const float* cos, const float* sin,
-                   const float* gain, const float* rstd, void* dx, float* dg_row, hipStream_t stream) {
+int ts_rownorm_bwd_to(const ts_rownorm_desc* d, ts_strided x, ts_strided dy, const float* cos, const float* sin,
+                      const float* gain, const float* rstd, ts_strided dx, float* dg_row, hipStream_t stream) {
   ts::RowNormP p;
   int rc = rn_prepare(d, x, cos, sin, &p);
   if (rc) return rc;
-  const int es = d->dtype == TS_BF16 ? 2 : 4;
-  if (!dy.ptr || !aligned16(dy.ptr) || (dy.sb * es) % 16 || (dy.sh * es) % 16 || (dy.st * es) % 16)
-    return fail(TS_ERR_VALUE, "row norm: dy rows must be 16-byte aligned");
-  if (!dx || !aligned16(dx) || !rstd) return fail(TS_ERR_VALUE, "row norm: missing or unaligned dx / rstd");
+  if (!aligned_rows(dy, d->dtype)) return fail(TS_ERR_VALUE, "row norm: dy rows must be 16-byte aligned");
+  if (!aligned_rows(dx, d->dtype) || !rstd) return fail(TS_ERR_VALUE, "row norm: missing or unaligned dx / rstd");
   if (d->T == 0) return TS_OK;
   p.dy = dy;
   p.dx = dx;

@@ -64,6 +64,15 @@ def _rms(x: torch.Tensor) -> torch.Tensor:
     return F.rms_norm(x, (x.shape[-1],))
 
 
+def _add_rms(x: torch.Tensor, u: torch.Tensor, a: torch.Tensor | None,
+             b: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """``y = a x + b u`` and its RMS norm: one row-glue launch on the GPU."""
+    if x.ndim == 3 and rowglue.add_norm_supported(x, u, a, b):
+        return rowglue.scale_add_norm(x, u, a, b)
+    y = rowglue.scale_add(x, u, a, b)
+    return y, _rms(y)
+
+
 class Rotary(nn.Module):
     def __init__(self, dim: int, base: float = ROPE_BASE):
         super().__init__()
@@ -108,7 +117,7 @@ class CausalSelfAttention(nn.Module):
         else:
             q, k = _rotate(_rms(q), cos, sin), _rotate(_rms(k), cos, sin)
             q = q * self.q_gain.to(q.dtype)[None, :, None, None]
-        y = attention(q.contiguous(), k.contiguous(), v.contiguous())
+        y = attention(q, k, v)
         return self.proj(y.transpose(1, 2).reshape(B, T, D))
 
 
@@ -118,12 +127,15 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor
     memory-efficient) kernels for bf16 on the GPU, which read the grouped
     heads in place, the math form in fp32 elsewhere (the bf16 math form
     multiplies by a transposed operand)."""
+    # (the fused kernels take the projections' token-major heads in place and
+    # return theirs in the query's order, which reshapes to rows without a copy)
     grouped = k.shape[1] != q.shape[1]
     if q.is_cuda and q.dtype == torch.bfloat16:
         from torch.nn.attention import SDPBackend, sdpa_kernel
 
         with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):
             return F.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=grouped)
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     if grouped:
         rep = q.shape[1] // k.shape[1]
         k, v = k.repeat_interleave(rep, dim=1), v.repeat_interleave(rep, dim=1)
@@ -158,10 +170,10 @@ class Block(nn.Module):
 
     def forward(self, x: torch.Tensor, x0: torch.Tensor) -> torch.Tensor:
         # mix0 x + mix1 x0, then x + scale * f(x) per sublayer: one row-glue
-        # launch each on the GPU
-        x = rowglue.scale_add(x, x0, self.resid_mix[0], self.resid_mix[1])
-        x = rowglue.scale_add(x, self.attn(_rms(x)), None, self.attn_scale)
-        return rowglue.scale_add(x, self.mlp(_rms(x)), None, self.mlp_scale)
+        # launch each on the GPU, with the norm that the sublayer reads
+        x, n = _add_rms(x, x0, self.resid_mix[0], self.resid_mix[1])
+        x, n = _add_rms(x, self.attn(n), None, self.attn_scale)
+        return rowglue.scale_add(x, self.mlp(n), None, self.mlp_scale)
 
 
 class HybridLM(nn.Module):
