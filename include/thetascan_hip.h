@@ -1023,6 +1023,19 @@ int ts_rownorm_fwd_to(const ts_rownorm_desc* desc, ts_strided x, const float* co
 int ts_rownorm_bwd_to(const ts_rownorm_desc* desc, ts_strided x, ts_strided dy, const float* cos, const float* sin,
                       const float* gain, const float* rstd, ts_strided dx, float* dg_row, hipStream_t stream);
 
+/* Causal softmax attention, forward: out[b,h,t] = sum_{s <= t}
+ * softmax_s(scale q_t . k_s) v_s for bf16 q, out [B,H,T,64] and k, v
+ * [B,Hkv,T,64] views (Hkv divides H: head h reads head h / (H / Hkv)) with
+ * 16-byte aligned rows.  fp32 scores and sums, one rounding of the output. */
+typedef struct ts_attention_desc {
+  int32_t B, H, Hkv, T, d;
+  int32_t dtype;
+  float scale;
+} ts_attention_desc;
+
+int ts_causal_attention_fwd(const ts_attention_desc* desc, ts_strided q, ts_strided k, ts_strided v, ts_strided out,
+                            hipStream_t stream);
+
 /* ------------------------------------------------ host LM row glue */
 
 /* Contiguous [rows, W] tensors of ts_dtype `dtype` (W a multiple of 8, every

@@ -26,7 +26,7 @@ SOURCES = ("ts_scan.hip", "ts_scan_wide.hip", "ts_scan_views.hip", "ts_features.
            "ts_gn.hip", "ts_gn_relu2.hip", "ts_gn_tanh.hip", "ts_gn_silu.hip", "ts_memory.hip", "ts_retention.hip",
            "ts_contract.hip", "ts_readout.hip", "ts_anchor.hip", "ts_kmap.hip", "ts_gnact.hip", "ts_absmass.hip",
            "ts_rownorm.hip", "ts_rowglue.hip", "ts_bankread.hip",
-           "ts_views_bwd.hip", "ts_step.hip")
+           "ts_views_bwd.hip", "ts_step.hip", "ts_attention.hip")
 
 HIPCC_FLAGS = (
     f"--offload-arch={ARCH}",

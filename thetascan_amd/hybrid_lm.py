@@ -28,7 +28,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from ._core.ops import rowglue, rownorm
+from ._core.ops import attention as hip_attention, rowglue, rownorm
 from .api import ThetaScan
 from .config import ThetaScanConfig
 
@@ -123,12 +123,15 @@ class CausalSelfAttention(nn.Module):
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
     """Causal softmax attention of q [B,H,T,d] against k, v [B,Hkv,T,d]
-    (Hkv divides H: grouped key/value heads): the fused (flash /
+    (Hkv divides H: grouped key/value heads): the HIP kernel for bf16 heads
+    of 64 where nothing is recorded for a backward, the fused (flash /
     memory-efficient) kernels for bf16 on the GPU, which read the grouped
     heads in place, the math form in fp32 elsewhere (the bf16 math form
     multiplies by a transposed operand)."""
     # (the fused kernels take the projections' token-major heads in place and
     # return theirs in the query's order, which reshapes to rows without a copy)
+    if hip_attention.supported(q, k, v):
+        return hip_attention.causal_attention(q, k, v)
     grouped = k.shape[1] != q.shape[1]
     if q.is_cuda and q.dtype == torch.bfloat16:
         from torch.nn.attention import SDPBackend, sdpa_kernel
