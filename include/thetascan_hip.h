@@ -1023,6 +1023,11 @@ int ts_rownorm_fwd_to(const ts_rownorm_desc* desc, ts_strided x, const float* co
 int ts_rownorm_bwd_to(const ts_rownorm_desc* desc, ts_strided x, ts_strided dy, const float* cos, const float* sin,
                       const float* gain, const float* rstd, ts_strided dx, float* dg_row, hipStream_t stream);
 
+/* cos and sin [T, half] (fp32) of t * inv_freq[j] for t in [0, T), the
+ * frequencies [half] of ts_dtype `dtype`: the phase tables of the turn. */
+int ts_rotary_tables(const void* inv_freq, int32_t dtype, int32_t T, int32_t half, float* cos, float* sin,
+                     hipStream_t stream);
+
 /* Causal softmax attention, forward: out[b,h,t] = sum_{s <= t}
  * softmax_s(scale q_t . k_s) v_s for bf16 q, out [B,H,T,64] and k, v
  * [B,Hkv,T,64] views (Hkv divides H: head h reads head h / (H / Hkv)) with

@@ -140,3 +140,17 @@ def test_rows_keep_their_memory_order(cuda, dtype):
     torch.cuda.synchronize()
     assert got[0][0].transpose(1, 2).is_contiguous() and got[1][0].is_contiguous()
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,half", [(1, 32), (129, 32), (1025, 7), (70001, 32)])
+def test_rotary_tables_equal_the_torch_expression(cuda, dtype, T, half):
+    """Within one fp32 rounding (2^-23) of torch's cos and sin of the same
+    fp32 product, at small and large angles."""
+    from thetascan_amd._core.ops import rownorm
+
+    inv = (1.0 / (10_000.0 ** (torch.arange(0, 2 * half, 2, dtype=torch.float32) / (2 * half)))).to(cuda, dtype)
+    f = torch.outer(torch.arange(T, device=cuda, dtype=torch.float32), inv)
+    cos, sin = rownorm.rotary_tables(inv, T)
+    assert cos.dtype == torch.float32 and cos.shape == f.shape
+    assert float((cos - f.cos()).abs().max()) <= 2.0 ** -23 and float((sin - f.sin()).abs().max()) <= 2.0 ** -23

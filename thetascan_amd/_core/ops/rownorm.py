@@ -130,3 +130,22 @@ def rms_rows(x: torch.Tensor, cos: torch.Tensor | None = None, sin: torch.Tensor
     if eps is None:
         eps = float(torch.finfo(torch.float32).eps)
     return _rownorm_op(x, cos, sin, gain, rope, float(eps))[0]
+
+
+def rotary_tables(inv_freq: torch.Tensor, T: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """cos and sin [T, W/2] (fp32) of the positions 0 .. T-1 times the
+    frequencies ``inv_freq`` [W/2]: one launch, the torch expression where
+    that does not apply (host tensors, tracing, other dtypes, gradients)."""
+    if (not inv_freq.is_cuda or torch.compiler.is_compiling() or inv_freq.dtype not in (torch.bfloat16, torch.float32)
+            or inv_freq.requires_grad or not inv_freq.is_contiguous()):
+        f = torch.outer(torch.arange(T, device=inv_freq.device, dtype=torch.float32), inv_freq)
+        return f.cos(), f.sin()
+    lib = _lib.load()
+    half = inv_freq.numel()
+    cos = torch.empty(T, half, dtype=torch.float32, device=inv_freq.device)
+    sin = torch.empty_like(cos)
+    with _lib.timed("ts_rotary_tables", lambda: _lib.nbytes(inv_freq, cos, sin)):
+        status = lib.ts_rotary_tables(inv_freq.data_ptr(), _lib.dtype_code(inv_freq.dtype), T, half, cos.data_ptr(),
+                                      sin.data_ptr(), _lib.stream_handle(inv_freq.device))
+    _lib.check(status, "ts_rotary_tables")
+    return cos, sin

@@ -688,6 +688,7 @@ def load() -> ctypes.CDLL:
         lib.ts_retention_grad.argtypes = [P(RetentionDesc), P(RetentionIO), ctypes.c_void_p, ctypes.c_void_p,
                                           ctypes.c_size_t, ctypes.c_void_p]
         lib.ts_stack_heads.argtypes = [P(StackDesc), P(Strided), ctypes.c_void_p, ctypes.c_void_p]
+        lib.ts_rotary_tables.argtypes = [ctypes.c_void_p] + [ctypes.c_int32] * 3 + [ctypes.c_void_p] * 3
         lib.ts_causal_attention_fwd.argtypes = [P(AttentionDesc), Strided, Strided, Strided, Strided, ctypes.c_void_p]
         lib.ts_scale_add_fwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 6
         lib.ts_scale_add_norm_fwd.argtypes = [P(RowsDesc)] + [ctypes.c_void_p] * 4 + [ctypes.c_float] + [

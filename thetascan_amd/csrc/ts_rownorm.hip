@@ -198,6 +198,19 @@ __global__ __launch_bounds__(256) void rownorm_bwd_kernel(RowNormP p) {
   }
 }
 
+// cos and sin of t * inv_freq[j], one element per thread (the position times
+// the frequency in fp32, as an outer product of fp32 positions forms it).
+// Bound by its launch: one, where the tensor expressions took five a layer.
+template <typename E>
+__global__ __launch_bounds__(256) void rotary_tables_kernel(const E* inv_freq, int half, int64_t n, float* cos,
+                                                            float* sin) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const float f = (float)(i / half) * (float)inv_freq[i % half];
+  cos[i] = cosf(f);
+  sin[i] = sinf(f);
+}
+
 }  // namespace ts
 
 namespace {
@@ -259,6 +272,24 @@ int ts_rownorm_fwd(const ts_rownorm_desc* d, ts_strided x, const float* cos, con
 int ts_rownorm_bwd(const ts_rownorm_desc* d, ts_strided x, ts_strided dy, const float* cos, const float* sin,
                    const float* gain, const float* rstd, void* dx, float* dg_row, hipStream_t stream) {
   return ts_rownorm_bwd_to(d, x, dy, cos, sin, gain, rstd, contiguous_rows(d, dx), dg_row, stream);
+}
+
+int ts_rotary_tables(const void* inv_freq, int32_t dtype, int32_t T, int32_t half, float* cos, float* sin,
+                     hipStream_t stream) {
+  if (T < 0 || half < 1) return fail(TS_ERR_VALUE, "rotary tables: bad shape");
+  if (dtype != TS_BF16 && dtype != TS_F32) return fail(TS_ERR_VALUE, "rotary tables: unknown dtype");
+  if (T == 0) return TS_OK;
+  if (!inv_freq || !cos || !sin) return fail(TS_ERR_VALUE, "rotary tables: missing tensors");
+  const int64_t n = (int64_t)T * half, blocks = (n + 255) / 256;
+  if (blocks > 0x7fffffff) return fail(TS_ERR_NOT_IMPLEMENTED, "rotary tables: too many positions");
+  const dim3 grid((unsigned)blocks);
+  if (dtype == TS_BF16)
+    hipLaunchKernelGGL(ts::rotary_tables_kernel<ts::bf16>, grid, dim3(256), 0, stream, (const ts::bf16*)inv_freq, half, n, cos, sin);
+  else
+    hipLaunchKernelGGL(ts::rotary_tables_kernel<float>, grid, dim3(256), 0, stream, (const float*)inv_freq, half, n, cos, sin);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TS_ERR_RUNTIME, "rotary tables: launch failed: %s", hipGetErrorString(e));
+  return TS_OK;
 }
 
 int ts_rownorm_fwd_to(const ts_rownorm_desc* d, ts_strided x, const float* cos, const float* sin, const float* gain,

@@ -80,8 +80,7 @@ class Rotary(nn.Module):
                              persistent=False)
 
     def forward(self, T: int, device):
-        f = torch.outer(torch.arange(T, device=device, dtype=torch.float32), self.inv_freq.to(device))
-        return f.cos(), f.sin()
+        return rownorm.rotary_tables(self.inv_freq.to(device), T)
 
 
 def _rotate(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
