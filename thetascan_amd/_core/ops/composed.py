@@ -370,8 +370,9 @@ class FastNet:
 
     # ---- the network at the slow weights
 
-    def run(self, k, own=None):
-        """The blocks in sequence on keys ``k`` -> (acts, output).  ``own``:
+    def run(self, k, own=None, output=True):
+        """The blocks in sequence on keys ``k`` -> (acts, output; None without
+        ``output``: the last block's W2 product and add are not formed).  ``own``:
         the previous step's deposits; each block then adds this token's own
         write of that step (a rank-one correction per token: the second
         Gauss-Newton step linearizes at theta0 + the token's own delta)."""
@@ -385,10 +386,12 @@ class FastNet:
                 if self.gated:
                     gate_shift = dep.jac[..., self.width:] * dot
             act = self.act(l, x, main_shift, gate_shift)
+            acts.append(act)
+            if not output and l + 1 == len(self.layers):
+                return acts, None
             u = self.out(l, act.h)
             if own is not None:
                 u = u + own[l].pay * (own[l].h0 * act.h).sum(-1, keepdim=True)
-            acts.append(act)
             x = x + self._scaled(u)
         return acts, x
 
@@ -414,7 +417,9 @@ class FastNet:
             h, pay, jac = gn.write(k, v, W1, W2, Wg[..., 0] if cfg.learn_thresh else None, s=self.s,
                                    inv_depth=1.0 / cfg.depth, eps=cfg.eps, nonlin=cfg.nonlin, damping=damping(cfg))
             return [[Deposit(self.rotate(h), pay, k if cfg.fast_w1 else None, jac if cfg.fast_w1 else None)]]
-        acts, out = self.run(k)
+        # (a kernel write deposits v itself: only a solve reads the keys' output.
+        # B2 T32768, 128 features: a 54 us product and a 32 us add of 1.13 ms)
+        acts, out = self.run(k, output=cfg.write_rule != "kernel")
         if cfg.write_rule == "kernel":
             lam = self._anchor_code(v) if cfg.value_centers else v
         else:
