@@ -105,3 +105,41 @@ def test_other_continuations_keep_their_path(cuda):
     with torch.no_grad(), _lib.record_launches() as recs:
         module(x, state=module.initial_state())
     assert "ts_memory_step" not in {r[0] for r in recs}
+
+
+def _prompted(cuda, dtype, case=CASES[0], seed=3, batch=3):
+    """A mixer of ``case`` on the GPU, its state after a prompt of 20 tokens and the next 8 tokens."""
+    import thetascan_amd as ts
+
+    torch.manual_seed(seed)
+    module = ts.ThetaScan(_config(*case))
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for _, p in sorted(module.named_parameters()):
+            p.add_(torch.randn(p.shape, generator=g) * 0.05)  # (the output projection starts at zero)
+    module = module.to(cuda, dtype)
+    x = torch.randn(batch, 28, module.config.d_model, generator=g).to(cuda, dtype)
+    with torch.no_grad():
+        _, state = module(x[:, :20], state=module.initial_state())
+    return module, state, x[:, 20:].contiguous()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("change", [-32, 32])
+def test_another_input_width_is_refused(cuda, dtype, change):
+    """An input of another width than the projection's rows raises, as its
+    product always did, before any launch of the step."""
+    from thetascan_amd import _lib
+    from thetascan_amd._core.ops import step
+
+    module, state, x = _prompted(cuda, dtype)
+    D = x.shape[-1]
+    other = torch.randn(3, 1, D + change, device=cuda).to(dtype)
+    before = [c.clone() for c in state._tensors()]
+    with torch.no_grad(), _lib.record_launches() as recs:
+        with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+            module(other, state=state)
+        with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+            step._linear(other.view(3, -1), module._core.proj_qkv.weight, None)
+    assert not recs
+    assert all(torch.equal(a, b) for a, b in zip(state._tensors(), before))

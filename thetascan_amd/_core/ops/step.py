@@ -24,9 +24,11 @@ SKINNY_ROWS = 64
 
 def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
     """Whether ts_memory_step takes this continuation: few tokens, widths of
-    the kernel, and every parameter a contiguous tensor of the input's dtype."""
+    the kernel, the input as wide as the projection's rows (``params[0]``; any
+    other width is refused by the multi-view path's product), and every
+    parameter a contiguous tensor of the input's dtype."""
     return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and 1 <= x.shape[1] <= MAX_TOKENS
-            and head_dim in WIDTHS and spec.m in WIDTHS
+            and head_dim in WIDTHS and spec.m in WIDTHS and x.shape[2] == params[0].shape[1]
             and all(p is None or (p.dtype == x.dtype and p.is_contiguous() and p.data_ptr() % 16 == 0) for p in params))
 
 
@@ -36,8 +38,10 @@ def _linear(x2: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor | None) -> torc
     4.8 us each against 3.7 us for both, with no concatenated weight)."""
     n, k = x2.shape
     na, nb = wa.shape[0], 0 if wb is None else wb.shape[0]
+    # (a weight of another row length is the library product's to refuse: the
+    # kernel reads k elements of every row)
     if not (x2.dtype == torch.bfloat16 and n <= SKINNY_ROWS and k % 32 == 0 and na % 16 == 0 and nb % 16 == 0
-            and x2.data_ptr() % 16 == 0):
+            and all(w is None or w.shape[1] == k for w in (wa, wb)) and x2.data_ptr() % 16 == 0):
         parts = [F.linear(x2, w) for w in (wa, wb) if w is not None]
         return parts[0] if wb is None else torch.cat(parts, dim=1)
     y = torch.empty(n, na + nb, dtype=x2.dtype, device=x2.device)
