@@ -143,3 +143,42 @@ def test_another_input_width_is_refused(cuda, dtype, change):
             step._linear(other.view(3, -1), module._core.proj_qkv.weight, None)
     assert not recs
     assert all(torch.equal(a, b) for a, b in zip(state._tensors(), before))
+
+
+def _layouts(x):
+    """The values of x [B,T,D] in other memory orders, by name."""
+    B, T, D = x.shape
+    wide = x.new_zeros(B, T, 2 * D)
+    wide[..., ::2] = x
+    padded = x.new_zeros(B, T, D + 4)
+    padded[..., :D] = x
+    longer = x.new_zeros(B, T + 7, D)
+    longer[:, 7:] = x
+    channels = x.new_zeros(B, D, 16)
+    channels[..., 8:8 + T] = x.transpose(1, 2)
+    return {
+        "every second channel": wide[..., ::2],
+        "rows of a wider buffer": padded[..., :D],
+        "the last tokens of a longer sequence": longer[:, 7:],
+        "channel-major": channels[..., 8:8 + T].transpose(1, 2),
+        "batch innermost": x.permute(1, 2, 0).contiguous().permute(2, 0, 1),
+        "one sequence for all": x[:1].expand(B, T, D),
+    }
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_inputs_of_any_layout(cuda, dtype, tokens):
+    """An input of any strides gives what its contiguous copy gives, in the
+    output and in the carried state.  Bars: fp32 1e-5 (a product's sums in
+    another order), bf16 1e-2 (its one rounding carried to the output)."""
+    module, state, x = _prompted(cuda, dtype)
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    for name, view in _layouts(x[:, :tokens]).items():
+        same = view.clone(memory_format=torch.contiguous_format)
+        with torch.no_grad():
+            y, new = module(view, state=state)
+            want, ref = module(same, state=state)
+        assert rel_err(y, want) < tol, name
+        for a, b in zip(new._tensors(), ref._tensors()):
+            assert rel_err(a, b) < tol, name

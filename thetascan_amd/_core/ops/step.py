@@ -39,9 +39,11 @@ def _linear(x2: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor | None) -> torc
     n, k = x2.shape
     na, nb = wa.shape[0], 0 if wb is None else wb.shape[0]
     # (a weight of another row length is the library product's to refuse: the
-    # kernel reads k elements of every row)
+    # kernel reads k elements of every row; rows of other strides, which a
+    # reshape leaves as they are, are its to read)
     if not (x2.dtype == torch.bfloat16 and n <= SKINNY_ROWS and k % 32 == 0 and na % 16 == 0 and nb % 16 == 0
-            and all(w is None or w.shape[1] == k for w in (wa, wb)) and x2.data_ptr() % 16 == 0):
+            and all(w is None or w.shape[1] == k for w in (wa, wb))
+            and x2.data_ptr() % 16 == 0 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0):
         parts = [F.linear(x2, w) for w in (wa, wb) if w is not None]
         return parts[0] if wb is None else torch.cat(parts, dim=1)
     y = torch.empty(n, na + nb, dtype=x2.dtype, device=x2.device)
