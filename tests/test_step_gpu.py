@@ -182,3 +182,23 @@ def test_inputs_of_any_layout(cuda, dtype, tokens):
         assert rel_err(y, want) < tol, name
         for a, b in zip(new._tensors(), ref._tensors()):
             assert rel_err(a, b) < tol, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [1, 8])
+def test_autocast(cuda, dtype, tokens):
+    """Under autocast to bf16 an fp32 mixer's projections are bf16: its steps
+    take the multi-view path, which follows them, and match the fp32 step at
+    bf16's bar; a bf16 mixer keeps its step."""
+    from thetascan_amd import _lib
+
+    module, state, x = _prompted(cuda, dtype)
+    with torch.no_grad():
+        want, ref = module(x[:, :tokens], state=state)
+        with torch.autocast("cuda", torch.bfloat16), _lib.record_launches() as recs:
+            y, new = module(x[:, :tokens], state=state)
+    assert ("ts_memory_step" in {r[0] for r in recs}) == (dtype == torch.bfloat16)
+    assert y.dtype == torch.bfloat16
+    assert rel_err(y, want) < 2e-2
+    for a, b in zip(new._tensors(), ref._tensors()):
+        assert rel_err(a, b) < 2e-2
