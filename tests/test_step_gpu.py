@@ -202,3 +202,13 @@ def test_autocast(cuda, dtype, tokens):
     assert rel_err(y, want) < 2e-2
     for a, b in zip(new._tensors(), ref._tensors()):
         assert rel_err(a, b) < 2e-2
+
+
+def test_parameters_on_another_device_are_refused(cuda):
+    """A mixer left on the host raises on a GPU input, as its product always did."""
+    import thetascan_amd as ts
+
+    module = ts.ThetaScan(_config(*CASES[0]))
+    x = torch.randn(2, 1, module.config.d_model, device=cuda)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="same device"):
+        module(x, state=module.initial_state())

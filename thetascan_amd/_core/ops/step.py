@@ -32,12 +32,14 @@ def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
     """Whether ts_memory_step takes this continuation: few tokens, widths of
     the kernel, the input as wide as the projection's rows (``params[0]``; any
     other width is refused by the multi-view path's product), and every
-    parameter a contiguous tensor of the input's dtype, which the projections
-    keep (the kernel's rows are of one dtype: under an autocast to another the
-    multi-view path follows the projection)."""
-    return (_keeps_dtype(x) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and 1 <= x.shape[1] <= MAX_TOKENS
-            and head_dim in WIDTHS and spec.m in WIDTHS and x.shape[2] == params[0].shape[1]
-            and all(p is None or (p.dtype == x.dtype and p.is_contiguous() and p.data_ptr() % 16 == 0) for p in params))
+    parameter a contiguous tensor beside the input and of its dtype, which the
+    projections keep (the kernel's rows are of one dtype: under an autocast to
+    another the multi-view path follows the projection)."""
+    return (_keeps_dtype(x) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float32)
+            and 1 <= x.shape[1] <= MAX_TOKENS and head_dim in WIDTHS and spec.m in WIDTHS
+            and x.shape[2] == params[0].shape[1]
+            and all(p is None or (p.dtype == x.dtype and p.device == x.device and p.is_contiguous()
+                                  and p.data_ptr() % 16 == 0) for p in params))
 
 
 def _linear(x2: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor | None) -> torch.Tensor:
