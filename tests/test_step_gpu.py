@@ -212,3 +212,24 @@ def test_parameters_on_another_device_are_refused(cuda):
     x = torch.randn(2, 1, module.config.d_model, device=cuda)
     with torch.no_grad(), pytest.raises(RuntimeError, match="same device"):
         module(x, state=module.initial_state())
+
+
+def test_states_as_the_scan_takes_them(cuda):
+    """A carried state is taken in the forms the scan takes: folded batch and
+    head axes, another memory order; a captured step, which writes its state in
+    place, refuses one it could not write."""
+    import dataclasses
+
+    import thetascan_amd as ts
+
+    module, state, x = _prompted(cuda, torch.float32)
+    (block,), = state.carries
+    with torch.no_grad():
+        want, ref = module(x[:, :1], state=state)
+        turned = block.transpose(2, 3).contiguous().transpose(2, 3)
+        for other in (block.flatten(0, 1), turned):
+            y, new = module(x[:, :1], state=dataclasses.replace(state, carries=([other],)))
+            assert torch.equal(y, want)
+            assert torch.equal(new.carries[0][0], ref.carries[0][0])
+        with pytest.raises(ValueError, match="contiguous"):
+            ts.DecodeGraph(module, dataclasses.replace(state, carries=([turned],)))

@@ -75,11 +75,15 @@ def kernel_step(x: torch.Tensor, w_qkv, w_g, b_g, w1, w2, tau, w_out, spec, norm
     cols = d + int(normalize)
     init = None
     if blocks is not None:
-        if len(blocks) != 1 or tuple(blocks[0].shape) != (B, H, spec.m, cols):
+        # (as scan_launch takes a carried state)
+        if (len(blocks) != 1 or tuple(blocks[0].shape[-2:]) != (spec.m, cols)
+                or blocks[0].numel() != B * H * spec.m * cols):
             raise ValueError("streaming state does not match this scan's widths")
         init = blocks[0].detach().to(device=dev, dtype=torch.float32).contiguous()
     if blocks is not None and stream.updates_in_place():
         fin = blocks[0]
+        if fin.dtype != torch.float32 or not fin.is_contiguous() or fin.device != dev:
+            raise ValueError("a state updated in place must be a contiguous fp32 tensor beside the input")
     else:
         fin = torch.empty(B, H, spec.m, cols, dtype=torch.float32, device=dev)
     proj = _linear(x.reshape(B * T, D), w_qkv, w_g)
