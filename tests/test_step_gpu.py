@@ -233,3 +233,21 @@ def test_states_as_the_scan_takes_them(cuda):
             assert torch.equal(new.carries[0][0], ref.carries[0][0])
         with pytest.raises(ValueError, match="contiguous"):
             ts.DecodeGraph(module, dataclasses.replace(state, carries=([turned],)))
+
+
+@pytest.mark.parametrize("tokens", [1, 9])
+def test_expanded_weights_are_formed_once(cuda, monkeypatch, tokens):
+    """A call forms its expanded weights once, whichever path takes it."""
+    import dataclasses
+
+    import thetascan_amd as ts
+
+    cfg = dataclasses.replace(_config(64, 2, "relu2_ridge", "none", "feature", True), feature_expansion=2)
+    module = ts.ThetaScan(cfg).to(cuda)
+    core, formed = module._core, []
+    weights = core._weights
+    monkeypatch.setattr(core, "_weights", lambda: formed.append(1) or weights())
+    x = torch.randn(2, tokens, cfg.d_model, device=cuda)
+    with torch.no_grad():
+        module(x, state=module.initial_state())
+    assert len(formed) == 1

@@ -440,13 +440,13 @@ class ThetaScan(nn.Module):
                                   self.ogate.g.lin.bias if gate else None, W1, W2, self.kernel_relu2_threshold,
                                   self.proj_out.weight, spec, cfg.read_norm, H)
 
-    def _forward_step(self, x: torch.Tensor) -> torch.Tensor | None:
+    def _forward_step(self, x: torch.Tensor, weights) -> torch.Tensor | None:
         """A continuation of at most eight tokens (a decode step) of the
         one-call memory: three launches, or None where ts_memory_step does not
         take it."""
         cfg = self.cfg
         lin = None if self.ogate is None else self.ogate.g.lin
-        (W1, W2, _), = self._weights()
+        (W1, W2, _), = weights
         args = (self.proj_qkv.weight, None if lin is None else lin.weight, None if lin is None else lin.bias, W1, W2,
                 self.kernel_relu2_threshold, self.proj_out.weight)
         if not step.eligible(x, self._spec, cfg.head_dim, args):
@@ -506,9 +506,10 @@ class ThetaScan(nn.Module):
         with stream.carrying(carry):
             if self.fused_eligible(x):
                 self.last_path = "fused"
-                y = self._forward_step(x) if self._fused_cfg else None
+                weights = self._weights()
+                y = self._forward_step(x, weights) if self._fused_cfg else None
                 if y is None:
-                    y = self._forward_views(x, backend)
+                    y = self._forward_views(x, backend, weights)
             else:
                 self.last_path = "composed"
                 y = self._forward_composed(x, backend)
@@ -653,19 +654,20 @@ class ThetaScan(nn.Module):
         y = y.transpose(1, 2).reshape(B, T, cfg.n_heads * cfg.head_dim)
         return linear(y, self.proj_out.weight)
 
-    def _forward_views(self, x: torch.Tensor, backend: str = "hip") -> torch.Tensor:
+    def _forward_views(self, x: torch.Tensor, backend: str = "hip", weights=None) -> torch.Tensor:
         """The kernel memory on the HIP feature kernels for any projection
         layout and temporal mode: the raw key and query streams go through
         ts_feature_fwd (input RoPE, L2 norm, W1, RMSNorm, threshold, feature
         map, feature RoPE, and the query's residual xn + s W2 h), every view
         is scanned by the multi-view scan and read by ts_read_fwd
-        (engine.py:345-544 for depth 1, write_iters 1)."""
+        (engine.py:345-544 for depth 1, write_iters 1).  ``weights``: the
+        caller's ``_weights()``, where it has formed them."""
         cfg = self.cfg
         q, k, v = self._project(x)
         v_w = v
         if self.vmlp_in is not None:
             v_w = v_w + self.vmlp_out(F.silu(self.vmlp_in(v_w)))
-        (W1, W2, _), = self._weights()
+        (W1, W2, _), = self._weights() if weights is None else weights
         tau = self.kernel_relu2_threshold
         phi_k, _ = features.kernel_features(k, W1, None, tau, self._spec, False)
         phi_q, resid = features.kernel_features(q, W1, W2, tau, self._spec, True)
