@@ -251,3 +251,28 @@ def test_expanded_weights_are_formed_once(cuda, monkeypatch, tokens):
     with torch.no_grad():
         module(x, state=module.initial_state())
     assert len(formed) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", [CASES[2], (32, 1, "softmax_partition", "none", "input", True, False)])
+def test_an_infinite_value_spreads_as_in_the_multi_view_path(cuda, monkeypatch, case, dtype):
+    """Feature counts below the kernel's padded width: an infinite value makes
+    the reads that see it infinite, not NaN (the padding's zeros stay out)."""
+    from thetascan_amd._core.ops import step
+
+    module, state, x = _prompted(cuda, dtype, case)
+    cfg = module.config
+    with torch.no_grad():
+        # channel 5 of head 1's values overflows for the tokens whose first channel is large
+        w = module._core.proj_qkv.weight
+        w[2 * cfg.d_model + cfg.d_model // 2 + 5, 0] = 3e38
+        x = x.clone()
+        x[..., 0] = 0.0
+        x[1, 1, 0] = 16.0
+        y, new = module(x[:, :3], state=state)
+        monkeypatch.setattr(step, "eligible", lambda *a: False)
+        want, ref = module(x[:, :3], state=state)
+    assert torch.isinf(want[1, 1:]).any() and not torch.isnan(want).any()
+    assert torch.equal(torch.isinf(y), torch.isinf(want)) and not torch.isnan(y).any()
+    for a, b in zip(new._tensors(), ref._tensors()):
+        assert torch.equal(torch.isinf(a), torch.isinf(b)) and torch.equal(torch.isnan(a), torch.isnan(b))

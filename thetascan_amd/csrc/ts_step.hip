@@ -226,10 +226,14 @@ __global__ __launch_bounds__(256) void memory_step_kernel(MemStepP p) {
       if (part == 0) rs[t][row] = xs[kStepT + t][row] + p.s * a;
     }
   }
-  // ---- the recurrence and the read
+  // ---- the recurrence and the read.  A group's state rows are all features
+  // or all padding (m is the padded width or a multiple of its rows a group);
+  // the padding's weights are zeros, and stay so against an infinite value
+  // only if it does not reach them.
+  const bool on = j < d && rg * RPT < m;
   for (int t = 0; t < T; ++t) {
     const int buf = t & 1;
-    const float vj = j < d ? vs[t][j] : 0.f;
+    const float vj = on ? vs[t][j] : 0.f;
     float num = 0.f;
 #pragma unroll
     for (int r = 0; r < RPT; ++r) {
