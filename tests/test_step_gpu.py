@@ -3,7 +3,7 @@ memory (GPU tests).
 
 A mixer fed a prompt and then pieces of at most eight tokens (the step kernel)
 must continue the sequence that one whole call computes in float64: every
-padded head width and feature count, both maps, both reads, with and without
+padded head width and feature count that a memory can have, both maps, both reads, with and without
 the output gate and the learned threshold, RoPE at either placement.  Bars:
 fp32 2e-5 (fp32 sums in another order), bf16 2e-2 (the activations' rounding).
 The skinny product: fp32 accumulation of bf16 products, one rounding (8e-3 of
@@ -105,6 +105,24 @@ def test_other_continuations_keep_their_path(cuda):
     with torch.no_grad(), _lib.record_launches() as recs:
         module(x, state=module.initial_state())
     assert "ts_memory_step" not in {r[0] for r in recs}
+
+
+def test_fewer_features_than_channels_are_refused(cuda):
+    """No memory has them: the kernels are built without that combination (a
+    host check, before any launch)."""
+    import ctypes
+
+    from thetascan_amd import _lib
+
+    t = torch.zeros(4096, device=cuda)
+    s = _lib.strided(t.view(1, 1, 32, 128))
+    desc = _lib.MemoryStepDesc(1, 1, 1, 128, 64, _lib.dtype_code(t.dtype), _lib.dtype_code(t.dtype), _lib.FEAT_RELU2,
+                               0, 0, 0, 0, 1.0, 1.0, 1e-6, 0)
+    p = t.data_ptr()
+    io = _lib.MemoryStepIO(s, s, s, _lib.strided(None), s, p, p, None, None, None, None, None, None, None)
+    status = _lib.load().ts_memory_step(ctypes.byref(desc), ctypes.byref(io), _lib.stream_handle(cuda))
+    with pytest.raises(NotImplementedError, match="below the head width"):
+        _lib.check(status, "ts_memory_step")
 
 
 def _prompted(cuda, dtype, case=CASES[0], seed=3, batch=3):

@@ -36,7 +36,7 @@ def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
     projections keep (the kernel's rows are of one dtype: under an autocast to
     another the multi-view path follows the projection)."""
     return (_keeps_dtype(x) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float32)
-            and 1 <= x.shape[1] <= MAX_TOKENS and head_dim in WIDTHS and spec.m in WIDTHS
+            and 1 <= x.shape[1] <= MAX_TOKENS and head_dim in WIDTHS and spec.m in WIDTHS and spec.m >= head_dim
             and x.shape[2] == params[0].shape[1]
             and all(p is None or (p.dtype == x.dtype and p.device == x.device and p.is_contiguous()
                                   and p.data_ptr() % 16 == 0) for p in params))

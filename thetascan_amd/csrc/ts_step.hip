@@ -80,7 +80,7 @@ struct WRow {
   }
 };
 
-// DP, MP: head width and feature count padded to 64 or 128.
+// DP, MP: head width and feature count padded to 64 or 128 (DP <= MP).
 template <typename E, int DP, int MP>
 __global__ __launch_bounds__(256) void memory_step_kernel(MemStepP p) {
   constexpr int NG = 256 / DP;    // row groups of the state
@@ -349,8 +349,7 @@ void launch_step(int d, int m, int bh, hipStream_t stream, const ts::MemStepP& p
     if (m <= 64) hipLaunchKernelGGL((ts::memory_step_kernel<E, 64, 64>), dim3(bh), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((ts::memory_step_kernel<E, 64, 128>), dim3(bh), dim3(256), 0, stream, p);
   } else {
-    if (m <= 64) hipLaunchKernelGGL((ts::memory_step_kernel<E, 128, 64>), dim3(bh), dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((ts::memory_step_kernel<E, 128, 128>), dim3(bh), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((ts::memory_step_kernel<E, 128, 128>), dim3(bh), dim3(256), 0, stream, p);
   }
 }
 
@@ -369,6 +368,8 @@ int ts_memory_step(const ts_memory_step_desc* d, const ts_memory_step_io* io, hi
   for (int v : {d->d, d->m})
     if (v != 16 && v != 32 && v != 64 && v != 128)
       return fail(TS_ERR_NOT_IMPLEMENTED, "memory step: widths d %d, m %d (16, 32, 64 or 128)", d->d, d->m);
+  if (d->m < d->d)  // a memory has at least as many features as head channels
+    return fail(TS_ERR_NOT_IMPLEMENTED, "memory step: %d features below the head width %d", d->m, d->d);
   if (d->in_rot < 0 || d->in_rot > d->d || d->in_rot % 2 || d->feat_rot < 0 || d->feat_rot > d->m || d->feat_rot % 2)
     return fail(TS_ERR_VALUE, "memory step: rotated widths %d, %d", d->in_rot, d->feat_rot);
   if ((d->in_rot && !io->inv_in) || (d->feat_rot && !io->inv_feat))
