@@ -93,18 +93,47 @@ def test_skinny_linear(cuda, n, k, na, nb):
     assert rel_err(many[:n], want[:, :na]) < 8e-3
 
 
+def _same_values_unaligned(p):
+    buf = p.new_empty(p.numel() + 1)[1:].view_as(p)
+    buf.copy_(p)
+    return buf
+
+
 def test_other_continuations_keep_their_path(cuda):
-    """Nine tokens, and parameters of another dtype than the input's, take the
-    multi-view path."""
-    import thetascan_amd as ts
+    """Nine tokens, and parameters that the kernel cannot read (another dtype,
+    memory order or alignment), take the multi-view path and give its values."""
     from thetascan_amd import _lib
 
-    cfg = _config(*CASES[0])
-    module = ts.ThetaScan(cfg).to(cuda)
-    x = torch.randn(2, 9, cfg.d_model, device=cuda)
-    with torch.no_grad(), _lib.record_launches() as recs:
-        module(x, state=module.initial_state())
-    assert "ts_memory_step" not in {r[0] for r in recs}
+    module, state, x = _prompted(cuda, torch.float32)
+    nine = torch.cat([x, x[:, :1]], 1)
+    with torch.no_grad():
+        pieces, s = [], state
+        for t in range(9):
+            y, s = module(nine[:, t:t + 1], state=s)
+            pieces.append(y)
+        with _lib.record_launches() as recs:
+            y, _ = module(nine, state=state)
+        assert "ts_memory_step" not in {r[0] for r in recs}
+        assert rel_err(y, torch.cat(pieces, 1)) < 2e-5
+        core = module._core
+        bias = core.ogate.g.lin.bias
+        changes = [(bias, bias.data.to(torch.bfloat16).to(torch.float64)),
+                   (core.proj_qkv.weight, core.proj_qkv.weight.data.t().contiguous().t()),
+                   (core.proj_out.weight, _same_values_unaligned(core.proj_out.weight.data))]
+        for param, other in changes:
+            held, param.data = param.data, other
+            if other.dtype == torch.float64:
+                held = other.float()  # the same numbers in the kernel's dtype
+            with _lib.record_launches() as recs:
+                y, new = module(x[:, :2], state=state)
+            assert "ts_memory_step" not in {r[0] for r in recs}
+            param.data = held
+            with _lib.record_launches() as recs:
+                want, ref = module(x[:, :2], state=state)
+            assert "ts_memory_step" in {r[0] for r in recs}
+            assert rel_err(y, want) < 2e-5
+            for a, b in zip(new._tensors(), ref._tensors()):
+                assert rel_err(a, b) < 2e-5
 
 
 def test_fewer_features_than_channels_are_refused(cuda):
