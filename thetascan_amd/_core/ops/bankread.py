@@ -64,7 +64,10 @@ def _call(nums, masses, resids, coef, gate, gate_bias, s, eps):
 def _forward(nums: list[torch.Tensor], masses: list[torch.Tensor], resids: list[torch.Tensor], coef: torch.Tensor,
              gate: torch.Tensor | None, gate_bias: torch.Tensor | None, s: float, eps: float) -> torch.Tensor:
     lib = _lib.load()
-    desc, io, (nk, mk, rk, _, gk, _) = _call(nums, masses, resids, coef, gate, gate_bias, s, eps)
+    # (every converted operand stays bound until the launch: a dropped one's
+    # memory could become y's)
+    desc, io, kept = _call(nums, masses, resids, coef, gate, gate_bias, s, eps)
+    nk, mk, rk, _, gk, _ = kept
     B, H, T, d = nk[0].shape
     y = torch.empty(B, T, H, d, dtype=nk[0].dtype, device=nk[0].device).transpose(1, 2)
     with _lib.timed("ts_bank_read_fwd", lambda: _lib.nbytes(*nk, *mk, *rk, gk, y)):
