@@ -88,3 +88,38 @@ def test_bank_of_static_views_takes_the_passes(cuda):
     assert "ts_views_bwd" not in names
     for a, e in zip(got, want):
         assert rel_err(a, e) < 1e-2
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "dout", "dmass"])
+@pytest.mark.parametrize("m", [64, 136])
+def test_values_that_are_not_finite_stay_where_the_scans_leave_them(cuda, where, value, m):
+    """One such value makes the same gradients not finite as in one scan per
+    view and gradient: those that depend on it, none on the other side of the
+    causal mask."""
+    from thetascan_amd._core.ops import scan_hip
+
+    g = torch.Generator().manual_seed(5)
+    B, H, T, dv = 1, 2, 200, 64
+    rnd = lambda *s: torch.randn(*s, generator=g).to(cuda)  # noqa: E731
+    ts = {"q": rnd(B, H, T, m).bfloat16(), "k": rnd(B, H, T, m).bfloat16(), "v": rnd(B, H, T, dv).bfloat16()}
+    las = [None, torch.log(torch.tensor([0.9, 0.97], device=cuda)), torch.log(torch.tensor([0.99, 0.5], device=cuda))]
+    dos, dms = [rnd(B, H, T, dv).bfloat16() for _ in las], [rnd(B, H, T) for _ in las]
+    hit = {"dout": dos[1], "dmass": dms[1]}.get(where, ts.get(where))
+    hit[(0, 1, 90, 3)[: hit.ndim]] = value
+    need_r = [False] * 3
+
+    def grads():
+        return scan_hip._views_backward(ts["q"], ts["k"], ts["v"], las, dos, dms, True, True, True, need_r)[:3]
+
+    got = grads()
+    real = scan_hip.views_bwd_eligible
+    try:
+        scan_hip.views_bwd_eligible = lambda *a: False
+        want = grads()
+    finally:
+        scan_hip.views_bwd_eligible = real
+    for name, a, e in zip(("dq", "dk", "dv"), got, want):
+        off = ~torch.isfinite(e.float())
+        assert off.any() or (where, name) in {("q", "dq"), ("k", "dk"), ("v", "dv"), ("dmass", "dv")}, name
+        assert torch.equal(~torch.isfinite(a.float()), off), name

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256, 2) void views_bwd_kernel(VbwdP vp) {
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4;
   const int l16 = lane & 15;
   const int seg = blockIdx.x;
@@ -300,6 +300,12 @@ __global__ __launch_bounds__(256, 2) void views_bwd_kernel(VbwdP vp) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) ps[kb][i] += sc[i] * wv[3 - i];
         }
+        // keys past the query are left out, not only weighted by zero: a score
+        // that is not finite stays with the queries that see its key
+        if (kb == w) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ps[kb][i] = 4 * g + i <= l16 ? ps[kb][i] : 0.0f;
+        }
       }
       // the summed score enters the contraction as hi + lo (one view's score
       // is rounded once; a sum of them would lose more to the same rounding)
@@ -358,6 +364,10 @@ __global__ __launch_bounds__(256, 2) void views_bwd_kernel(VbwdP vp) {
             if (kb > w) continue;
 #pragma unroll
             for (int j = 0; j < 2; ++j) sb[kb] = mma32(frow8<E>(Vs, P, kb * 16 + l16, j, g), qk[j], sb[kb]);
+            if (kb == w) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sb[kb][i] = 4 * g + i <= l16 ? sb[kb][i] : 0.0f;
+            }
           }
 #pragma unroll
           for (int r = 0; r < NV; ++r) {
