@@ -123,3 +123,30 @@ def test_values_that_are_not_finite_stay_where_the_scans_leave_them(cuda, where,
         off = ~torch.isfinite(e.float())
         assert off.any() or (where, name) in {("q", "dq"), ("k", "dk"), ("v", "dv"), ("dmass", "dv")}, name
         assert torch.equal(~torch.isfinite(a.float()), off), name
+
+
+def test_an_overflowed_score_is_infinite(cuda):
+    """An upstream score dO . v past the largest float gives infinite gradients
+    of its sign, as one scan per view gives, not NaN."""
+    from thetascan_amd._core.ops import scan_hip
+
+    g = torch.Generator().manual_seed(9)
+    q, k, v, do = ((torch.rand(1, 1, 150, 64, generator=g) + 0.5) for _ in range(4))
+    k[..., ::2] *= -1
+    do[:, :, 20] *= 1e20
+    v[:, :, 10] *= 1e20
+    q, k, v, do = (t.to(cuda, torch.bfloat16) for t in (q, k, v, do))
+    las = [None, torch.log(torch.tensor([0.9], device=cuda))]
+    args = (q, k, v, las, [do, do], [None, None], True, True, True, [False, False])
+    got = scan_hip._views_backward(*args)[:3]
+    real = scan_hip.views_bwd_eligible
+    try:
+        scan_hip.views_bwd_eligible = lambda *a: False
+        want = scan_hip._views_backward(*args)[:3]
+    finally:
+        scan_hip.views_bwd_eligible = real
+    assert torch.isinf(want[0][0, 0, 20]).all() and torch.isinf(want[1][0, 0, 10]).all()
+    for name, a, e in zip(("dq", "dk", "dv"), got, want):
+        off = torch.isinf(e)
+        assert not torch.isnan(e).any() and not torch.isnan(a).any(), name
+        assert torch.equal(torch.isinf(a), off) and torch.equal(a[off].float(), e[off].float()), name

@@ -96,3 +96,24 @@ def test_states_of_wide_scans_stay_refused(cuda):
         scan_hip.scan_launch(*dev, want_final=True)
     with pytest.raises(NotImplementedError):
         scan_hip.scan_launch(*dev, init_state=torch.zeros(2, 2, 192, 64, device=cuda))
+
+
+@pytest.mark.parametrize("Dk", [192, 384])
+def test_an_overflowed_score_is_infinite(cuda, monkeypatch, Dk):
+    """A score past the largest float gives an infinite output of its sign, as
+    the block-wise scan gives, not NaN (its hi + lo pair is inf + 0)."""
+    from thetascan_amd._core.ops import scan_hip
+
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.rand(1, 1, 150, w, generator=g) + 0.5 for w in (Dk, Dk, 64))
+    q[:, :, 20] *= 1e20
+    k[:, :, 10] *= 1e20
+    v[..., ::2] *= -1
+    q, k, v = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
+    got, _, _ = scan_hip.scan_launch(q, k, v)
+    monkeypatch.setattr(scan_hip, "WIDE_KEYS", 128)
+    want, _, _ = scan_hip.scan_launch(q, k, v)
+    assert torch.isinf(want[0, 0, 20]).all() and not torch.isnan(want).any()
+    off = torch.isinf(want)
+    assert not torch.isnan(got).any() and torch.equal(torch.isinf(got), off)
+    assert torch.equal(got[off], want[off]) and rel_err(got[~off], want[~off]) < TOL

@@ -117,6 +117,14 @@ __device__ __forceinline__ typename Frag<E>::f4 frow4(const E* rows, int pitch, 
   return LdsIO<E>::ld4(rows + row * pitch + 32 * j + 4 * g);
 }
 
+// What bf16(x) leaves of x, as the second operand of a hi + lo pair.  Nothing
+// where it is infinite (x, or its rounding, past the largest bf16) or NaN: the
+// pair then is what one rounding of x is.
+__device__ __forceinline__ bf16 bf16_rest(float x, bf16 hi) {
+  const float r = x - tof(hi);
+  return (bf16)(fabsf(r) < INFINITY ? r : 0.f);
+}
+
 // A broadcast operand: eight fp32 LDS values (the same two runs of four a
 // frow8 / col8 fragment covers), identical for every lane of the group.
 template <typename E>

@@ -384,8 +384,8 @@ __global__ __launch_bounds__(256, DK == 192 || DK == 256 ? 2 : 1) void scan_kern
       if constexpr (LO) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          p0lo[e] = cvt<E>(sc[e >> 2][e & 3] - tof(p0[e]));
-          p1lo[e] = cvt<E>(sc[2 + (e >> 2)][e & 3] - tof(p1[e]));
+          p0lo[e] = bf16_rest(sc[e >> 2][e & 3], p0[e]);
+          p1lo[e] = bf16_rest(sc[2 + (e >> 2)][e & 3], p1[e]);
         }
       }
       const E* st = st_base + (c & (L.nst - 1)) * L.st;

@@ -312,8 +312,8 @@ __global__ __launch_bounds__(256, 2) void views_bwd_kernel(VbwdP vp) {
       F8 p0 = IO::from_acc(ps[0], ps[1]), p1 = IO::from_acc(ps[2], ps[3]), p0l, p1l;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        p0l[e] = (E)(ps[e >> 2][e & 3] - tof(p0[e]));
-        p1l[e] = (E)(ps[2 + (e >> 2)][e & 3] - tof(p1[e]));
+        p0l[e] = bf16_rest(ps[e >> 2][e & 3], p0[e]);
+        p1l[e] = bf16_rest(ps[2 + (e >> 2)][e & 3], p1[e]);
       }
       const uint32_t ro = row_off(p, t0, query, (int)vp.out.st * 2);
       const rsrc_t out_rs =
