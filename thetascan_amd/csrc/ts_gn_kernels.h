@@ -1134,8 +1134,12 @@ __global__ __launch_bounds__(256) void gn_write_fwd_wide_kernel(GnP p) {
   }
 }
 
-// Two waves per SIMD (two workgroups' LDS fit a CU): 205 -> 166 us at B4 H8 T3001
-// d64 m192 when it was given them.
+// Two waves per SIMD, with half the registers each: two workgroups' LDS fit a
+// CU at hidden width 192 (205 -> 166 us at B4 H8 T3001 d64 m192 when it was
+// given them) and at 384 of 32-wide tokens.  At 384 of 64-wide tokens one
+// workgroup (116 KB) fits, and the 256 registers still measure no slower than
+// 512: 290 us against 302, the read backward's two calls 222 and 116 us
+// against 242 and 119.
 template <int ACT, int D, int MB>
 __global__ __launch_bounds__(256, 2) void gn_write_bwd_wide_kernel(GnP p) {
   typedef bf16 E;
