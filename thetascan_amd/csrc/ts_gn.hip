@@ -27,15 +27,21 @@ int check_gn(const ts_gn_desc* d) {
   return TS_OK;
 }
 
-// 64 rows stay below the 32-bit offsets of their buffer resource.
-int64_t gn_max_stride(int vec) { return (int64_t)(ts::kGnRowsEnd / (16u / vec)) / 64 - 512; }
-
-bool gn_stream_ok(const ts_strided& s, int vec) {
-  return s.ptr == nullptr || (((uintptr_t)s.ptr & 15u) == 0 && s.sb % vec == 0 && s.sh % vec == 0 && s.st % vec == 0 &&
-                              s.st >= 0 && s.st <= gn_max_stride(vec));
+// A group's rows stay below the 32-bit offsets of their buffer resource: the
+// rows that there are from the first, or, backwards, all 64 from the last.
+bool gn_stream_ok(const ts_strided& s, int T, int vec) {
+  if (!s.ptr) return true;
+  if (((uintptr_t)s.ptr & 15u) || s.sb % vec || s.sh % vec || s.st % vec) return false;
+  if (T <= 1) return true;
+  const int rows = s.st < 0 || T > ts::TT ? ts::TT : T;
+  const int64_t most = (int64_t)(ts::kGnRowsEnd / (16u / vec) - 512u) / (rows - 1);
+  return -most <= s.st && s.st <= most;
 }
 
-ts::Str gn_str(const ts_strided& s) { return ts::Str{const_cast<void*>(s.ptr), s.sb, s.sh, (int)s.st}; }
+// (one row has no stride)
+ts::Str gn_str(const ts_strided& s, int T) {
+  return ts::Str{const_cast<void*>(s.ptr), s.sb, s.sh, T > 1 ? (int)s.st : 0};
+}
 
 // Hidden widths the chunked kernels take (bf16, head widths 32 and 64).
 bool gn_is_wide(const ts_gn_desc* d) {
@@ -147,12 +153,12 @@ int ts_gn_write_fwd(const ts_gn_desc* d, const ts_gn_io* io, hipStream_t stream)
   if (d->has_tau && !io->tau) return fail(TS_ERR_VALUE, "gn: missing tau");
   const int vec = d->dtype == TS_BF16 ? 8 : 4;
   for (const ts_strided* s : {&io->x, &io->v, &io->h, &io->lam, &io->g})
-    if (!gn_stream_ok(*s, vec)) return fail(TS_ERR_VALUE, "gn: streams need 16-byte aligned rows (64 of them under 4 GiB)");
+    if (!gn_stream_ok(*s, d->T, vec)) return fail(TS_ERR_VALUE, "gn: streams need 16-byte aligned rows (64 of them under 4 GiB)");
   if (d->T == 0) return TS_OK;
   ts::GnP p;
   gn_fill(d, p);
-  p.x = gn_str(io->x); p.v = gn_str(io->v);
-  p.h = gn_str(io->h); p.lam = gn_str(io->lam); p.g = gn_str(io->g);
+  p.x = gn_str(io->x, d->T); p.v = gn_str(io->v, d->T);
+  p.h = gn_str(io->h, d->T); p.lam = gn_str(io->lam, d->T); p.g = gn_str(io->g, d->T);
   p.w1 = io->w1; p.w2 = io->w2; p.w2t = io->w2t; p.tau = io->tau;
   return gn_launch(d, p, true, stream);
 }
@@ -166,13 +172,13 @@ int ts_gn_write_bwd(const ts_gn_desc* d, const ts_gn_bwd_io* io, hipStream_t str
   if (d->has_tau && !io->tau) return fail(TS_ERR_VALUE, "gn bwd: missing tau");
   const int vec = d->dtype == TS_BF16 ? 8 : 4;
   for (const ts_strided* s : {&io->x, &io->v, &io->dh, &io->dlam, &io->dg, &io->dx_in, &io->dx, &io->dv})
-    if (!gn_stream_ok(*s, vec)) return fail(TS_ERR_VALUE, "gn bwd: streams need 16-byte aligned rows (64 of them under 4 GiB)");
+    if (!gn_stream_ok(*s, d->T, vec)) return fail(TS_ERR_VALUE, "gn bwd: streams need 16-byte aligned rows (64 of them under 4 GiB)");
   if (d->T == 0) return TS_OK;
   ts::GnP p;
   gn_fill(d, p);
-  p.x = gn_str(io->x); p.v = gn_str(io->v);
-  p.dh = gn_str(io->dh); p.dlam = gn_str(io->dlam); p.dg = gn_str(io->dg); p.dxin = gn_str(io->dx_in);
-  p.dx = gn_str(io->dx); p.dv = gn_str(io->dv);
+  p.x = gn_str(io->x, d->T); p.v = gn_str(io->v, d->T);
+  p.dh = gn_str(io->dh, d->T); p.dlam = gn_str(io->dlam, d->T); p.dg = gn_str(io->dg, d->T); p.dxin = gn_str(io->dx_in, d->T);
+  p.dx = gn_str(io->dx, d->T); p.dv = gn_str(io->dv, d->T);
   p.w1 = io->w1; p.w2 = io->w2; p.w1t = io->w1t; p.w2t = io->w2t; p.tau = io->tau;
   p.tm = io->tiles_m; p.td = io->tiles_d;
   return gn_launch(d, p, false, stream);
@@ -190,11 +196,11 @@ int ts_gn_read_fwd(const ts_gn_read_desc* r, const ts_gn_read_io* io, hipStream_
   if (r->has_tau && !io->tau) return fail(TS_ERR_VALUE, "gn read: missing tau");
   const int vec = r->dtype == TS_BF16 ? 8 : 4;
   for (const ts_strided* s : {&io->q, &io->num, &io->h, &io->resid})
-    if (!gn_stream_ok(*s, vec)) return fail(TS_ERR_VALUE, "gn read: streams need 16-byte aligned rows (64 of them under 4 GiB)");
+    if (!gn_stream_ok(*s, r->T, vec)) return fail(TS_ERR_VALUE, "gn read: streams need 16-byte aligned rows (64 of them under 4 GiB)");
   if (r->T == 0) return TS_OK;
   ts::GnReadP p;
   gn_read_fill(r, &d, p, io->mass);
-  p.q = gn_str(io->q); p.num = gn_str(io->num); p.h = gn_str(io->h); p.resid = gn_str(io->resid);
+  p.q = gn_str(io->q, r->T); p.num = gn_str(io->num, r->T); p.h = gn_str(io->h, r->T); p.resid = gn_str(io->resid, r->T);
   p.w1 = io->w1; p.w2 = io->w2; p.tau = io->tau;
   return gn_read_launch(&d, p, true, stream);
 }
@@ -211,12 +217,12 @@ int ts_gn_read_bwd(const ts_gn_read_desc* r, const ts_gn_read_bwd_io* io, hipStr
   if (r->has_tau && !io->tau) return fail(TS_ERR_VALUE, "gn read bwd: missing tau");
   const int vec = r->dtype == TS_BF16 ? 8 : 4;
   for (const ts_strided* s : {&io->q, &io->num, &io->dh, &io->dresid, &io->dq, &io->dnum})
-    if (!gn_stream_ok(*s, vec)) return fail(TS_ERR_VALUE, "gn read bwd: streams need 16-byte aligned rows");
+    if (!gn_stream_ok(*s, r->T, vec)) return fail(TS_ERR_VALUE, "gn read bwd: streams need 16-byte aligned rows (64 of them under 4 GiB)");
   if (r->T == 0) return TS_OK;
   ts::GnReadP p;
   gn_read_fill(r, &d, p, io->mass);
-  p.q = gn_str(io->q); p.num = gn_str(io->num);
-  p.dh = gn_str(io->dh); if (r->want_resid) p.dresid = gn_str(io->dresid); p.dq = gn_str(io->dq); p.dnum = gn_str(io->dnum);
+  p.q = gn_str(io->q, r->T); p.num = gn_str(io->num, r->T);
+  p.dh = gn_str(io->dh, r->T); if (r->want_resid) p.dresid = gn_str(io->dresid, r->T); p.dq = gn_str(io->dq, r->T); p.dnum = gn_str(io->dnum, r->T);
   p.dmass = io->dmass;
   p.w1 = io->w1; p.w1t = io->w1t; p.w2t = io->w2t; p.tau = io->tau;
   p.tm = io->tiles_m; p.td = io->tiles_d;

@@ -142,8 +142,8 @@ struct GnTok {
 // an offset past its end, so its loads return zero and its stores are dropped
 // with no branch around the access (a branch per access kept the loads of a
 // chain from being in flight together).  A stream without a pointer reads as
-// zeros.  Strides: any st >= 0 (0: one row for every token) whose 64 rows
-// stay under 4 GiB (the host checks).
+// zeros.  Strides: any st (0: one row for every token; below 0: the resource
+// starts at the group's last row) whose 64 rows stay under 4 GiB (the host checks).
 template <typename E>
 __device__ __forceinline__ void gn_ld(rsrc_t rs, uint32_t off, float* o) {
   if constexpr (sizeof(E) == 2) {
@@ -169,15 +169,22 @@ constexpr uint32_t kGnRowsEnd = 0xffffe000u;
 __device__ __forceinline__ uint32_t gn_off(const GnTok& tk, uint32_t off) { return tk.valid() ? off : 0xfffff000u; }
 template <typename E>
 __device__ __forceinline__ rsrc_t gn_rows(const Str& s, int b, int h, const GnTok& tk) {
-  return make_rsrc((const E*)s.ptr + b * s.sb + h * s.sh + (int64_t)tk.t0 * s.st, s.ptr ? kGnRowsEnd : 0u);
+  return make_rsrc((const E*)s.ptr + b * s.sb + h * s.sh + (int64_t)tk.t0 * s.st + (int64_t)(TT - 1) * min(s.st, 0),
+                   s.ptr ? kGnRowsEnd : 0u);
+}
+// Byte offset of column c of this lane's row in gn_rows' resource.
+template <typename E>
+__device__ __forceinline__ uint32_t gn_row(const Str& s, const GnTok& tk, int c) {
+  return gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st - (uint32_t)(TT - 1) * (uint32_t)min(s.st, 0) + c) *
+                        (uint32_t)sizeof(E));
 }
 template <typename E>
 __device__ __forceinline__ void ld4_row(const Str& s, int b, int h, const GnTok& tk, int c, float* o) {
-  gn_ld<E>(gn_rows<E>(s, b, h, tk), gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c) * (uint32_t)sizeof(E)), o);
+  gn_ld<E>(gn_rows<E>(s, b, h, tk), gn_row<E>(s, tk, c), o);
 }
 template <typename E>
 __device__ __forceinline__ void st4_row(const Str& s, int b, int h, const GnTok& tk, int c, const float* v) {
-  gn_st<E>(gn_rows<E>(s, b, h, tk), gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c) * (uint32_t)sizeof(E)), v);
+  gn_st<E>(gn_rows<E>(s, b, h, tk), gn_row<E>(s, tk, c), v);
 }
 // Row n0 + row of a head-major tile [.., N, w] (n0: the group's first row).
 template <typename E>
@@ -199,7 +206,7 @@ struct GnAhead {
       const rsrc_t rs = gn_rows<E>(s, b, h, tk);
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
-        const uint32_t off = gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c0 + 16 * i) * (uint32_t)sizeof(E));
+        const uint32_t off = gn_row<E>(s, tk, c0 + 16 * i);
         if constexpr (sizeof(E) == 2) r[i] = bld8(rs, off);
         else r[i] = bld16(rs, off);
       }
@@ -228,8 +235,7 @@ struct GnRing {
   __device__ __forceinline__ void load(const Str& s, int b, int h, const GnTok& tk, int g, int c) {
     const rsrc_t rs = gn_rows<bf16>(s, b, h, tk);
 #pragma unroll
-    for (int f = 0; f < 4; ++f)
-      nxt[f] = bld8(rs, gn_off(tk, ((uint32_t)tk.row * (uint32_t)s.st + c * 64 + f * 16 + 4 * g) * 2u));
+    for (int f = 0; f < 4; ++f) nxt[f] = bld8(rs, gn_row<bf16>(s, tk, c * 64 + f * 16 + 4 * g));
   }
   // the loaded chunk becomes the present one; chunk c is loaded
   __device__ __forceinline__ void step(const Str& s, int b, int h, const GnTok& tk, int g, int c) {
