@@ -94,3 +94,27 @@ def test_gn_rows_of_negative_stride(cuda, monkeypatch, dtype, d, m, T):
             assert torch.equal(a, b), i
         else:
             assert rel_err(a, b) < (2e-2 if dtype == torch.bfloat16 else 1e-5), i
+
+
+@pytest.mark.parametrize("dtype,d,m", [(torch.bfloat16, 64, 128), (torch.bfloat16, 32, 192)])
+@pytest.mark.parametrize("layout", ["token_major", "one for all tokens"])
+def test_gn_read_with_a_strided_mass(cuda, dtype, d, m, layout):
+    """The gradient of a mass of any strides is the contiguous copy's."""
+    from thetascan_amd._core.ops import gn
+
+    B, H, T = 2, 3, 70
+    g = torch.Generator().manual_seed(m)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(cuda, dtype)  # noqa: E731
+    q, num, w1 = rnd(B, H, T, d), rnd(B, H, T, m), rnd(H, m, d) / d ** 0.5
+    if layout == "token_major":
+        mass = (torch.rand(B, T, H, generator=g) + 0.5).to(cuda).transpose(1, 2)
+    else:
+        mass = (torch.rand(B, H, 1, generator=g) + 0.5).to(cuda).expand(B, H, T)
+    dy = rnd(B, H, T, m)
+
+    def run(mass):
+        mass = mass.detach().requires_grad_(True)
+        h, _ = gn.read_stage(q, w1, None, None, num, mass, corr=gn.READ_NORMALIZED)
+        return torch.autograd.grad(h, mass, dy)[0]
+
+    assert torch.equal(run(mass), run(mass.contiguous()))

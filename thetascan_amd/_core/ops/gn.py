@@ -293,7 +293,8 @@ def _gn_read_backward_impl(dh: torch.Tensor | None, dresid: torch.Tensor | None,
     w2t = w2.detach().to(dt).transpose(1, 2).contiguous() if want_resid else None
     tc = None if tau is None else tau.detach().to(torch.float32).contiguous()
     nk = None if num is None else _rows(num.to(dt))
-    mk = None if mass is None else mass.detach().to(torch.float32)
+    # (the kernel writes dmass with the mass's own strides)
+    mk = None if mass is None else mass.detach().to(torch.float32).contiguous()
     dh = None if dh is None else _rows(dh.to(dt))
     dresid = None if (dresid is None or not want_resid) else _rows(dresid.to(dt))
     dq = torch.empty(B, H, T, d, dtype=dt, device=qk.device)
