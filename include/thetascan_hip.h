@@ -46,8 +46,15 @@ extern "C" {
  * 16: ts_stack_heads; nothing earlier changed.
  * 17: ts_scale_add_fwd / ts_scale_add_bwd / ts_scale_add_parts, ts_relu2_fwd /
  *     ts_relu2_bwd, ts_softcap_xent_fwd / ts_softcap_xent_bwd, ts_blend_gated_fwd;
- *     nothing earlier changed. */
-#define TS_ABI_VERSION 17
+ *     nothing earlier changed.
+ * 18: ts_views_bwd, ts_memory_step, ts_skinny_linear, ts_bank_read_fwd /
+ *     ts_bank_read_bwd / ts_bank_read_parts, ts_bank_params_fwd /
+ *     ts_bank_params_bwd, ts_rownorm_fwd_to / ts_rownorm_bwd_to,
+ *     ts_rotary_tables, ts_causal_attention_fwd, ts_scale_add_norm_fwd and
+ *     ts_contract_sums; bf16 scans take up to 384 keys and 512 values; the 64
+ *     rows of a token group of a GN stream have to lie within 4 GiB (a row
+ *     stride of 32 Mi elements and more was taken before). */
+#define TS_ABI_VERSION 18
 
 enum ts_status {
   TS_OK = 0,
@@ -610,7 +617,8 @@ typedef struct ts_gn_desc {
 } ts_gn_desc;
 
 typedef struct ts_gn_io {
-  ts_strided x, v;      /* [B,H,T,d] keys (as written) and values               */
+  ts_strided x, v;      /* [B,H,T,d] keys (as written) and values; of every GN
+                           stream, any time stride whose 64 rows span < 4 GiB   */
   const void* w1;       /* [H,m,d]                                              */
   const void* w2;       /* [H,d,m]                                              */
   const void* w2t;      /* [H,m,d] transposed copy of w2                        */
@@ -843,7 +851,7 @@ int ts_views_bwd(const ts_views_bwd_desc* desc, const ts_views_bwd_io* io, void*
  * positions position .. position + T - 1, the position from io->position (an
  * int64 on the device) where set, else desc->position. */
 typedef struct ts_memory_step_desc {
-  int32_t B, H, T, d, m;          /* d, m: 16, 32, 64 or 128; T <= 8           */
+  int32_t B, H, T, d, m;          /* d <= m: 16, 32, 64 or 128; T <= 8         */
   int32_t dtype;                  /* of q, k, v, g, y, w1, w2                  */
   int32_t param_dtype;            /* of tau, gbias                             */
   int32_t kind;                   /* ts_feature_kind                           */

@@ -37,7 +37,27 @@ def test_library_exports_every_declared_symbol():
     missing = [name for name in declared_functions() if not hasattr(lib, name)]
     assert not missing, missing
     lib.ts_abi_version.restype = ctypes.c_int
-    assert lib.ts_abi_version() == 17
+    header = (REPO / "include" / "thetascan_hip.h").read_text()
+    assert lib.ts_abi_version() == int(re.search(r"#define TS_ABI_VERSION (\d+)", header).group(1)) == _lib.ABI_VERSION
+
+
+def test_a_library_of_another_version_is_refused(tmp_path, monkeypatch):
+    """By its version, before any entry point it may lack is looked up."""
+    import shutil
+    import subprocess
+
+    from thetascan_amd import _lib
+
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("no C compiler")
+    source, library = tmp_path / "older.c", tmp_path / "older.so"
+    source.write_text("int ts_abi_version(void) { return 17; }\n")
+    subprocess.run([gcc, "-shared", "-fPIC", str(source), "-o", str(library)], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", library)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match="ABI version 17"):
+        _lib.load()
 
 
 def test_views_descriptor_validation_on_the_host():

@@ -545,6 +545,8 @@ class RetentionIO(ctypes.Structure):
 FEAT_RELU2 = 0
 FEAT_SOFTMAX = 1
 
+ABI_VERSION = 18  # the include/thetascan_hip.h these bindings are written for
+
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
 
@@ -569,6 +571,10 @@ def load() -> ctypes.CDLL:
             )
         lib = ctypes.CDLL(str(LIB_PATH), mode=ctypes.RTLD_LOCAL)
         lib.ts_abi_version.restype = ctypes.c_int
+        # before any other entry point is looked up: another version may lack it
+        if lib.ts_abi_version() != ABI_VERSION:
+            raise RuntimeError(f"{LIB_PATH.name} is of ABI version {lib.ts_abi_version()}, these bindings of "
+                               f"{ABI_VERSION}: build it again")
         lib.ts_last_error.restype = ctypes.c_char_p
         lib.ts_scan_layout.argtypes = [
             ctypes.POINTER(ScanDesc),
@@ -702,8 +708,6 @@ def load() -> ctypes.CDLL:
         lib.ts_softcap_xent_bwd.argtypes = [P(RowsDesc), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
                                             ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p,
                                             ctypes.c_void_p]
-        if lib.ts_abi_version() != 17:
-            raise RuntimeError("libthetascan_hip.so ABI version mismatch")
         _lib = lib
         return lib
 
