@@ -150,3 +150,31 @@ def test_an_overflowed_score_is_infinite(cuda):
         off = torch.isinf(e)
         assert not torch.isnan(e).any() and not torch.isnan(a).any(), name
         assert torch.equal(torch.isinf(a), off) and torch.equal(a[off].float(), e[off].float()), name
+
+
+@pytest.mark.parametrize("layout", ["token_major", "padded", "one row for all tokens", "one value for all"])
+def test_upstream_gradients_of_any_layout(cuda, layout):
+    """Upstream gradients as autograd hands them on: rows of a projection or of
+    a wider matrix, and broadcast ones (a sum's), give the contiguous copies'
+    bits."""
+    from thetascan_amd._core.ops import scan_hip
+
+    g = torch.Generator().manual_seed(4)
+    B, H, T, m, dv = 2, 2, 150, 72, 40
+    rnd = lambda *s: torch.randn(*s, generator=g).to(cuda)  # noqa: E731
+
+    def upstream():
+        if layout == "token_major":
+            return rnd(B, T, H, dv).bfloat16().transpose(1, 2), rnd(B, T, H).transpose(1, 2)
+        if layout == "padded":
+            return rnd(B, H, T, dv + 4).bfloat16()[..., 4:], rnd(B, H, T + 3)[..., 3:]
+        if layout == "one row for all tokens":
+            return rnd(B, H, 1, dv).bfloat16().expand(B, H, T, dv), rnd(B, H, 1).expand(B, H, T)
+        return rnd(1).bfloat16().expand(B, H, T, dv), rnd(1).expand(B, H, T)
+
+    q, k, v = rnd(B, H, T, m).bfloat16(), rnd(B, H, T, m).bfloat16(), rnd(B, H, T, dv).bfloat16()
+    las = [None, torch.log(torch.tensor([0.9, 0.97], device=cuda)), torch.log(torch.tensor([0.99, 0.5], device=cuda))]
+    dos, dms = zip(*(upstream() for _ in las))
+    run = lambda dos, dms: scan_hip.views_bwd_launch(q, k, v, las, dos, dms, need_q=True, need_kv=True)  # noqa: E731
+    for a, b in zip(run(dos, dms), run([t.contiguous() for t in dos], [t.contiguous() for t in dms])):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
