@@ -455,7 +455,11 @@ def views_eligible(q: torch.Tensor, v: torch.Tensor, kinds) -> bool:
 def views_bwd_eligible(q: torch.Tensor, v: torch.Tensor, kinds) -> bool:
     """Whether ts_views_bwd forms these views' gradients: bf16 on the GPU, 2
     or 3 retentions that are none or static, m <= 512, dv <= 64, and (batch,
-    head) slices of 31-bit offsets."""
+    head) slices of 31-bit offsets.  The kernels hold every view's [64][64]
+    state in a wave's accumulators, which at three views is what two waves per
+    SIMD leave room for; a larger bank takes one scan per view and gradient
+    (groups of its views, whose gradients would add up through memory, were
+    not measured)."""
     B, H, T, m = q.shape
     return (q.is_cuda and q.dtype == torch.bfloat16 and 2 <= len(kinds) <= _lib.MAX_VIEWS
             and all(k in (_lib.RET_NONE, _lib.RET_STATIC) for k in kinds)

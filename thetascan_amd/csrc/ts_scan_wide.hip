@@ -6,13 +6,15 @@
 // into 128-wide key blocks it took three launches per block, with the partial
 // outputs added up in fp32 through memory.
 //
-// Bound: HBM for the main pass (B8 H8 T4096, 384 x 64: 0.70 GB in 202 us,
-// against 277 us for three 128-wide blocks; B4 H8 T3001, 192 x 192: 85 us
-// against 193 us), then LDS bandwidth: a wave of a 384-wide tile reads about
-// 125 KB of K and state fragments for about 126 MFMAs.  K [64][392],
-// V [64][72] and one state copy [64][392] take 113 KB, so one workgroup per
-// CU is resident (192 and 256 wide: two), and the next tile's rows are
-// fetched into registers while a tile is computed.
+// Bound: HBM for the main pass, then LDS bandwidth: a wave of a 384-wide tile
+// reads about 125 KB of K and state fragments for about 126 MFMAs.  Whole
+// calls (summary, prefix and main pass) against the 128-wide blocks:
+//   B8 H8 T4096, 384 x 64 (0.70 GB): plain 202 and 282 us, with the mass
+//   column 234 and 592, with a static retention and the mass 266 and 594;
+//   B4 H8 T3001, 192 x 192: 89 and 194 us, with both 110 and 333.
+// K [64][392], V [64][72] and one state copy [64][392] take 113 KB, so one
+// workgroup per CU is resident (192 and 256 wide: two), and the next tile's
+// rows are fetched into registers while a tile is computed.
 
 #include "ts_scan_kernel.h"
 
