@@ -3,7 +3,8 @@
 A decode step at a small batch is launch-bound: one token per sequence gives
 every kernel of the step (projections, feature maps, the scan's token-by-token
 recurrence, the read, the output projection) a few microseconds of work, while
-issuing its twenty-odd launches through Python costs several times that.
+issuing its launches (three for the one-call kernel memory, twenty-odd for the
+others) through Python costs several times that.
 :class:`DecodeGraph` records one step once -- with the carried state in fixed
 buffers that the step updates in place and the position (RoPE phases) held in
 a device counter -- and replays it::
