@@ -22,10 +22,10 @@ WIDTHS = (16, 32, 64, 128)
 SKINNY_ROWS = 64
 
 
-def _keeps_dtype(x: torch.Tensor) -> bool:
-    """Whether a library product of x's dtype gives that dtype (autocast may
-    choose another for it)."""
-    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
+def _keeps_dtype(dtype: torch.dtype) -> bool:
+    """Whether a library product of ``dtype`` operands gives that dtype
+    (autocast may choose another for it)."""
+    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == dtype
 
 
 def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
@@ -35,11 +35,17 @@ def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
     parameter a contiguous tensor beside the input and of its dtype, which the
     projections keep (the kernel's rows are of one dtype: under an autocast to
     another the multi-view path follows the projection)."""
-    return (_keeps_dtype(x) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float32)
-            and 1 <= x.shape[1] <= MAX_TOKENS and head_dim in WIDTHS and spec.m in WIDTHS and spec.m >= head_dim
-            and x.shape[2] == params[0].shape[1]
-            and all(p is None or (p.dtype == x.dtype and p.device == x.device and p.is_contiguous()
-                                  and p.data_ptr() % 16 == 0) for p in params))
+    dtype, device = x.dtype, x.get_device()
+    _, T, D = x.shape
+    if not (x.is_cuda and (dtype == torch.bfloat16 or dtype == torch.float32) and 1 <= T <= MAX_TOKENS
+            and spec.m in WIDTHS and head_dim in WIDTHS and spec.m >= head_dim and D == params[0].shape[1]
+            and _keeps_dtype(dtype)):
+        return False
+    for p in params:
+        if p is not None and not (p.dtype == dtype and p.get_device() == device and p.is_contiguous()
+                                  and p.data_ptr() % 16 == 0):
+            return False
+    return True
 
 
 def _linear(x2: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor | None) -> torch.Tensor:
@@ -47,18 +53,19 @@ def _linear(x2: torch.Tensor, wa: torch.Tensor, wb: torch.Tensor | None) -> torc
     a library GEMM of so few rows is all latency (B8, 512 -> 1536 and 512:
     4.8 us each against 3.7 us for both, with no concatenated weight)."""
     n, k = x2.shape
-    na, nb = wa.shape[0], 0 if wb is None else wb.shape[0]
+    row, col = x2.stride()
+    na, ka = wa.shape
+    nb, kb = (0, k) if wb is None else wb.shape
     # (a weight of another row length is the library product's to refuse: the
     # kernel reads k elements of every row; rows of other strides, which a
     # reshape leaves as they are, are its to read)
-    if not (x2.dtype == torch.bfloat16 and n <= SKINNY_ROWS and k % 32 == 0 and na % 16 == 0 and nb % 16 == 0
-            and all(w is None or w.shape[1] == k for w in (wa, wb))
-            and x2.data_ptr() % 16 == 0 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0):
+    if not (x2.dtype == torch.bfloat16 and n <= SKINNY_ROWS and ka == k and kb == k and k % 32 == 0 and na % 16 == 0
+            and nb % 16 == 0 and col == 1 and row % 8 == 0 and x2.data_ptr() % 16 == 0):
         parts = [F.linear(x2, w) for w in (wa, wb) if w is not None]
         return parts[0] if wb is None else torch.cat(parts, dim=1)
     y = torch.empty(n, na + nb, dtype=x2.dtype, device=x2.device)
-    status = _lib.load().ts_skinny_linear(x2.data_ptr(), n, k, x2.stride(0), wa.data_ptr(), na, _lib.ptr(wb), nb,
-                                          y.data_ptr(), y.stride(0), _lib.stream_handle(x2.device))
+    status = _lib.load().ts_skinny_linear(x2.data_ptr(), n, k, row, wa.data_ptr(), na, _lib.ptr(wb), nb, y.data_ptr(),
+                                          na + nb, _lib.stream_handle(x2.device))
     _lib.check(status, "ts_skinny_linear")
     return y
 
@@ -76,7 +83,7 @@ def kernel_step(x: torch.Tensor, w_qkv, w_g, b_g, w1, w2, tau, w_out, spec, norm
     init = None
     if blocks is not None:
         # (as scan_launch takes a carried state)
-        if (len(blocks) != 1 or tuple(blocks[0].shape[-2:]) != (spec.m, cols)
+        if (len(blocks) != 1 or blocks[0].shape[-2:] != (spec.m, cols)
                 or blocks[0].numel() != B * H * spec.m * cols):
             raise ValueError("streaming state does not match this scan's widths")
         init = blocks[0].detach().to(device=dev, dtype=torch.float32).contiguous()
