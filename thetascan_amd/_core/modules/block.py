@@ -25,7 +25,7 @@ import torch.nn.functional as F
 from ..config import ThetaScanConfig
 from ...state import ThetaScanState, config_fingerprint
 from ..ops import bankread, composed, features, fused, gn, interface, maps, prologue, step, stream
-from ..ops.linear import linear, stack_heads
+from ..ops.linear import keeps_dtype, linear, stack_heads
 from ..ops.interface import Accumulator, FadeFast, FadeStale, NullAccumulator, resolve_backend
 from .gates import DecayGate, OutGate
 from .norms import l2norm
@@ -641,7 +641,8 @@ class ThetaScan(nn.Module):
         y = reads[0]
         if cfg.read_fade:
             if (self.ogate is not None and not torch.is_grad_enabled() and x.is_cuda
-                    and all(r.dtype == x.dtype for r in reads) and self.ogate.g.lin.weight.dtype == x.dtype):
+                    and all(r.dtype == x.dtype for r in reads) and self.ogate.g.lin.weight.dtype == x.dtype
+                    and keeps_dtype(x.dtype)):
                 # inference: the output gate in the blend's epilogue (one
                 # launch, no gate or transposing copy of the blended read)
                 lin = self.ogate.g.lin

@@ -37,6 +37,13 @@ def eligible(nums, masses, resids, heads: int) -> bool:
             and all((m is None) == (masses[0] is None) for m in masses))
 
 
+def check_gate(gate: torch.Tensor | None, num: torch.Tensor) -> None:
+    """Raise unless ``gate`` has the rows that a read epilogue of ``num`` reads."""
+    if gate is not None and (gate.dtype != num.dtype or gate.shape != num.shape or gate.device != num.device):
+        raise ValueError(f"the output gate's pre-activation ({gate.dtype}, {tuple(gate.shape)}, {gate.device}) does not "
+                         f"match the reads ({num.dtype}, {tuple(num.shape)}, {num.device})")
+
+
 def _rows(t: torch.Tensor) -> torch.Tensor:
     vec = 16 // t.element_size()
     ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:3])
@@ -153,6 +160,7 @@ def bank_read(nums, masses, resids, coef: torch.Tensor, *, s: float = 1.0, eps: 
     ``coef`` [n,H]; with ``gate`` (the [B,H,T,d] view of x W_g^T, the dtype of
     ``nums``) the output gate is applied too."""
     mass = [] if masses[0] is None else list(masses)
+    check_gate(gate, nums[0])
     return _bank_read_op(list(nums), mass, list(resids), coef, gate, gate_bias, float(s), float(eps))
 
 

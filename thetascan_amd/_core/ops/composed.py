@@ -40,7 +40,7 @@ import torch
 import torch.nn.functional as F
 
 from . import bankread, gn, interface, kernel_features, maps
-from .linear import head_matmul
+from .linear import head_matmul, keeps_dtype
 from ..modules.norms import rmsnorm
 
 
@@ -82,7 +82,9 @@ class OutputRequest:
         B, T, _ = self.x.shape
         if len(nums) != (1 if self.coef is None else self.coef.shape[0]):
             return False
-        if self.weight is not None and not (self.x.dtype == num.dtype and self.weight.dtype == num.dtype):
+        # the epilogue reads the gate's pre-activation in the reads' dtype
+        if self.weight is not None and not (self.x.dtype == num.dtype and self.weight.dtype == num.dtype
+                                            and keeps_dtype(num.dtype)):
             return False
         if tuple(num.shape) != (B, self.heads, T, self.width):
             return False

@@ -15,6 +15,7 @@ import ctypes
 import torch
 
 from ... import _lib
+from . import bankread
 from .dispatch import HipOp
 
 GN_HEAD_DIMS = (16, 32, 64, 128)
@@ -449,6 +450,7 @@ _normalized_read_op = HipOp("normalized_read", forward=_normalized_read_forward,
 def normalized_read(num, mass, resid, *, s: float = 1.0, eps: float = 1e-6, gate=None, gate_bias=None):
     """Read epilogue of one view on the GPU (ts_read_fwd / ts_read_bwd),
     optionally with the output gate (see :func:`_normalized_read_forward`)."""
+    bankread.check_gate(gate, num)
     return _normalized_read_op(num, mass, resid, gate, gate_bias, float(s), float(eps))
 
 

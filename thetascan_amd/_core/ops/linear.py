@@ -156,6 +156,13 @@ _linear_op = HipOp("linear", forward=_linear_forward, forward_fake=_linear_fake,
                    setup=_linear_setup, backward=_linear_backward)
 
 
+def keeps_dtype(dtype: torch.dtype) -> bool:
+    """Whether a product of ``dtype`` operands on the GPU gives that dtype
+    (autocast may choose another for it): what a kernel that reads the product
+    as ``dtype`` rows has to know beforehand."""
+    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == dtype
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear`` whose weight gradient is a split-K batched GEMM."""
     if not x.is_cuda:

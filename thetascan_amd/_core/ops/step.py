@@ -16,16 +16,11 @@ import torch.nn.functional as F
 
 from ... import _lib
 from . import fused, stream
+from .linear import keeps_dtype
 
 MAX_TOKENS = 8
 WIDTHS = (16, 32, 64, 128)
 SKINNY_ROWS = 64
-
-
-def _keeps_dtype(dtype: torch.dtype) -> bool:
-    """Whether a library product of ``dtype`` operands gives that dtype
-    (autocast may choose another for it)."""
-    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == dtype
 
 
 def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
@@ -39,7 +34,7 @@ def eligible(x: torch.Tensor, spec, head_dim: int, params) -> bool:
     _, T, D = x.shape
     if not (x.is_cuda and (dtype == torch.bfloat16 or dtype == torch.float32) and 1 <= T <= MAX_TOKENS
             and spec.m in WIDTHS and head_dim in WIDTHS and spec.m >= head_dim and D == params[0].shape[1]
-            and _keeps_dtype(dtype)):
+            and keeps_dtype(dtype)):
         return False
     for p in params:
         if p is not None and not (p.dtype == dtype and p.get_device() == device and p.is_contiguous()
